@@ -71,11 +71,36 @@ __device__ __forceinline__ float r2o_round_dtype(float x, int dtype) {
     return dtype == 0 ? r2o_bf16_to_f32(r2o_f32_to_bf16(x)) : r2o_f16_to_f32(r2o_f32_to_f16(x));
 }
 
-// ------------------------------------------------------------------------ wave reductions
-__device__ __forceinline__ float r2o_wave_max(float v) {
+// Eight 16-bit elements of a row.  VEC: one 16-byte load (p 16-byte aligned); otherwise element loads, for
+// rows that start anywhere.
+template <bool VEC>
+__device__ __forceinline__ r2o_u4 r2o_load8(const uint16_t* p) {
+    if constexpr (VEC) return r2o_ldg(reinterpret_cast<const r2o_u4*>(p));
+    r2o_u4 v;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, R2O_WAVE));
+    for (int i = 0; i < 4; ++i) v[i] = (uint32_t)r2o_ldg(p + 2 * i) | ((uint32_t)r2o_ldg(p + 2 * i + 1) << 16);
     return v;
+}
+
+// Elements of a packed row as fp32 (DT: 0 = bf16, 1 = fp16).
+template <int DT>
+__device__ __forceinline__ void r2o_unpack8(const r2o_u4& w, float (&x)[8]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        x[2 * i] = DT == 0 ? __uint_as_float(w[i] << 16) : r2o_f16_to_f32(w[i] & 0xffffu);
+        x[2 * i + 1] = DT == 0 ? __uint_as_float(w[i] & 0xffff0000u) : r2o_f16_to_f32(w[i] >> 16);
+    }
+}
+
+// x / s correctly rounded, for a divisor whose correctly rounded reciprocal y = RN(1 / s) is kept: an
+// approximate quotient and two corrections with exact fma remainders.  The quotient before the last
+// correction is faithful, so the last one rounds correctly (Markstein, IBM J. Res. Dev. 34(1), 1990).
+// 5 instructions in place of the ~12 of a division.  For finite x and s in [2^-100, 2^100]; a quotient
+// below the normal range may be off, which no caller's rounding to an integer can see.
+__device__ __forceinline__ float r2o_div_by(float x, float s, float y) {
+    float q = x * y;
+    q = __builtin_fmaf(__builtin_fmaf(-q, s, x), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-q, s, x), y, q);
 }
 
 // ------------------------------------------------------------------------- bit utilities
@@ -122,9 +147,11 @@ __device__ __forceinline__ uint32_t r2o_pack_bf2(float lo, float hi) {
 
 // Cross-lane exchanges through the VALU, in place of the LDS-unit permute behind __shfl_xor:
 // DPP within rows of 16 lanes, gfx950's v_permlane16_swap / v_permlane32_swap across rows.
+// Every control used here reads a lane of the same row, so no lane is out of bounds and bound_ctrl only
+// spares the move a zeroed destination (and lets it fold into the instruction that uses it).
 template <int CTRL>
 __device__ __forceinline__ float r2o_dpp(float x) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, false));
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
 }
 
 // The value of lane (lane ^ M), M = 1, 2, 4 or 8.

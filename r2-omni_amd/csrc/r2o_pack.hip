@@ -300,95 +300,183 @@ __global__ __launch_bounds__(64) void pack_int2_k_kernel(
     }
 }
 
-// ---------------------------------------------------------------------------- INT4 values
-// One wave per token row (thread t owns channels 2t, 2t+1); each wave of a 256-thread block takes
-// kVRows consecutive rows and issues all their loads first.  grid (ceil(n / (4 kVRows)), hkv).
-constexpr int kVRows = 8;
+// --------------------------------------------------------------------------------- values
+// INT4 (per-token symmetric) and INT2 (per-token-group affine) values.  A row is 16 lanes of 8 channels
+// (one 16-byte load), so a wave takes 4 rows per load and kVRows loads in flight; the reductions over a
+// row or group are in-lane maxima and at most 4 DPP exchanges, and a lane's codes leave as one 4- or
+// 2-byte store (256 or 128 contiguous bytes a wave).  VALU issue and the stream bound it about equally.
+// Measured, bf16: INT2 of 131k tokens x 8 heads, group 128, 264 -> 70 us (1.15 -> 4.3 TB/s); of 23k x 4,
+// group 32, 28 -> 10.9 us; INT4 of 27k x 4, 19.3 -> 10.6 us.  Before, one wave took a row at 2 channels a
+// lane: 6 LDS permutes per row, two ~12-instruction divisions per element and byte stores.
+// The codes are integers after RN(x / s) (+ z): the quotient is r2o_div_by's, and adding 1.5 * 2^23
+// rounds it half to even into the low mantissa bits, from which v_alignbit collects the codes.
+// Rows whose range is near or past the top of fp32 (kWideRange; infinities) take plain divisions.
+constexpr int kVRows = 4;                              // rows per lane
+constexpr int kVBlockRows = 4 * 4 * kVRows;            // per 256-thread block
+constexpr float kRoundMagic = 12582912.f;              // 1.5 * 2^23
+constexpr float kWideRange = 1e30f;
 
-__global__ __launch_bounds__(256) void pack_int4_v_kernel(
-    const uint16_t* __restrict__ src, int dtype, int64_t src_tokens, const int64_t* __restrict__ index,
-    int64_t n, int64_t dst_start, uint8_t* packed, float* scale, int64_t capacity) {
-    const int t = threadIdx.x & 63;
-    const int64_t h = blockIdx.y;
-    const int64_t i0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * kVRows;
-    // every load first: the rows' indices (clamped to the last row, branch-free), then the rows
-    int64_t rows[kVRows];
+struct ValuePack {
+    const uint16_t* src;
+    int64_t src_tokens;
+    const int64_t* index;  // nullable: token i is source row i
+    int64_t n, dst_start;
+    uint8_t* packed;
+    void* scale;    // INT4: f32; INT2: fp16
+    uint8_t* zero;  // INT2 only
+    int64_t capacity;
+    int group;      // INT2 only
+};
+
+// The 8 codes of a lane, BITS bits each, from the 8 integers rounded into the low mantissa bits of u.
+template <int BITS>
+__device__ __forceinline__ uint32_t collect_codes(const float (&u)[8]) {
+    uint32_t w = 0;
 #pragma unroll
-    for (int r = 0; r < kVRows; ++r) {
-        const int64_t i = min(i0 + r, n - 1);
-        rows[r] = index ? index[i] : i;
+    for (int i = 0; i < 8; ++i) w = __builtin_amdgcn_alignbit(__float_as_uint(u[i]), w, BITS);
+    return BITS == 4 ? w : w >> 16;
+}
+
+// max (or, negated, min) over the 2, 4, 8 or 16 lanes that share a group of `lanes` lanes.
+template <int BITS>
+__device__ __forceinline__ float lanes_max(float v, int lanes) {
+    v = fmaxf(v, r2o_lane_xor<1>(v));
+    v = fmaxf(v, r2o_lane_xor<2>(v));
+    if (BITS == 4 || lanes >= 8) v = fmaxf(v, r2o_lane_xor<4>(v));
+    if (BITS == 4 || lanes >= 16) v = fmaxf(v, r2o_lane_xor<8>(v));
+    return v;
+}
+
+template <int BITS, bool WIDE>
+__device__ __forceinline__ uint32_t value_codes(const float (&x)[8], float s, float y, float z) {
+    float u[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float q = WIDE ? __fdiv_rn(x[i], s) : r2o_div_by(x[i], s, y);
+        // v_med3 of a NaN is the smaller of the other two, as fminf(fmaxf(NaN, lo), hi)
+        u[i] = (BITS == 4 ? __builtin_amdgcn_fmed3f(q, -7.f, 7.f) : __builtin_amdgcn_fmed3f(q + z, 0.f, 3.f)) + kRoundMagic;
     }
-    uint32_t pair[kVRows];
+    return collect_codes<BITS>(u);
+}
+
+// Element j of v for a lane index j (three selects; an array would be indexed through memory).
+__device__ __forceinline__ float of_lane(int j, r2o_f4 v) {
+    const float lo = (j & 1) ? v.y : v.x, hi = (j & 1) ? v.w : v.z;
+    return (j & 2) ? hi : lo;
+}
+
+// Steps, zero points and codes of a lane's rows.  Lane j of a quad forms the step, its reciprocal and the
+// zero point of row j for the quad's group (a quad never crosses a group), and each row reads its lane's.
+template <int BITS, int DT, bool VEC, bool WIDE>
+__device__ __forceinline__ void store_values(const ValuePack& a, int64_t h, int64_t i0, int c8, int glanes,
+                                             const r2o_u4 (&raw)[kVRows], r2o_f4 range, r2o_f4 mn) {
+    static_assert(kVRows == 4, "one row per lane of a quad");
+    constexpr float kSteps = BITS == 4 ? 7.f : 3.f;
+    const int j = c8 & 3;
+    const float my_range = of_lane(j, range);
+    const float s = fmaxf(WIDE ? __fdiv_rn(my_range, kSteps) : r2o_div_by(my_range, kSteps, 1.f / kSteps), kEps);
+    const float y = WIDE ? 0.f : __fdiv_rn(1.f, s);
+    float z = 0.f;
+    if constexpr (BITS == 2) {
+        const float my_mn = of_lane(j, mn);
+        z = fminf(fmaxf(__builtin_rintf(WIDE ? __fdiv_rn(-my_mn, s) : r2o_div_by(-my_mn, s, y)), 0.f), 3.f);
+    }
+    const int64_t dst0 = h * a.capacity + a.dst_start + i0;  // row k of the lane is dst0 + 4 k
+    if ((c8 & (glanes - 1)) < 4 && i0 + 4 * j < a.n) {
+        if constexpr (BITS == 4) {
+            reinterpret_cast<float*>(a.scale)[dst0 + 4 * j] = s;
+        } else {
+            const int64_t e = (dst0 + 4 * j) * (16 / glanes) + c8 / glanes;
+            reinterpret_cast<uint16_t*>(a.scale)[e] = (uint16_t)r2o_f32_to_f16(s);
+            a.zero[e] = (uint8_t)z;
+        }
+    }
+    uint32_t codes[kVRows];
+    auto row = [&](int k, float sk, float yk, float zk) {
+        float x[8];
+        r2o_unpack8<DT>(raw[k], x);
+        codes[k] = value_codes<BITS, WIDE>(x, sk, yk, zk);
+    };
+    row(0, r2o_dpp<0x00>(s), r2o_dpp<0x00>(y), r2o_dpp<0x00>(z));
+    row(1, r2o_dpp<0x55>(s), r2o_dpp<0x55>(y), r2o_dpp<0x55>(z));
+    row(2, r2o_dpp<0xAA>(s), r2o_dpp<0xAA>(y), r2o_dpp<0xAA>(z));
+    row(3, r2o_dpp<0xFF>(s), r2o_dpp<0xFF>(y), r2o_dpp<0xFF>(z));
+    uint8_t* p = a.packed + dst0 * (16 * BITS) + BITS * c8;
 #pragma unroll
-    for (int r = 0; r < kVRows; ++r)
-        pair[r] = *reinterpret_cast<const uint32_t*>(src + (h * src_tokens + rows[r]) * 128 + 2 * t);
+    for (int k = 0; k < kVRows; ++k, p += 4 * 16 * BITS) {
+        if (i0 + 4 * k >= a.n) break;
+        if constexpr (!VEC) {
 #pragma unroll
-    for (int r = 0; r < kVRows; ++r) {
-        const int64_t i = i0 + r;
-        if (i >= n) break;
-        const float x0 = dtype == 0 ? r2o_bf16_to_f32(pair[r] & 0xffffu) : r2o_f16_to_f32(pair[r] & 0xffffu);
-        const float x1 = dtype == 0 ? r2o_bf16_to_f32(pair[r] >> 16) : r2o_f16_to_f32(pair[r] >> 16);
-        const float amax = r2o_wave_max(fmaxf(fabsf(x0), fabsf(x1)));
-        const float s = fmaxf(__fdiv_rn(amax, 7.0f), kEps);
-        const int q0 = (int)fminf(fmaxf(__builtin_rintf(__fdiv_rn(x0, s)), -7.f), 7.f);
-        const int q1 = (int)fminf(fmaxf(__builtin_rintf(__fdiv_rn(x1, s)), -7.f), 7.f);
-        const int64_t dst = h * capacity + dst_start + i;
-        packed[dst * 64 + t] = (uint8_t)((q0 & 15) | ((q1 & 15) << 4));
-        if (t == 0) scale[dst] = s;
+            for (int b = 0; b < BITS; ++b) p[b] = (uint8_t)(codes[k] >> (8 * b));
+        } else if constexpr (BITS == 4) {
+            *reinterpret_cast<uint32_t*>(p) = codes[k];
+        } else {
+            *reinterpret_cast<uint16_t*>(p) = (uint16_t)codes[k];
+        }
     }
 }
 
-// ---------------------------------------------------------------------------- INT2 values
-// One wave per token row as for INT4 values (thread t owns channels 2t, 2t+1; a group of G
-// channels is G/2 consecutive threads), kVRows rows per wave with all loads issued first.
-__device__ __forceinline__ void int2_value_row(uint32_t pair, int t, int dtype, int group, int64_t dst,
-                                               uint8_t* packed, uint16_t* scale, uint8_t* zero) {
-    const float x0 = dtype == 0 ? r2o_bf16_to_f32(pair & 0xffffu) : r2o_f16_to_f32(pair & 0xffffu);
-    const float x1 = dtype == 0 ? r2o_bf16_to_f32(pair >> 16) : r2o_f16_to_f32(pair >> 16);
-    float mn = fminf(x0, x1), mx = fmaxf(x0, x1);
-    for (int o = 1; o < group / 2; o <<= 1) {
-        mn = fminf(mn, __shfl_xor(mn, o, R2O_WAVE));
-        mx = fmaxf(mx, __shfl_xor(mx, o, R2O_WAVE));
-    }
-    mn = fminf(mn, 0.f);
-    mx = fmaxf(mx, 0.f);
-    const float s = fmaxf(__fdiv_rn(mx - mn, 3.0f), kEps);
-    const float z = fminf(fmaxf(__builtin_rintf(__fdiv_rn(-mn, s)), 0.f), 3.f);
-    const uint32_t c0 = (uint32_t)fminf(fmaxf(__builtin_rintf(__fdiv_rn(x0, s) + z), 0.f), 3.f);
-    const uint32_t c1 = (uint32_t)fminf(fmaxf(__builtin_rintf(__fdiv_rn(x1, s) + z), 0.f), 3.f);
-    const uint32_t mine = c0 | (c1 << 2);
-    const uint32_t next = (uint32_t)__shfl_down((int)mine, 1, R2O_WAVE);
-    if ((t & 1) == 0) packed[dst * 32 + t / 2] = (uint8_t)(mine | (next << 4));
-    const int groups = 128 / group;
-    if (t % (group / 2) == 0) {
-        const int gi = t / (group / 2);
-        scale[dst * groups + gi] = (uint16_t)r2o_f32_to_f16(s);
-        zero[dst * groups + gi] = (uint8_t)z;
-    }
-}
-
-__global__ __launch_bounds__(256) void pack_int2_v_kernel(
-    const uint16_t* __restrict__ src, int dtype, int64_t src_tokens, const int64_t* __restrict__ index,
-    int64_t n, int64_t dst_start, int group, uint8_t* packed, uint16_t* scale, uint8_t* zero, int64_t capacity) {
-    const int t = threadIdx.x & 63;
-    const int64_t h = blockIdx.y;
-    const int64_t i0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * kVRows;
+template <int BITS, int DT, bool VEC>
+__device__ __forceinline__ void pack_values(const ValuePack& a, int64_t block, int64_t h) {
+    const int lane = threadIdx.x & 63, c8 = lane & 15;
+    const int64_t i0 = (block * 4 + (threadIdx.x >> 6)) * (4 * kVRows) + (lane >> 4);
     // every load first: the rows' indices (clamped to the last row, branch-free), then the rows
     int64_t rows[kVRows];
 #pragma unroll
-    for (int r = 0; r < kVRows; ++r) {
-        const int64_t i = min(i0 + r, n - 1);
-        rows[r] = index ? index[i] : i;
+    for (int k = 0; k < kVRows; ++k) {
+        const int64_t i = min(i0 + 4 * k, a.n - 1);
+        rows[k] = a.index ? r2o_ldg(a.index + i) : i;
     }
-    uint32_t pair[kVRows];
+    r2o_u4 raw[kVRows];
 #pragma unroll
-    for (int r = 0; r < kVRows; ++r)
-        pair[r] = *reinterpret_cast<const uint32_t*>(src + (h * src_tokens + rows[r]) * 128 + 2 * t);
+    for (int k = 0; k < kVRows; ++k) raw[k] = r2o_load8<VEC>(a.src + (h * a.src_tokens + rows[k]) * 128 + 8 * c8);
+    const int glanes = BITS == 4 ? 16 : a.group / 8;  // lanes per group
+    r2o_f4 range, mn;
 #pragma unroll
-    for (int r = 0; r < kVRows; ++r) {
-        const int64_t i = i0 + r;
-        if (i >= n) break;
-        int2_value_row(pair[r], t, dtype, group, h * capacity + dst_start + i, packed, scale, zero);
+    for (int k = 0; k < kVRows; ++k) {
+        float x[8];
+        r2o_unpack8<DT>(raw[k], x);
+        mn[k] = 0.f;
+        if constexpr (BITS == 4) {
+            float mx = fabsf(x[0]);
+#pragma unroll
+            for (int i = 1; i < 8; ++i) mx = fmaxf(mx, fabsf(x[i]));
+            range[k] = lanes_max<4>(mx, 16);
+        } else {
+            float lo = -x[0], hi = x[0];
+#pragma unroll
+            for (int i = 1; i < 8; ++i) {
+                lo = fmaxf(lo, -x[i]);
+                hi = fmaxf(hi, x[i]);
+            }
+            lo = lanes_max<2>(lo, glanes);
+            hi = lanes_max<2>(hi, glanes);
+            mn[k] = fminf(-lo, 0.f);
+            range[k] = fmaxf(hi, 0.f) - mn[k];
+        }
+    }
+    float most = range[0];
+#pragma unroll
+    for (int k = 1; k < kVRows; ++k) most = fmaxf(most, range[k]);
+    if (__any(most > kWideRange)) store_values<BITS, DT, VEC, true>(a, h, i0, c8, glanes, raw, range, mn);
+    else store_values<BITS, DT, VEC, false>(a, h, i0, c8, glanes, raw, range, mn);
+}
+
+template <int BITS, int DT, bool VEC>
+__global__ __launch_bounds__(256) void pack_values_kernel(ValuePack a) {
+    pack_values<BITS, DT, VEC>(a, blockIdx.x, blockIdx.y);
+}
+
+template <int BITS>
+void launch_pack_values(const ValuePack& a, int64_t dtype, int64_t hkv, hipStream_t stream) {
+    const dim3 grid((unsigned)((a.n + kVBlockRows - 1) / kVBlockRows), (unsigned)hkv);
+    const bool vec = reinterpret_cast<uintptr_t>(a.src) % 16 == 0 && reinterpret_cast<uintptr_t>(a.packed) % 4 == 0;
+    if (dtype == 0) {
+        if (vec) hipLaunchKernelGGL((pack_values_kernel<BITS, 0, true>), grid, dim3(256), 0, stream, a);
+        else hipLaunchKernelGGL((pack_values_kernel<BITS, 0, false>), grid, dim3(256), 0, stream, a);
+    } else {
+        if (vec) hipLaunchKernelGGL((pack_values_kernel<BITS, 1, true>), grid, dim3(256), 0, stream, a);
+        else hipLaunchKernelGGL((pack_values_kernel<BITS, 1, false>), grid, dim3(256), 0, stream, a);
     }
 }
 
@@ -556,8 +644,8 @@ int r2o_pack_int4_v(const uint16_t* src, int64_t dtype, int64_t hkv, int64_t src
     if ((dtype != 0 && dtype != 1) || hkv <= 0 || n < 0 || dst_start < 0 || dst_start + n > capacity) return R2O_EINVAL;
     if (n == 0) return R2O_OK;
     if (!src || src_tokens <= 0 || n > 0x7fffffff || (!index && n > src_tokens)) return R2O_EINVAL;
-    hipLaunchKernelGGL(pack_int4_v_kernel, dim3((unsigned)((n + 4 * kVRows - 1) / (4 * kVRows)), (unsigned)hkv), dim3(256),
-                       0, (hipStream_t)stream, src, (int)dtype, src_tokens, index, n, dst_start, packed, scale, capacity);
+    launch_pack_values<4>({src, src_tokens, index, n, dst_start, packed, scale, nullptr, capacity, 128}, dtype, hkv,
+                          (hipStream_t)stream);
     R2O_CHECK_LAUNCH();
     return R2O_OK;
 }
@@ -569,9 +657,8 @@ int r2o_pack_int2_v(const uint16_t* src, int64_t dtype, int64_t hkv, int64_t src
     if (hkv <= 0 || n < 0 || dst_start < 0 || dst_start + n > capacity) return R2O_EINVAL;
     if (n == 0) return R2O_OK;
     if (!src || src_tokens <= 0 || n > 0x7fffffff || (!index && n > src_tokens)) return R2O_EINVAL;
-    hipLaunchKernelGGL(pack_int2_v_kernel, dim3((unsigned)((n + 4 * kVRows - 1) / (4 * kVRows)), (unsigned)hkv), dim3(256),
-                       0, (hipStream_t)stream, src, (int)dtype, src_tokens, index, n, dst_start, (int)group, packed, scale,
-                       zero, capacity);
+    launch_pack_values<2>({src, src_tokens, index, n, dst_start, packed, scale, zero, capacity, (int)group}, dtype, hkv,
+                          (hipStream_t)stream);
     R2O_CHECK_LAUNCH();
     return R2O_OK;
 }
