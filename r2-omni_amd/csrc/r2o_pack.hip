@@ -3,302 +3,13 @@
 // Bit-exactness with the reference's torch CPU quantisers (compact_int4_key.py:83-110,
 // quantization.py:19-50, int2_reference.py:96-151): IEEE fp32 division (__fdiv_rn), round half
 // to even (__builtin_rintf -> v_rndne_f32), no contraction (the file is built with
-// -ffp-contract=off), fp32 step quantisation with fp16-RNE storage of the step.
+// -ffp-contract=off), fp32 step quantisation with fp16-RNE storage of the step.  Where many values share a
+// divisor its reciprocal is kept and r2o_div_by gives the same correctly rounded quotients.
 #include "r2o_common.hpp"
 
 namespace {
 
 constexpr float kEps = 1.0e-6f;
-
-// ----------------------------------------------------------------------------- INT4 keys
-// grid (superblocks to write, hkv), block 64: thread t owns channels 2t, 2t+1 (byte t).
-__global__ __launch_bounds__(64) void pack_int4_k_kernel(
-    const uint16_t* __restrict__ src, int dtype, int64_t src_tokens, const int64_t* __restrict__ index,
-    int64_t n, int64_t tail, int64_t dst_start, uint8_t* packed, uint16_t* scale, uint8_t* zero,
-    uint32_t* operands, int64_t capacity, int64_t superblocks, int sb) {
-    __shared__ uint16_t s_half[128];
-    __shared__ uint8_t s_zero[128];
-    const int t = threadIdx.x;
-    const int64_t h = blockIdx.y;
-    const int64_t total = tail + n;
-    const int64_t first = (int64_t)blockIdx.x * sb;  // relative to dst_start
-    const int64_t count = min((int64_t)sb, total - first);
-    if (count <= 0) return;
-    const int64_t block_row = dst_start / sb + blockIdx.x;
-    uint8_t* prow = packed + (h * capacity + dst_start + first) * 64 + t;
-    uint16_t* srow = scale + (h * superblocks + block_row) * 128 + 2 * t;
-    uint8_t* zrow = zero + (h * superblocks + block_row) * 128 + 2 * t;
-    // old metadata of the tail superblock (only block 0 can hold tail positions)
-    const float os0 = r2o_f16_to_f32(srow[0]), os1 = r2o_f16_to_f32(srow[1]);
-    const float oz0 = (float)zrow[0], oz1 = (float)zrow[1];
-    auto value = [&](int64_t j, float& x0, float& x1) {
-        const int64_t pos = first + j;
-        if (pos < tail) {  // dequantise-then-round the partial tail (compact_int4_key.py:215-216)
-            const uint32_t b = prow[j * 64];
-            x0 = r2o_round_dtype(((float)(b & 15u) - oz0) * os0, dtype);
-            x1 = r2o_round_dtype(((float)(b >> 4) - oz1) * os1, dtype);
-        } else {
-            const int64_t i = pos - tail;
-            const int64_t row = index ? index[i] : i;
-            const uint32_t pair = *reinterpret_cast<const uint32_t*>(src + (h * src_tokens + row) * 128 + 2 * t);
-            x0 = dtype == 0 ? r2o_bf16_to_f32(pair & 0xffffu) : r2o_f16_to_f32(pair & 0xffffu);
-            x1 = dtype == 0 ? r2o_bf16_to_f32(pair >> 16) : r2o_f16_to_f32(pair >> 16);
-        }
-    };
-    float mn0 = 0.f, mn1 = 0.f, mx0 = 0.f, mx1 = 0.f;  // min(min x, 0), max(max x, 0)
-    for (int64_t j = 0; j < count; ++j) {
-        float x0, x1;
-        value(j, x0, x1);
-        mn0 = fminf(mn0, x0); mx0 = fmaxf(mx0, x0);
-        mn1 = fminf(mn1, x1); mx1 = fmaxf(mx1, x1);
-    }
-    const float st0 = fmaxf(__fdiv_rn(mx0 - mn0, 15.0f), kEps);
-    const float st1 = fmaxf(__fdiv_rn(mx1 - mn1, 15.0f), kEps);
-    const float zp0 = fminf(fmaxf(__builtin_rintf(__fdiv_rn(-mn0, st0)), 0.f), 15.f);
-    const float zp1 = fminf(fmaxf(__builtin_rintf(__fdiv_rn(-mn1, st1)), 0.f), 15.f);
-    for (int64_t j = 0; j < count; ++j) {
-        float x0, x1;
-        value(j, x0, x1);  // reads the old tail code before this thread overwrites it
-        const float c0 = fminf(fmaxf(__builtin_rintf(__fdiv_rn(x0, st0) + zp0), 0.f), 15.f);
-        const float c1 = fminf(fmaxf(__builtin_rintf(__fdiv_rn(x1, st1) + zp1), 0.f), 15.f);
-        prow[j * 64] = (uint8_t)((uint32_t)c0 | ((uint32_t)c1 << 4));
-    }
-    const uint16_t h0 = (uint16_t)r2o_f32_to_f16(st0), h1 = (uint16_t)r2o_f32_to_f16(st1);
-    srow[0] = h0;
-    srow[1] = h1;
-    zrow[0] = (uint8_t)zp0;
-    zrow[1] = (uint8_t)zp1;
-    if (operands) {  // QK MFMA operands of this superblock (layout in r2o_sspa.h)
-        s_half[2 * t] = h0;
-        s_half[2 * t + 1] = h1;
-        s_zero[2 * t] = (uint8_t)zp0;
-        s_zero[2 * t + 1] = (uint8_t)zp1;
-        __syncthreads();
-        const int g = t >> 4, j = (t >> 2) & 3, u = t & 3;
-        const int c = 32 * g + 8 * j + u;
-        uint32_t* orow = operands + (h * superblocks + block_row) * 128 + g * 32 + 4 * j + u;
-        if (u & 1) {  // channel pair read in place 4 bits up: code enters as 1024 + 16 c
-            orow[0] = r2o_f32_to_f16(r2o_f16_to_f32(s_half[c]) * 0.0625f) |
-                      (r2o_f32_to_f16(r2o_f16_to_f32(s_half[c + 4]) * 0.0625f) << 16);
-            orow[16] = (0xE400u | ((uint32_t)s_zero[c] << 4)) | ((0xE400u | ((uint32_t)s_zero[c + 4] << 4)) << 16);
-        } else {
-            orow[0] = (uint32_t)s_half[c] | ((uint32_t)s_half[c + 4] << 16);
-            orow[16] = (0xE400u | s_zero[c]) | ((0xE400u | (uint32_t)s_zero[c + 4]) << 16);
-        }
-    }
-}
-
-// Whole superblocks (no tail to requantise), staged through LDS in chunks of 32 token rows by
-// global->LDS DMA (four 256-byte rows per instruction, every DMA of a chunk issued before any is
-// waited for; token rows from the gather index, broadcast by lane).  One pass over the chunks for
-// the range and one for the codes (a 32-token superblock keeps its only chunk in LDS between the
-// two; a larger one reads its chunks again, from L2).  The code rows leave through LDS as 16-byte
-// stores.  10 KB of LDS for every superblock size.  Same arithmetic per element as
-// pack_int4_k_kernel.
-template <int SB>
-__global__ __launch_bounds__(64) void pack_int4_k_full_kernel(
-    const uint16_t* __restrict__ src, int dtype, int64_t src_tokens, const int64_t* __restrict__ index,
-    int64_t n, int64_t dst_start, uint8_t* packed, uint16_t* scale, uint8_t* zero, uint32_t* operands,
-    int64_t capacity, int64_t superblocks) {
-    __shared__ uint16_t s_half[128];
-    __shared__ uint8_t s_zero[128];
-    __shared__ __align__(16) uint32_t s_raw[32 * 64];
-    __shared__ __align__(16) uint8_t s_codes[32 * 64];
-    const int t = threadIdx.x;
-    const int64_t h = blockIdx.y;
-    const int64_t first = (int64_t)blockIdx.x * SB;
-    const int count = (int)min((int64_t)SB, n - first);
-    const int64_t block_row = dst_start / SB + blockIdx.x;
-    int row_lo = 0, row_hi = 0;  // source rows of tokens first + t and first + 64 + t
-    if (t < count) row_lo = (int)(index ? index[first + t] : first + t);
-    if (SB > 64 && t + 64 < count) row_hi = (int)(index ? index[first + 64 + t] : first + 64 + t);
-    const int last = count > 64 ? __builtin_amdgcn_readlane(row_hi, count - 65)
-                                : __builtin_amdgcn_readlane(row_lo, count - 1);
-    // lane t moves 16-byte chunk t % 16 of token 32 c + 4 k + t / 16 (rows past the end re-read
-    // the last token, whose LDS copy is never used)
-    const uint16_t* hsrc = src + h * src_tokens * 128 + 8 * (t & 15);
-    auto load_chunk = [&](int c) {
-        int rows[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {  // every row first, then every DMA
-            const int tk = 32 * c + 4 * k + (t >> 4);
-            const int row = tk < 64 ? __shfl(row_lo, tk & 63, R2O_WAVE) : __shfl(row_hi, tk & 63, R2O_WAVE);
-            rows[k] = tk < count ? row : last;
-        }
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-            if (32 * c + 4 * k < count)
-                __builtin_amdgcn_global_load_lds(
-                    (const __attribute__((address_space(1))) void*)(hsrc + (int64_t)rows[k] * 128),
-                    (__attribute__((address_space(3))) void*)(s_raw + 4 * k * 64), 16, 0, 0);
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the chunk has landed
-        __builtin_amdgcn_wave_barrier();
-    };
-    const int chunks = (count + 31) / 32;
-    float mn0 = 0.f, mn1 = 0.f, mx0 = 0.f, mx1 = 0.f;  // min(min x, 0), max(max x, 0)
-    for (int c = 0; c < chunks; ++c) {
-        if (c > 0) __builtin_amdgcn_wave_barrier();  // every lane is done reading the previous chunk
-        load_chunk(c);
-        for (int j = 0; j < min(32, count - 32 * c); ++j) {
-            const uint32_t raw = s_raw[j * 64 + t];
-            const float x0 = dtype == 0 ? r2o_bf16_to_f32(raw & 0xffffu) : r2o_f16_to_f32(raw & 0xffffu);
-            const float x1 = dtype == 0 ? r2o_bf16_to_f32(raw >> 16) : r2o_f16_to_f32(raw >> 16);
-            mn0 = fminf(mn0, x0); mx0 = fmaxf(mx0, x0);
-            mn1 = fminf(mn1, x1); mx1 = fmaxf(mx1, x1);
-        }
-    }
-    const float st0 = fmaxf(__fdiv_rn(mx0 - mn0, 15.0f), kEps);
-    const float st1 = fmaxf(__fdiv_rn(mx1 - mn1, 15.0f), kEps);
-    const float zp0 = fminf(fmaxf(__builtin_rintf(__fdiv_rn(-mn0, st0)), 0.f), 15.f);
-    const float zp1 = fminf(fmaxf(__builtin_rintf(__fdiv_rn(-mn1, st1)), 0.f), 15.f);
-    uint8_t* pbase = packed + (h * capacity + dst_start + first) * 64;
-    for (int c = 0; c < chunks; ++c) {
-        if (chunks > 1) {
-            __builtin_amdgcn_wave_barrier();
-            load_chunk(c);
-        }
-        const int nj = min(32, count - 32 * c);
-        for (int j = 0; j < nj; ++j) {
-            const uint32_t raw = s_raw[j * 64 + t];
-            const float x0 = dtype == 0 ? r2o_bf16_to_f32(raw & 0xffffu) : r2o_f16_to_f32(raw & 0xffffu);
-            const float x1 = dtype == 0 ? r2o_bf16_to_f32(raw >> 16) : r2o_f16_to_f32(raw >> 16);
-            const float c0 = fminf(fmaxf(__builtin_rintf(__fdiv_rn(x0, st0) + zp0), 0.f), 15.f);
-            const float c1 = fminf(fmaxf(__builtin_rintf(__fdiv_rn(x1, st1) + zp1), 0.f), 15.f);
-            s_codes[j * 64 + t] = (uint8_t)((uint32_t)c0 | ((uint32_t)c1 << 4));
-        }
-        __builtin_amdgcn_wave_barrier();
-        for (int k = t; k < nj * 4; k += 64)
-            *reinterpret_cast<uint4*>(pbase + (32 * c) * 64 + k * 16) = *reinterpret_cast<const uint4*>(s_codes + k * 16);
-        __builtin_amdgcn_wave_barrier();
-    }
-    const uint16_t h0 = (uint16_t)r2o_f32_to_f16(st0), h1 = (uint16_t)r2o_f32_to_f16(st1);
-    s_half[2 * t] = h0;
-    s_half[2 * t + 1] = h1;
-    s_zero[2 * t] = (uint8_t)zp0;
-    s_zero[2 * t + 1] = (uint8_t)zp1;
-    __syncthreads();
-    uint16_t* srow = scale + (h * superblocks + block_row) * 128 + 2 * t;
-    uint8_t* zrow = zero + (h * superblocks + block_row) * 128 + 2 * t;
-    srow[0] = h0;
-    srow[1] = h1;
-    zrow[0] = (uint8_t)zp0;
-    zrow[1] = (uint8_t)zp1;
-    if (operands) {  // QK MFMA operands of this superblock (layout in r2o_sspa.h)
-        const int g = t >> 4, j = (t >> 2) & 3, u = t & 3;
-        const int c = 32 * g + 8 * j + u;
-        uint32_t* orow = operands + (h * superblocks + block_row) * 128 + g * 32 + 4 * j + u;
-        if (u & 1) {  // channel pair read in place 4 bits up: code enters as 1024 + 16 c
-            orow[0] = r2o_f32_to_f16(r2o_f16_to_f32(s_half[c]) * 0.0625f) |
-                      (r2o_f32_to_f16(r2o_f16_to_f32(s_half[c + 4]) * 0.0625f) << 16);
-            orow[16] = (0xE400u | ((uint32_t)s_zero[c] << 4)) | ((0xE400u | ((uint32_t)s_zero[c + 4] << 4)) << 16);
-        } else {
-            orow[0] = (uint32_t)s_half[c] | ((uint32_t)s_half[c + 4] << 16);
-            orow[16] = (0xE400u | s_zero[c]) | ((0xE400u | (uint32_t)s_zero[c + 4]) << 16);
-        }
-    }
-}
-
-// ----------------------------------------------------------------------------- INT2 keys
-// OScaR per-channel affine INT2 over superblocks (int2_reference.py:159-214, clip ratio 1):
-// block min/max without 0, scale = range / 3, inv = (1 / range) * 3 (torch's ``3.0 / t``),
-// zero = rne(-min * inv), offset = -zero * scale; constant channels keep scale 0 and offset = min.
-// grid (superblocks to write, hkv), block 64: threads 0..31 quantise channels 4t..4t+3 (byte t
-// of the 32-byte row); then all 64 write the QK MFMA operand pairs of the superblock.
-__global__ __launch_bounds__(64) void pack_int2_k_kernel(
-    const uint16_t* __restrict__ src, int dtype, int64_t src_tokens, const int64_t* __restrict__ index,
-    int64_t n, int64_t tail, int64_t dst_start, uint8_t* packed, uint16_t* scale, uint16_t* offset,
-    uint32_t* operands, int64_t capacity, int64_t superblocks, int sb) {
-    __shared__ uint16_t s_half[128];
-    __shared__ uint16_t s_off[128];
-    const int t = threadIdx.x;
-    const int64_t h = blockIdx.y;
-    const int64_t total = tail + n;
-    const int64_t first = (int64_t)blockIdx.x * sb;  // relative to dst_start
-    const int64_t count = min((int64_t)sb, total - first);
-    if (count <= 0) return;
-    const int64_t block_row = dst_start / sb + blockIdx.x;
-    if (t < 32) {
-        uint8_t* prow = packed + (h * capacity + dst_start + first) * 32 + t;
-        uint16_t* srow = scale + (h * superblocks + block_row) * 128 + 4 * t;
-        uint16_t* orow = offset + (h * superblocks + block_row) * 128 + 4 * t;
-        // old metadata of the tail superblock (only block 0 can hold tail positions)
-        float os[4], oo[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            os[i] = r2o_f16_to_f32(srow[i]);
-            oo[i] = r2o_f16_to_f32(orow[i]);
-        }
-        auto value = [&](int64_t j, float (&x)[4]) {
-            const int64_t pos = first + j;
-            if (pos < tail) {  // dequantise-then-round the partial tail (compact_int2_key.py:114-121)
-                const uint32_t b = prow[j * 32];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    x[i] = r2o_round_dtype(__fadd_rn(__fmul_rn((float)((b >> (2 * i)) & 3u), os[i]), oo[i]), dtype);
-            } else {
-                const int64_t i0 = pos - tail;
-                const int64_t row = index ? index[i0] : i0;
-                const uint2 q = *reinterpret_cast<const uint2*>(src + (h * src_tokens + row) * 128 + 4 * t);
-                const uint32_t w[4] = {q.x & 0xffffu, q.x >> 16, q.y & 0xffffu, q.y >> 16};
-#pragma unroll
-                for (int i = 0; i < 4; ++i) x[i] = dtype == 0 ? r2o_bf16_to_f32(w[i]) : r2o_f16_to_f32(w[i]);
-            }
-        };
-        float mn[4], mx[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            mn[i] = INFINITY;
-            mx[i] = -INFINITY;
-        }
-        for (int64_t j = 0; j < count; ++j) {
-            float x[4];
-            value(j, x);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                mn[i] = fminf(mn[i], x[i]);
-                mx[i] = fmaxf(mx[i], x[i]);
-            }
-        }
-        float sc[4], inv[4], zp[4], off[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float rng = __fsub_rn(mx[i], mn[i]);
-            const bool nonconst = rng > 0.f;
-            sc[i] = nonconst ? __fdiv_rn(rng, 3.0f) : 0.f;
-            inv[i] = nonconst ? __fmul_rn(__fdiv_rn(1.0f, fmaxf(rng, 1e-30f)), 3.0f) : 0.f;
-            zp[i] = nonconst ? __builtin_rintf(__fmul_rn(-mn[i], inv[i])) : 0.f;
-            off[i] = nonconst ? __fmul_rn(-zp[i], sc[i]) : mn[i];
-        }
-        for (int64_t j = 0; j < count; ++j) {
-            float x[4];
-            value(j, x);  // reads the old tail code before this thread overwrites it
-            uint32_t byte = 0;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float c = fminf(fmaxf(__builtin_rintf(__fadd_rn(__fmul_rn(x[i], inv[i]), zp[i])), 0.f), 3.f);
-                byte |= (uint32_t)c << (2 * i);
-            }
-            prow[j * 32] = (uint8_t)byte;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint16_t hs = (uint16_t)r2o_f32_to_f16(sc[i]), ho = (uint16_t)r2o_f32_to_f16(off[i]);
-            srow[i] = hs;
-            orow[i] = ho;
-            s_half[4 * t + i] = hs;
-            s_off[4 * t + i] = ho;
-        }
-    }
-    if (operands) {  // QK MFMA operands of this superblock (layout in r2o_sspa.h)
-        __syncthreads();
-        const int g = t >> 4, j = (t >> 2) & 3, u = t & 3;
-        const int c = 32 * g + 16 * (j >> 1) + 4 * (j & 1) + u;  // pair (c, c + 8)
-        const float k = u == 0 ? 1.f : (u == 1 ? 0.25f : (u == 2 ? 0.0625f : 0.015625f));  // crumb u enters x 4^u
-        uint32_t* orow = operands + (h * superblocks + block_row) * 128 + g * 32 + 4 * j + u;
-        orow[0] = r2o_f32_to_f16(r2o_f16_to_f32(s_half[c]) * k) | (r2o_f32_to_f16(r2o_f16_to_f32(s_half[c + 8]) * k) << 16);
-        orow[16] = (uint32_t)s_off[c] | ((uint32_t)s_off[c + 8] << 16);
-    }
-}
 
 // --------------------------------------------------------------------------------- values
 // INT4 (per-token symmetric) and INT2 (per-token-group affine) values.  A row is 16 lanes of 8 channels
@@ -480,6 +191,307 @@ void launch_pack_values(const ValuePack& a, int64_t dtype, int64_t hkv, hipStrea
     }
 }
 
+// ------------------------------------------------------------------------------------ keys
+// INT4 (per-channel affine over min(min x, 0) .. max(max x, 0)) and INT2 (OScaR form, int2_reference.py:
+// 159-214, clip ratio 1: block min / max without 0, scale = range / 3, inv = (1 / range) * 3 as torch's
+// ``3.0 / t``, zero = rne(-min * inv), offset = -zero * scale; constant channels keep scale 0 and offset =
+// min) keys over superblocks of SB tokens.
+//
+// A wave takes 32 tokens of a superblock: lane (r, c8) holds channels 8 c8 .. 8 c8 + 7 of tokens 4 k + r in
+// registers from one 16-byte load each, all 8 in flight at once.  The channel ranges fold over the lane's
+// tokens, then over r by permlane swaps that also scatter them, so that lane (r, c8) ends with channels
+// 8 c8 + 2 r and + 1 and forms their step, zero point and reciprocal once; the waves of a larger
+// superblock meet in LDS.  Every lane reads the 8 channels it needs back and the codes leave as one store
+// per token (256 or 128 contiguous bytes a wave).  Each key row is read once, and the stream bounds it.
+// Measured, bf16: INT2 of 131k tokens x 8 heads, SB 128, 218 -> 61 us (5.1 TB/s); INT4 of 59k x 4, SB 32,
+// 35 -> 20 us (4.0 TB/s); INT4 of a flush (128 tokens and a partial superblock x 4 heads) 20.6 -> 6.0 us.
+// Before, a wave took a superblock at 2 or 4 channels a lane, token after token, reading it twice.
+struct KeyPack {
+    const uint16_t* src;
+    int64_t src_tokens;
+    const int64_t* index;  // nullable: token i is source row i
+    int64_t n, tail, dst_start;
+    uint8_t* packed;
+    uint16_t* scale;
+    void* zero;            // INT4: u8 zero points; INT2: fp16 offsets
+    uint32_t* operands;    // nullable
+    int64_t capacity, superblocks;
+};
+
+constexpr int kKeyWaves = 4;
+constexpr int kKeyBlockTokens = 32 * kKeyWaves;
+
+struct KeyLds {  // per wave: one value per channel
+    float step[kKeyWaves][128];  // INT4: step; INT2: scale
+    float mul[kKeyWaves][128];   // INT4: RN(1 / step); INT2: inv
+    float zero[kKeyWaves][128];  // zero point
+    float off[kKeyWaves][128];   // INT2: offset
+};
+
+// (m over the 4 lanes that share c8, for channel pairs) from 8 per-lane channel values: lane (r, c8) gets
+// channels 8 c8 + 2 r and + 1.
+__device__ __forceinline__ void scatter_max(const float (&m)[8], float& a, float& b) {
+    float h[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // lanes below 32 keep channels 0 .. 3, lanes above them 4 .. 7
+        const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(m[i]), __float_as_uint(m[i + 4]), false, false);
+        h[i] = fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1]));
+    }
+    const auto s0 = __builtin_amdgcn_permlane16_swap(__float_as_uint(h[0]), __float_as_uint(h[2]), false, false);
+    const auto s1 = __builtin_amdgcn_permlane16_swap(__float_as_uint(h[1]), __float_as_uint(h[3]), false, false);
+    a = fmaxf(__uint_as_float(s0[0]), __uint_as_float(s0[1]));
+    b = fmaxf(__uint_as_float(s1[0]), __uint_as_float(s1[1]));
+}
+
+__device__ __forceinline__ void read8(const float* p, float (&x)[8]) {
+    const r2o_f4 lo = reinterpret_cast<const r2o_f4*>(p)[0], hi = reinterpret_cast<const r2o_f4*>(p)[1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        x[i] = lo[i];
+        x[i + 4] = hi[i];
+    }
+}
+
+// Old metadata of a partial tail superblock for channels 8 c8 ..: what its codes dequantise with.
+template <int BITS>
+__device__ __forceinline__ void tail_metadata(const KeyPack& a, int64_t meta_row, int c8, float (&s)[8], float (&z)[8]) {
+    const int64_t m = meta_row * 128 + 8 * c8;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        s[i] = r2o_f16_to_f32(a.scale[m + i]);
+        z[i] = BITS == 4 ? (float)reinterpret_cast<const uint8_t*>(a.zero)[m + i]
+                         : r2o_f16_to_f32(reinterpret_cast<const uint16_t*>(a.zero)[m + i]);
+    }
+}
+
+// The 8 channels of a tail position, dequantised and rounded to the row dtype (compact_int4_key.py:215-216,
+// compact_int2_key.py:114-121).
+template <int BITS, int DT, bool VEC>
+__device__ __forceinline__ r2o_u4 tail_row(const uint8_t* code, const float (&s)[8], const float (&z)[8]) {
+    uint32_t w = 0;
+    if constexpr (!VEC) {
+#pragma unroll
+        for (int b = 0; b < BITS; ++b) w |= (uint32_t)code[b] << (8 * b);
+    } else {
+        w = BITS == 4 ? *reinterpret_cast<const uint32_t*>(code) : *reinterpret_cast<const uint16_t*>(code);
+    }
+    r2o_u4 out = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float c = (float)((w >> (i * BITS)) & ((1 << BITS) - 1));
+        const float x = BITS == 4 ? __fmul_rn(__fsub_rn(c, z[i]), s[i]) : __fadd_rn(__fmul_rn(c, s[i]), z[i]);
+        out[i >> 1] |= (DT == 0 ? r2o_f32_to_bf16(x) : r2o_f32_to_f16(x)) << (16 * (i & 1));
+    }
+    return out;
+}
+
+// Codes of the wave's tokens own + 4 k + r < count of its superblock, from the channels' values in LDS.
+template <int BITS, int DT, bool VEC, bool WIDE>
+__device__ __forceinline__ void store_key_codes(const KeyPack& a, const KeyLds& lds, int wave, int64_t row0, int own,
+                                                int count, int r, int c8, const r2o_u4 (&raw)[8]) {
+    float step[8], mul[8], zero[8];
+    if constexpr (BITS == 4) read8(lds.step[wave] + 8 * c8, step);
+    read8(lds.mul[wave] + 8 * c8, mul);
+    read8(lds.zero[wave] + 8 * c8, zero);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        float x[8], u[8];
+        r2o_unpack8<DT>(raw[k], x);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            float q;  // v_med3 of a NaN is the smaller of the other two, as fminf(fmaxf(NaN, lo), hi)
+            if constexpr (BITS == 2) q = __fmul_rn(x[i], mul[i]);
+            else q = WIDE ? __fdiv_rn(x[i], step[i]) : r2o_div_by(x[i], step[i], mul[i]);
+            u[i] = __builtin_amdgcn_fmed3f(q + zero[i], 0.f, BITS == 4 ? 15.f : 3.f) + kRoundMagic;
+        }
+        const uint32_t codes = collect_codes<BITS>(u);
+        if (own + 4 * k + r >= count) break;
+        uint8_t* p = a.packed + (row0 + own + 4 * k + r) * (16 * BITS) + BITS * c8;
+        if constexpr (!VEC) {
+#pragma unroll
+            for (int b = 0; b < BITS; ++b) p[b] = (uint8_t)(codes >> (8 * b));
+        } else if constexpr (BITS == 4) {
+            *reinterpret_cast<uint32_t*>(p) = codes;
+        } else {
+            *reinterpret_cast<uint16_t*>(p) = (uint16_t)codes;
+        }
+    }
+}
+
+// Superblock metadata and QK MFMA operands (layout in r2o_sspa.h), by one wave.
+template <int BITS, bool VEC>
+__device__ __forceinline__ void store_key_metadata(const KeyPack& a, const KeyLds& lds, int wave, int64_t meta_row) {
+    const int lane = threadIdx.x & 63;
+    const float* step = lds.step[wave];
+    const float* zero = BITS == 4 ? lds.zero[wave] : lds.off[wave];
+    const uint32_t h0 = r2o_f32_to_f16(step[2 * lane]), h1 = r2o_f32_to_f16(step[2 * lane + 1]);
+    const float z0 = zero[2 * lane], z1 = zero[2 * lane + 1];
+    uint16_t* srow = a.scale + meta_row * 128 + 2 * lane;
+    if constexpr (VEC) {
+        *reinterpret_cast<uint32_t*>(srow) = h0 | (h1 << 16);
+    } else {
+        srow[0] = (uint16_t)h0;
+        srow[1] = (uint16_t)h1;
+    }
+    if constexpr (BITS == 4) {
+        uint8_t* zrow = reinterpret_cast<uint8_t*>(a.zero) + meta_row * 128 + 2 * lane;
+        zrow[0] = (uint8_t)z0;
+        zrow[1] = (uint8_t)z1;
+    } else {
+        uint16_t* zrow = reinterpret_cast<uint16_t*>(a.zero) + meta_row * 128 + 2 * lane;
+        zrow[0] = (uint16_t)r2o_f32_to_f16(z0);
+        zrow[1] = (uint16_t)r2o_f32_to_f16(z1);
+    }
+    if (!a.operands) return;
+    const int g = lane >> 4, j = (lane >> 2) & 3, u = lane & 3;
+    uint32_t* orow = a.operands + meta_row * 128 + g * 32 + 4 * j + u;
+    if constexpr (BITS == 4) {
+        const int c = 32 * g + 8 * j + u;  // pair (c, c + 4); odd u: read in place 4 bits up, 1024 + 16 code
+        const float k = (u & 1) ? 0.0625f : 1.f;
+        const uint32_t s0 = r2o_f32_to_f16(step[c]), s1 = r2o_f32_to_f16(step[c + 4]);
+        const uint32_t shift = (u & 1) ? 4 : 0;
+        orow[0] = r2o_f32_to_f16(r2o_f16_to_f32(s0) * k) | (r2o_f32_to_f16(r2o_f16_to_f32(s1) * k) << 16);
+        orow[16] = (0xE400u | ((uint32_t)zero[c] << shift)) | ((0xE400u | ((uint32_t)zero[c + 4] << shift)) << 16);
+    } else {
+        const int c = 32 * g + 16 * (j >> 1) + 4 * (j & 1) + u;  // pair (c, c + 8); crumb u enters x 4^u
+        const float k = u == 0 ? 1.f : (u == 1 ? 0.25f : (u == 2 ? 0.0625f : 0.015625f));
+        const uint32_t s0 = r2o_f32_to_f16(step[c]), s1 = r2o_f32_to_f16(step[c + 8]);
+        orow[0] = r2o_f32_to_f16(r2o_f16_to_f32(s0) * k) | (r2o_f32_to_f16(r2o_f16_to_f32(s1) * k) << 16);
+        orow[16] = r2o_f32_to_f16(zero[c]) | (r2o_f32_to_f16(zero[c + 8]) << 16);
+    }
+}
+
+// Tokens [128 block, 128 block + 128) of the destination range, by a 256-thread block (every thread calls
+// this: the waves of a superblock of 64 or 128 tokens meet at a barrier).  Every read of old codes and
+// metadata precedes the first store of a superblock: a wave's own reads before its own stores, the other
+// waves' before the barrier.
+template <int BITS, int SB, int DT, bool VEC>
+__device__ __forceinline__ void pack_keys(const KeyPack& a, int64_t block, int64_t h, KeyLds& lds) {
+    constexpr int kSbWaves = SB / 32;  // waves of a superblock
+    const int lane = threadIdx.x & 63, c8 = lane & 15, r = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lead = wave & ~(kSbWaves - 1);
+    const int own = 32 * (wave - lead);                                      // the wave's first token in it
+    const int64_t first = block * kKeyBlockTokens + 32 * lead;               // relative to dst_start
+    const int count = (int)min((int64_t)SB, a.tail + a.n - first);           // tokens of the superblock
+    const int64_t block_row = (a.dst_start + first) / SB;
+    r2o_u4 raw[8];
+    float a0 = 0.f, a1 = 0.f, b0 = 0.f, b1 = 0.f;  // -min and max of channels 8 c8 + 2 r, + 1
+    if (count > 0) {
+        // tokens past the end read the superblock's last one again, which no range notices
+        if (first >= a.tail) {
+            int64_t rows[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int64_t i = first + min(own + 4 * k + r, count - 1) - a.tail;
+                rows[k] = a.index ? r2o_ldg(a.index + i) : i;
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) raw[k] = r2o_load8<VEC>(a.src + (h * a.src_tokens + rows[k]) * 128 + 8 * c8);
+        } else {  // the one superblock that holds tail positions
+            float ts[8], tz[8];
+            tail_metadata<BITS>(a, h * a.superblocks + block_row, c8, ts, tz);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int64_t pos = first + min(own + 4 * k + r, count - 1), i = pos - a.tail;
+                const uint8_t* code = a.packed + (h * a.capacity + a.dst_start + pos) * (16 * BITS) + BITS * c8;
+                r2o_u4 v;
+                if (i < 0) v = tail_row<BITS, DT, VEC>(code, ts, tz);
+                else v = r2o_load8<VEC>(a.src + (h * a.src_tokens + (a.index ? r2o_ldg(a.index + i) : i)) * 128 + 8 * c8);
+                raw[k] = v;
+            }
+        }
+        float lo[8], hi[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) lo[i] = hi[i] = BITS == 4 ? 0.f : -INFINITY;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            float x[8];
+            r2o_unpack8<DT>(raw[k], x);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                lo[i] = fmaxf(lo[i], -x[i]);
+                hi[i] = fmaxf(hi[i], x[i]);
+            }
+        }
+        scatter_max(lo, a0, a1);
+        scatter_max(hi, b0, b1);
+    }
+    const int ch = 8 * c8 + 2 * r;
+    if constexpr (kSbWaves > 1) {
+        if (count > 0) {
+            *reinterpret_cast<float2*>(&lds.step[wave][ch]) = make_float2(a0, a1);
+            *reinterpret_cast<float2*>(&lds.mul[wave][ch]) = make_float2(b0, b1);
+        }
+        __syncthreads();
+        if (count > 0) {
+#pragma unroll
+            for (int w = 1; w < kSbWaves; ++w) {
+                const int o = lead + ((wave + w) & (kSbWaves - 1));
+                const float2 lo = *reinterpret_cast<const float2*>(&lds.step[o][ch]);
+                const float2 hi = *reinterpret_cast<const float2*>(&lds.mul[o][ch]);
+                a0 = fmaxf(a0, lo.x);
+                a1 = fmaxf(a1, lo.y);
+                b0 = fmaxf(b0, hi.x);
+                b1 = fmaxf(b1, hi.y);
+            }
+        }
+        __syncthreads();  // the ranges are read: the same LDS takes the metadata
+    }
+    if (count <= 0) return;
+    float step[2], mul[2], zero[2], off[2];
+    bool wide = false;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const float mn = -(e ? a1 : a0), mx = e ? b1 : b0;
+        const float range = mx - mn;
+        if constexpr (BITS == 4) {
+            wide |= range > kWideRange;
+            step[e] = fmaxf(__fdiv_rn(range, 15.f), kEps);
+            mul[e] = __fdiv_rn(1.f, step[e]);
+            zero[e] = fminf(fmaxf(__builtin_rintf(__fdiv_rn(-mn, step[e])), 0.f), 15.f);
+            off[e] = 0.f;
+        } else {
+            const bool nonconst = range > 0.f;
+            step[e] = nonconst ? __fdiv_rn(range, 3.f) : 0.f;
+            mul[e] = nonconst ? __fmul_rn(__fdiv_rn(1.f, fmaxf(range, 1e-30f)), 3.f) : 0.f;
+            zero[e] = nonconst ? __builtin_rintf(__fmul_rn(-mn, mul[e])) : 0.f;
+            off[e] = nonconst ? __fmul_rn(-zero[e], step[e]) : mn;
+        }
+    }
+    *reinterpret_cast<float2*>(&lds.step[wave][ch]) = make_float2(step[0], step[1]);
+    *reinterpret_cast<float2*>(&lds.mul[wave][ch]) = make_float2(mul[0], mul[1]);
+    *reinterpret_cast<float2*>(&lds.zero[wave][ch]) = make_float2(zero[0], zero[1]);
+    if constexpr (BITS == 2) *reinterpret_cast<float2*>(&lds.off[wave][ch]) = make_float2(off[0], off[1]);
+    __builtin_amdgcn_wave_barrier();  // a wave's LDS operations complete in order
+    const int64_t row0 = h * a.capacity + a.dst_start + first;
+    if (BITS == 4 && __any(wide)) store_key_codes<BITS, DT, VEC, true>(a, lds, wave, row0, own, count, r, c8, raw);
+    else store_key_codes<BITS, DT, VEC, false>(a, lds, wave, row0, own, count, r, c8, raw);
+    if (wave == lead) store_key_metadata<BITS, VEC>(a, lds, wave, h * a.superblocks + block_row);
+}
+
+template <int BITS, int SB, int DT, bool VEC>
+__global__ __launch_bounds__(64 * kKeyWaves) void pack_keys_kernel(KeyPack a) {
+    __shared__ __align__(16) KeyLds lds;
+    pack_keys<BITS, SB, DT, VEC>(a, blockIdx.x, blockIdx.y, lds);
+}
+
+template <int BITS, int SB, int DT>
+void launch_pack_keys_of(const KeyPack& a, int64_t hkv, hipStream_t stream) {
+    const dim3 grid((unsigned)((a.tail + a.n + kKeyBlockTokens - 1) / kKeyBlockTokens), (unsigned)hkv);
+    const bool vec = reinterpret_cast<uintptr_t>(a.src) % 16 == 0 && reinterpret_cast<uintptr_t>(a.packed) % 4 == 0 &&
+                     reinterpret_cast<uintptr_t>(a.scale) % 4 == 0;
+    if (vec) hipLaunchKernelGGL((pack_keys_kernel<BITS, SB, DT, true>), grid, dim3(64 * kKeyWaves), 0, stream, a);
+    else hipLaunchKernelGGL((pack_keys_kernel<BITS, SB, DT, false>), grid, dim3(64 * kKeyWaves), 0, stream, a);
+}
+
+template <int BITS>
+void launch_pack_keys(const KeyPack& a, int64_t superblock, int64_t dtype, int64_t hkv, hipStream_t stream) {
+    if (superblock == 32) dtype == 0 ? launch_pack_keys_of<BITS, 32, 0>(a, hkv, stream) : launch_pack_keys_of<BITS, 32, 1>(a, hkv, stream);
+    else if (superblock == 64) dtype == 0 ? launch_pack_keys_of<BITS, 64, 0>(a, hkv, stream) : launch_pack_keys_of<BITS, 64, 1>(a, hkv, stream);
+    else dtype == 0 ? launch_pack_keys_of<BITS, 128, 0>(a, hkv, stream) : launch_pack_keys_of<BITS, 128, 1>(a, hkv, stream);
+}
+
 // ---------------------------------------------------------------------------- gather rows
 // 64 rows per 256-thread block: thread t moves 16-byte chunk t % 16 of rows t / 16 + 16 k, all
 // loads first.  grid (ceil(n / 64), hkv).
@@ -599,25 +611,9 @@ int r2o_pack_int4_k(const uint16_t* src, int64_t dtype, int64_t hkv, int64_t src
     if (hkv <= 0 || n < 0 || tail < 0 || tail >= superblock || dst_start < 0 || dst_start % superblock) return R2O_EINVAL;
     if (dst_start + tail + n > capacity || capacity % superblock || superblocks * superblock != capacity) return R2O_EINVAL;
     if (n > 0 && (!src || src_tokens <= 0)) return R2O_EINVAL;
-    const int64_t total = tail + n;
-    if (total == 0) return R2O_OK;
-    const int64_t blocks = (total + superblock - 1) / superblock;
-    if (tail == 0 && src_tokens <= 0x7fffffff) {  // whole superblocks: the register-resident packer
-        const dim3 grid((unsigned)blocks, (unsigned)hkv);
-        if (superblock == 32)
-            hipLaunchKernelGGL(pack_int4_k_full_kernel<32>, grid, dim3(64), 0, (hipStream_t)stream, src, (int)dtype,
-                               src_tokens, index, n, dst_start, packed, scale, zero, operands, capacity, superblocks);
-        else if (superblock == 64)
-            hipLaunchKernelGGL(pack_int4_k_full_kernel<64>, grid, dim3(64), 0, (hipStream_t)stream, src, (int)dtype,
-                               src_tokens, index, n, dst_start, packed, scale, zero, operands, capacity, superblocks);
-        else
-            hipLaunchKernelGGL(pack_int4_k_full_kernel<128>, grid, dim3(64), 0, (hipStream_t)stream, src, (int)dtype,
-                               src_tokens, index, n, dst_start, packed, scale, zero, operands, capacity, superblocks);
-    } else {
-        hipLaunchKernelGGL(pack_int4_k_kernel, dim3((unsigned)blocks, (unsigned)hkv), dim3(64), 0, (hipStream_t)stream,
-                           src, (int)dtype, src_tokens, index, n, tail, dst_start, packed, scale, zero, operands,
-                           capacity, superblocks, (int)superblock);
-    }
+    if (tail + n == 0) return R2O_OK;
+    launch_pack_keys<4>({src, src_tokens, index, n, tail, dst_start, packed, scale, zero, operands, capacity, superblocks},
+                        superblock, dtype, hkv, (hipStream_t)stream);
     R2O_CHECK_LAUNCH();
     return R2O_OK;
 }
@@ -629,12 +625,9 @@ int r2o_pack_int2_k(const uint16_t* src, int64_t dtype, int64_t hkv, int64_t src
     if (hkv <= 0 || n < 0 || tail < 0 || tail >= superblock || dst_start < 0 || dst_start % superblock) return R2O_EINVAL;
     if (dst_start + tail + n > capacity || capacity % superblock || superblocks * superblock != capacity) return R2O_EINVAL;
     if (n > 0 && (!src || src_tokens <= 0)) return R2O_EINVAL;
-    const int64_t total = tail + n;
-    if (total == 0) return R2O_OK;
-    const int64_t blocks = (total + superblock - 1) / superblock;
-    hipLaunchKernelGGL(pack_int2_k_kernel, dim3((unsigned)blocks, (unsigned)hkv), dim3(64), 0, (hipStream_t)stream,
-                       src, (int)dtype, src_tokens, index, n, tail, dst_start, packed, scale, offset, operands,
-                       capacity, superblocks, (int)superblock);
+    if (tail + n == 0) return R2O_OK;
+    launch_pack_keys<2>({src, src_tokens, index, n, tail, dst_start, packed, scale, offset, operands, capacity, superblocks},
+                        superblock, dtype, hkv, (hipStream_t)stream);
     R2O_CHECK_LAUNCH();
     return R2O_OK;
 }

@@ -95,3 +95,70 @@ def test_value_packers_at_the_ends_of_the_range():
     np.testing.assert_array_equal(codes(a.packed[:, :64].cpu().numpy(), 2), w2)
     np.testing.assert_array_equal(a.scale[:, :64].cpu().numpy(), s2)
     np.testing.assert_array_equal(a.zero_point[:, :64].cpu().numpy(), z2)
+
+
+KEYS = {4: ("build_compact_int4_key_arena", "quantize_int4_key_per_channel", "dequantize_int4_key"),
+        2: ("build_compact_int2_key_arena", "quantize_int2_key_per_channel", "dequantize_int2_key")}
+
+
+@pytest.mark.parametrize("dtype", sorted(DTYPES))
+@pytest.mark.parametrize("bits,superblock", [(b, sb) for b in (4, 2) for sb in (32, 64, 128)])
+@pytest.mark.parametrize("n,offset", [(1, 0), (31, 2), (33, 0), (127, 0), (128, 0), (161, 8), (700, 0)])
+def test_key_packers_match_the_oracle_through_a_flush(n, offset, bits, superblock, dtype):
+    """A gathered build of n tokens, then a flush of 128 that requantises the partial tail superblock."""
+    import r2omni_amd as ro
+    from oracle import quant
+
+    dev = _dev()
+    build, quantise, dequantise = KEYS[bits]
+    quantise, dequantise = getattr(quant, quantise), getattr(quant, dequantise)
+    cpu = torch.cat([_rows(128, n + 17 * b, dtype).transpose(1, 2) for b in range(n // 128 + 1)] + [_rows(3, n, dtype)], 1)
+    cpu = cpu[:, -(n + 3):].contiguous()  # the row kinds as channel kinds
+    idx = torch.randperm(n + 3, generator=torch.Generator().manual_seed(n))[:n]
+    segments = [idx[: n // 2].to(dev), idx[n // 2: n // 2].to(dev), idx[n // 2:].to(dev)]
+    arena = getattr(ro, build)(_offset(cpu.to(dev), offset), segments, append_capacity=256, superblock_size=superblock)
+    src = cpu[:, idx].float().numpy()
+
+    def check(total, packed, scale, zero, first=0):
+        blocks = -(-total // superblock)
+        np.testing.assert_array_equal(arena.packed[:, first:total].cpu().numpy(), packed)
+        np.testing.assert_array_equal(arena.scale[:, first // superblock:blocks].cpu().numpy(), scale)
+        np.testing.assert_array_equal(arena.zero_point[:, first // superblock:blocks].cpu().numpy(), zero)
+        assert not arena.packed[:, total:].any() and not arena.scale[:, blocks:].any()
+        assert not arena.zero_point[:, blocks:].any() and not arena.kernel_operands[:, blocks:].any()
+
+    packed, scale, zero = quantise(src, superblock)
+    check(n, packed, scale, zero)
+    ring = _rows(130, n + 1, dtype)
+    first = n // superblock * superblock
+    old = quant.round_to_dtype(dequantise(packed, scale, zero, first, n - first, superblock), dtype)
+    arena.append_superblock(ring.to(dev)[:, :128], source_tokens=130)
+    want = quantise(np.concatenate((old, ring[:, :128].float().numpy()), axis=1), superblock)
+    check(n + 128, *want, first=first)
+
+
+def test_int4_key_packer_at_the_ends_of_the_range():
+    """Channels whose range overflows fp32, holds infinities or NaN or is subnormal; the channels beside them
+    in a lane keep theirs."""
+    import r2omni_amd as ro
+    from oracle.quant import quantize_int4_key_per_channel
+
+    dev = _dev()
+    x = _rows(64, 5, "bfloat16", heads=1)
+    x[0, :, 3] *= 2.0 ** 126
+    x[0, ::2, 8], x[0, 1::2, 8] = 3.0e38, -3.0e38
+    x[0, 7, 17] = float("inf")
+    x[0, 40, 26] = float("nan")
+    x[0, :, 35] = float("nan")
+    x[0, :, 44] *= 2.0 ** -130
+    nan, inf = torch.isnan(x).numpy(), torch.isinf(x).numpy()
+    with np.errstate(invalid="ignore", over="ignore"):
+        packed, scale, zero = quantize_int4_key_per_channel(torch.where(torch.isnan(x), torch.zeros_like(x), x).float().numpy(), 32)
+    codes = np.stack((packed & 15, packed >> 4), -1).reshape(1, 64, 128)
+    codes[nan | inf] = 0
+    arena = ro.build_compact_int4_key_arena(x.to(dev), [torch.arange(64, device=dev)] + [torch.arange(0, device=dev)] * 2,
+                                            superblock_size=32)
+    got = arena.packed[:, :64].cpu().numpy()
+    np.testing.assert_array_equal(np.stack((got & 15, got >> 4), -1).reshape(1, 64, 128), codes)
+    np.testing.assert_array_equal(arena.scale[:, :2].cpu().numpy(), scale)
+    np.testing.assert_array_equal(arena.zero_point[:, :2].cpu().numpy(), zero)
