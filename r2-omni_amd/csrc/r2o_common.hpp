@@ -223,6 +223,57 @@ __device__ __forceinline__ void r2o_fwht128_pair(float& y0, float& y1, int t) {
     y1 = s1 * 0.08838834764831845f;
 }
 
+// The same transform of a row whose dims 8 l16 .. 8 l16 + 7 this lane of a 16-lane group holds: strides 1 .. 4
+// inside the lane, 8 .. 64 across lanes l16 ^ 1 .. l16 ^ 8.  The upper lane of a pair negates its own value
+// and adds, which is its partner's minus its own to the bit.
+template <int M>
+__device__ __forceinline__ void r2o_fwht_row8_stage(float (&y)[8], int l16) {
+    const uint32_t sign = (l16 & M) ? 0x80000000u : 0u;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[i] = r2o_lane_xor<M>(y[i]) + __uint_as_float(__float_as_uint(y[i]) ^ sign);
+}
+
+__device__ __forceinline__ void r2o_fwht_row8(float (&y)[8], int l16) {
+#pragma unroll
+    for (int h = 1; h < 8; h <<= 1)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if ((i & h) == 0) {
+                const float a = y[i], c = y[i + h];
+                y[i] = a + c;
+                y[i + h] = a - c;
+            }
+    r2o_fwht_row8_stage<1>(y, l16);
+    r2o_fwht_row8_stage<2>(y, l16);
+    r2o_fwht_row8_stage<4>(y, l16);
+    r2o_fwht_row8_stage<8>(y, l16);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[i] *= 0.08838834764831845f;
+}
+
+// Eight fp32 values rounded to a packed row (DT: 0 = bf16, 1 = fp16).
+template <int DT>
+__device__ __forceinline__ r2o_u4 r2o_pack8(const float (&y)[8]) {
+    r2o_u4 w;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        w[i] = DT == 0 ? r2o_pack_bf2(y[2 * i], y[2 * i + 1]) : r2o_f32_to_f16(y[2 * i]) | (r2o_f32_to_f16(y[2 * i + 1]) << 16);
+    return w;
+}
+
+template <bool VEC>
+__device__ __forceinline__ void r2o_store8(uint16_t* p, const r2o_u4& w) {
+    if constexpr (VEC) {
+        *reinterpret_cast<R2O_GLOBAL r2o_u4*>((R2O_GLOBAL uint16_t*)p) = w;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            p[2 * i] = (uint16_t)w[i];
+            p[2 * i + 1] = (uint16_t)(w[i] >> 16);
+        }
+    }
+}
+
 #define R2O_CHECK_LAUNCH()                                      \
     do {                                                        \
         if (hipGetLastError() != hipSuccess) return R2O_ELAUNCH; \

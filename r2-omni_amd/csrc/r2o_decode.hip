@@ -147,33 +147,6 @@ constexpr int kRotKeyRow = 16;
 constexpr int kRotBytes = 18 * kRotStride * 2;
 static_assert(kRotBytes == kRotLdsBytes, "one size for the rotation's LDS rows");
 
-// Orthonormal FWHT-128 of a row whose dims 8 l16 .. 8 l16 + 7 this lane holds (the V layout of a
-// Recent-FP tile): strides 1 .. 4 inside the lane, 8 .. 64 across lanes l16 ^ 1 .. l16 ^ 8 of a row.
-__device__ __forceinline__ void fwht_row8(float (&y)[8], int l16) {
-#pragma unroll
-    for (int h = 1; h < 8; h <<= 1)
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if ((i & h) == 0) {
-                const float a = y[i], c = y[i + h];
-                y[i] = a + c;
-                y[i + h] = a - c;
-            }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        float v = y[i], o;
-        o = r2o_lane_xor<1>(v);
-        v = (l16 & 1) ? o - v : v + o;
-        o = r2o_lane_xor<2>(v);
-        v = (l16 & 2) ? o - v : v + o;
-        o = r2o_lane_xor<4>(v);
-        v = (l16 & 4) ? o - v : v + o;
-        o = r2o_lane_xor<8>(v);
-        v = (l16 & 8) ? o - v : v + o;
-        y[i] = v * 0.08838834764831845f;
-    }
-}
-
 // Elements from one request's query (appended) rows to the next.  Only calls with a folded rotation
 // take strided rows (views of a fused projection; the launch helpers spell a stride of 0 out as the
 // dense figure); the other calls' rows are dense, as the reference requires, and the kernels
@@ -337,7 +310,7 @@ __device__ __forceinline__ r2o_u4 rot_row(const r2o_decode_params& p, const r2o_
             y[k] = rope ? rk : xv;
         }
     }
-    if (had) fwht_row8(y, c8);  // whole 16-lane groups take the same branch
+    if (had) r2o_fwht_row8(y, c8);  // whole 16-lane groups take the same branch
     r2o_u4 out;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {

@@ -1,4 +1,4 @@
-// Quantise/pack, gather, Recent-FP append/shift and FWHT kernels for gfx950.
+// Quantise/pack, gather and Recent-FP append/shift kernels for gfx950.
 //
 // Bit-exactness with the reference's torch CPU quantisers (compact_int4_key.py:83-110,
 // quantization.py:19-50, int2_reference.py:96-151): IEEE fp32 division (__fdiv_rn), round half
@@ -567,39 +567,6 @@ __global__ __launch_bounds__(256) void recent_shift_kernel(
     if (threadIdx.x == 0) *length = (int32_t)new_active;
 }
 
-// ---------------------------------------------------------------------------------- FWHT
-// One 128-thread block per row; butterflies in the reference's stage order (stride 1 .. 64),
-// then the fp32 normalisation 0.08838834764831845.
-__global__ __launch_bounds__(128) void fwht128_kernel(const uint16_t* __restrict__ src, uint16_t* dst, int dtype) {
-    __shared__ float buf[128];
-    const int64_t row = blockIdx.x;
-    const int d = threadIdx.x;
-    buf[d] = r2o_load_elem(src, row * 128 + d, dtype);
-    __syncthreads();
-    for (int stride = 1; stride < 128; stride <<= 1) {
-        const int pos = d & (stride - 1);
-        const int base = (d / stride) * stride * 2;  // only the first 64 threads are used
-        float a = 0.f, b = 0.f;
-        if (d < 64) {
-            const int blk = d / stride;
-            const int i0 = blk * 2 * stride + pos;
-            a = buf[i0];
-            b = buf[i0 + stride];
-        }
-        __syncthreads();
-        if (d < 64) {
-            const int blk = d / stride;
-            const int i0 = blk * 2 * stride + pos;
-            buf[i0] = a + b;
-            buf[i0 + stride] = a - b;
-        }
-        (void)base;
-        __syncthreads();
-    }
-    const float y = buf[d] * 0.08838834764831845f;
-    dst[row * 128 + d] = (uint16_t)(dtype == 0 ? r2o_f32_to_bf16(y) : r2o_f32_to_f16(y));
-}
-
 }  // namespace
 
 extern "C" {
@@ -688,14 +655,6 @@ int r2o_recent_shift(uint16_t* recent_k, uint16_t* recent_v, int64_t hkv, int64_
         return R2O_EINVAL;
     hipLaunchKernelGGL(recent_shift_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, recent_k, recent_v, hkv,
                        capacity, flush, active, global_buf, logical_buf, length, page_lengths, page_size);
-    R2O_CHECK_LAUNCH();
-    return R2O_OK;
-}
-
-int r2o_fwht128(const uint16_t* src, uint16_t* dst, int64_t rows, int64_t dtype, void* stream) {
-    if (rows < 0 || rows > 0x7fffffff || (dtype != 0 && dtype != 1)) return R2O_EINVAL;
-    if (rows == 0) return R2O_OK;
-    hipLaunchKernelGGL(fwht128_kernel, dim3((unsigned)rows), dim3(128), 0, (hipStream_t)stream, src, dst, (int)dtype);
     R2O_CHECK_LAUNCH();
     return R2O_OK;
 }
