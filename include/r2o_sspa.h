@@ -325,6 +325,40 @@ int r2o_recent_shift(uint16_t* recent_k, uint16_t* recent_v, int64_t hkv, int64_
                      int64_t flush, int64_t active, int64_t* global_buf, int64_t* logical_buf,
                      int32_t* length, int64_t* page_lengths, int64_t page_size, void* stream);
 
+/* The flush of a full Recent-FP ring, with the append that follows it, in two launches: the ring's oldest
+ * `flush` tokens into the compact K arena (k_bits 4 or 2, as r2o_pack_int4_k / r2o_pack_int2_k without an
+ * index: k_tail positions from k_start on are requantised with them) and the V arena (v_bits 4 or 2, as
+ * r2o_pack_int4_v / r2o_pack_int2_v), their token indices to dst_global / dst_logical (both NULL: none),
+ * then r2o_recent_shift and, with new_k / new_v ([hkv, 128], both NULL: none), r2o_recent_append of one
+ * token at the first free slot.  Replaces the sequence of append_generated_token for a full ring
+ * (dynamic_fourq_cache.py:185-267): six launches in one host call. */
+typedef struct r2o_ring_flush_params {
+    uint16_t* recent_k;           /* [hkv, capacity, 128] */
+    uint16_t* recent_v;
+    int64_t dtype, hkv, capacity, flush, active;
+    int64_t* global_buf;          /* [capacity] */
+    int64_t* logical_buf;
+    int32_t* length;
+    int64_t* page_lengths;        /* [capacity / page_size] */
+    int64_t page_size;
+    uint8_t* k_packed;
+    uint16_t* k_scale;
+    void* k_zero;                 /* u8 zero points (k_bits 4) or fp16 offsets (2) */
+    uint32_t* k_operands;         /* nullable */
+    int64_t k_bits, superblock, k_capacity, k_superblocks, k_start, k_tail;
+    uint8_t* v_packed;
+    void* v_scale;                /* f32 (v_bits 4) or fp16 (2) */
+    uint8_t* v_zero;              /* v_bits 2 */
+    int64_t v_bits, v_group, v_capacity, v_start;
+    int64_t* dst_global;          /* [flush] or NULL */
+    int64_t* dst_logical;
+    const uint16_t* new_k;        /* [hkv, 128] or NULL */
+    const uint16_t* new_v;
+    int64_t new_global, new_logical;
+} r2o_ring_flush_params;
+
+int r2o_ring_flush(const r2o_ring_flush_params* params, void* stream);
+
 /* Orthonormal 128-point FWHT of `rows` rows (in place allowed), dtype in/out.  Replaces
  * triton_fwht_128 (triton_qwen_mrope.py:325-346). */
 int r2o_fwht128(const uint16_t* src, uint16_t* dst, int64_t rows, int64_t dtype, void* stream);

@@ -108,6 +108,20 @@ class PlanConfig(ctypes.Structure):  # r2o_plan_config
     ]
 
 
+class RingFlush(ctypes.Structure):  # r2o_ring_flush_params
+    _fields_ = [
+        ("recent_k", c_vp), ("recent_v", c_vp), ("dtype", c_i64), ("hkv", c_i64), ("capacity", c_i64), ("flush", c_i64),
+        ("active", c_i64), ("global_buf", c_vp), ("logical_buf", c_vp), ("length", c_vp), ("page_lengths", c_vp),
+        ("page_size", c_i64),
+        ("k_packed", c_vp), ("k_scale", c_vp), ("k_zero", c_vp), ("k_operands", c_vp), ("k_bits", c_i64),
+        ("superblock", c_i64), ("k_capacity", c_i64), ("k_superblocks", c_i64), ("k_start", c_i64), ("k_tail", c_i64),
+        ("v_packed", c_vp), ("v_scale", c_vp), ("v_zero", c_vp), ("v_bits", c_i64), ("v_group", c_i64),
+        ("v_capacity", c_i64), ("v_start", c_i64),
+        ("dst_global", c_vp), ("dst_logical", c_vp), ("new_k", c_vp), ("new_v", c_vp), ("new_global", c_i64),
+        ("new_logical", c_i64),
+    ]
+
+
 _SIGNATURES = {
     "r2o_plan_work_items": (ctypes.POINTER(PlanRun), c_i64, ctypes.POINTER(PlanConfig), c_vp, c_i64, c_i64, c_i64,
                             c_vp, c_i64, c_vp, c_i64, ctypes.POINTER(c_i64)),
@@ -125,6 +139,7 @@ _SIGNATURES = {
     "r2o_gather_rows": (c_vp, c_i64, c_i64, c_vp, c_i64, c_vp, c_i64, c_vp),
     "r2o_recent_append": (c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_i64, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp),
     "r2o_recent_shift": (c_vp, c_vp, c_i64, c_i64, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp),
+    "r2o_ring_flush": (ctypes.POINTER(RingFlush), c_vp),
     "r2o_fwht128": (c_vp, c_vp, c_i64, c_i64, c_vp),
     "r2o_qk_mrope": (c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_i64, c_i64, c_vp, c_vp, c_i64, c_vp, c_vp,
                      c_i64, c_i64, c_i64, c_vp),

@@ -75,14 +75,11 @@ class CompactMetadataArena:
     int4_page_count: int
     int4_token_count: int
 
-    def _append_pages(self, pool: "PrecisionPool", global_indices: torch.Tensor, logical_positions: torch.Tensor,
-                      page_size: int, tier: str) -> None:
-        n = int(global_indices.numel())
-        if n <= 0 or n != int(logical_positions.numel()) or n % int(page_size):
+    def _take_pages(self, pool: "PrecisionPool", n: int, page_size: int, tier: str) -> tuple[torch.Tensor, torch.Tensor]:
+        """Add ``n`` tokens of whole pages to the tier and return its (global, logical) index slots for them,
+        which the caller fills on the pool's stream."""
+        if n <= 0 or n % int(page_size):
             raise ValueError(f"compact {tier.upper()} metadata append requires matching complete pages")
-        if global_indices.dtype != torch.long or logical_positions.dtype != torch.long \
-                or global_indices.device != self.storage.device or logical_positions.device != self.storage.device:
-            raise ValueError(f"compact {tier.upper()} metadata append requires same-device int64 indices")
         ids, offs, lens, g, l = (getattr(self, f"{tier}_{name}_buffer") for name in
                                  ("original_page_ids", "physical_offsets", "lengths", "global_index",
                                   "logical_position"))
@@ -93,13 +90,24 @@ class CompactMetadataArena:
             raise RuntimeError(f"compact {tier.upper()} page metadata capacity exhausted")
         if token_end > g.numel():
             raise RuntimeError(f"compact {tier.upper()} token metadata capacity exhausted")
-        g[tokens:token_end].copy_(global_indices)
-        l[tokens:token_end].copy_(logical_positions)
         setattr(self, f"{tier}_page_count", page_end)
         setattr(self, f"{tier}_token_count", token_end)
         pool.page_index = PhysicalPageIndex(original_page_ids=ids[:page_end], physical_offsets=offs[:page_end],
                                             lengths=lens[:page_end], global_token_indices=g[:token_end],
                                             logical_positions=l[:token_end])
+        return g[tokens:token_end], l[tokens:token_end]
+
+    def _append_pages(self, pool: "PrecisionPool", global_indices: torch.Tensor, logical_positions: torch.Tensor,
+                      page_size: int, tier: str) -> None:
+        n = int(global_indices.numel())
+        if n <= 0 or n != int(logical_positions.numel()) or n % int(page_size):
+            raise ValueError(f"compact {tier.upper()} metadata append requires matching complete pages")
+        if global_indices.dtype != torch.long or logical_positions.dtype != torch.long \
+                or global_indices.device != self.storage.device or logical_positions.device != self.storage.device:
+            raise ValueError(f"compact {tier.upper()} metadata append requires same-device int64 indices")
+        g, l = self._take_pages(pool, n, page_size, tier)
+        g.copy_(global_indices)
+        l.copy_(logical_positions)
 
     def append_int2_pages(self, pool: "PrecisionPool", global_indices: torch.Tensor,
                           logical_positions: torch.Tensor, page_size: int) -> None:
@@ -1223,59 +1231,99 @@ def flush_full_recent_pool(cache: ThreePrecisionCache, stats: DynamicCacheStats)
     ``append_generated_token`` (dynamic_fourq_cache.py:185-253).  Returns whether it flushed.  The
     caller re-prepares its executors afterwards."""
     pool = cache.recent_fp_pool
-    flush = int(cache.recent_flush_size)
-    if pool.active_length is None or pool.capacity < flush or pool.length_device is None:
+    if pool.active_length is None or pool.capacity < int(cache.recent_flush_size) or pool.length_device is None:
         raise RuntimeError("Recent-FP pool was not preallocated for dynamic generation")
     if pool.active_length != pool.capacity:
         return False
-    h, cap = int(pool.fp_k.shape[0]), int(pool.capacity)
-    stream = _lib.stream_of(pool.fp_k.device)
-    key_block = pool.fp_k[:, :flush]
-    value_block = pool.fp_v[:, :flush]
-    # Views of the ring's oldest indices: every consumer below copies them on this stream before
-    # the ring shift is launched, so no snapshot is needed.
-    global_block = pool.global_index_buffer[:flush]
-    logical_block = pool.logical_position_buffer[:flush]
-    if cache.matched_fp:  # _append_matched_fp_block (dynamic_fourq_cache.py:145-170)
-        _append_lowbit_page_metadata(cache.fp_pool, global_block, logical_block, cache.page_size)
-        cache.bf16_key.append_block(key_block)
-        n = cache.bf16_key.active_length
-        cache.bf16_key.segment_offsets = (0, n, n)
-        cache.fp_pool.fp_k = cache.bf16_key.view(0, n)
-        cache.fp_pool.fp_v = torch.cat((cache.fp_pool.fp_v, value_block), dim=1)
-        cache.generated_k_offset = n
+    if cache.matched_fp:
+        _flush_matched(cache)
     elif cache.bf16_key is not None:  # dynamic_fourq_cache.py:226-230
         raise RuntimeError("K-BF16/V-FourQ requires an append_fp_only Recent-FP capacity covering the "
                            "requested generation horizon")
     else:
-        if cache.compact_key is None:
-            raise RuntimeError("compact K cache is missing its compact K arena")
-        int4_values = cache.generated_value_precision == "int4"
-        if int4_values and cache.compact_int4_value is None:
-            raise RuntimeError("generated INT4 V policy is missing its compact arena")
-        if not int4_values and cache.compact_value is None:
-            raise RuntimeError("compact INT2 K cache is missing its compact INT2 V arena")
-        stats.local_tail_dequant_tokens += cache.compact_key.append_superblock(key_block, source_tokens=cap) \
-            if flush == 128 else _flush_size_error(flush)
-        if int4_values:  # dynamic_fourq_cache.py:212-219
-            cache.compact_int4_value.append_block(value_block, source_tokens=cap)
-            stats.flushed_int4_value_tokens += flush
-            target = cache.int4_pool
-        else:
-            cache.compact_value.append_superblock(value_block, source_tokens=cap)
-            target = cache.int2_pool
-        if cache.metadata_arena is not None:  # in place (dynamic_fourq_cache.py:236-243)
-            append = cache.metadata_arena.append_int4_pages if int4_values else cache.metadata_arena.append_int2_pages
-            append(target, global_block, logical_block, cache.page_size)
-        else:
-            _append_lowbit_page_metadata(target, global_block, logical_block, cache.page_size)
-    _lib.call("r2o_recent_shift", _lib.ptr(pool.fp_k), _lib.ptr(pool.fp_v), h, cap, flush, pool.active_length,
-              _lib.ptr(pool.global_index_buffer), _lib.ptr(pool.logical_position_buffer),
-              _lib.ptr(pool.length_device), _lib.ptr(pool.page_index.lengths), cache.page_size, stream)
-    pool.active_length -= flush
+        _flush_compact(cache, stats, None)
+    pool.active_length -= int(cache.recent_flush_size)
     stats.flushed_superblocks += 1
-    stats.flushed_tokens += flush
+    stats.flushed_tokens += int(cache.recent_flush_size)
     return True
+
+
+def _flush_matched(cache: ThreePrecisionCache) -> None:
+    """_append_matched_fp_block (dynamic_fourq_cache.py:145-170) and the ring's shift."""
+    pool, flush = cache.recent_fp_pool, int(cache.recent_flush_size)
+    # Views of the ring's oldest slots: every consumer copies them on this stream before the ring shift is
+    # launched, so no snapshot is needed.
+    _append_lowbit_page_metadata(cache.fp_pool, pool.global_index_buffer[:flush], pool.logical_position_buffer[:flush],
+                                 cache.page_size)
+    cache.bf16_key.append_block(pool.fp_k[:, :flush])
+    n = cache.bf16_key.active_length
+    cache.bf16_key.segment_offsets = (0, n, n)
+    cache.fp_pool.fp_k = cache.bf16_key.view(0, n)
+    cache.fp_pool.fp_v = torch.cat((cache.fp_pool.fp_v, pool.fp_v[:, :flush]), dim=1)
+    cache.generated_k_offset = n
+    _lib.call("r2o_recent_shift", _lib.ptr(pool.fp_k), _lib.ptr(pool.fp_v), int(pool.fp_k.shape[0]), int(pool.capacity),
+              flush, pool.active_length, _lib.ptr(pool.global_index_buffer), _lib.ptr(pool.logical_position_buffer),
+              _lib.ptr(pool.length_device), _lib.ptr(pool.page_index.lengths), cache.page_size,
+              _lib.stream_of(pool.fp_k.device))
+
+
+def _flush_compact(cache: ThreePrecisionCache, stats: DynamicCacheStats, append) -> None:
+    """The flush of a full ring into the compact arenas and its page metadata, the ring's shift and, with
+    ``append`` = (K rows, V rows [Hkv, D], global index, logical position), the token that follows: one
+    host call of two launches (r2o_ring_flush).  Every refusal comes before the first launch."""
+    pool, flush, ck = cache.recent_fp_pool, int(cache.recent_flush_size), cache.compact_key
+    if ck is None:
+        raise RuntimeError("compact K cache is missing its compact K arena")
+    int4_values = cache.generated_value_precision == "int4"
+    if int4_values and cache.compact_int4_value is None:
+        raise RuntimeError("generated INT4 V policy is missing its compact arena")
+    if not int4_values and cache.compact_value is None:
+        raise RuntimeError("compact INT2 K cache is missing its compact INT2 V arena")
+    if flush != 128:
+        _flush_size_error(flush)
+    values = cache.compact_int4_value if int4_values else cache.compact_value
+    target = cache.int4_pool if int4_values else cache.int2_pool
+    bits = ck.bit_width
+    if (int(pool.fp_k.shape[0]), int(pool.fp_k.shape[2])) != (ck.head_count, ck.head_dim):
+        raise ValueError(f"compact INT{bits} K flush requires 128 matching tokens")
+    if (int(pool.fp_v.shape[0]), int(pool.fp_v.shape[2])) != values.original_shape[::2]:
+        raise ValueError(f"compact INT{4 if int4_values else 2} V flush must contain matching tokens")
+    if not (pool.fp_k.is_contiguous() and pool.fp_v.is_contiguous()):
+        raise ValueError(f"compact INT{bits} K flush block must have contiguous rows")
+    if ck.active_length + flush > ck.capacity:
+        raise RuntimeError(f"compact INT{bits} K capacity exhausted")
+    if values.active_length + flush > values.capacity:
+        raise RuntimeError(f"compact INT{4 if int4_values else 2} V capacity exhausted: need "
+                           f"{values.active_length + flush}, have {values.capacity}")
+    dev = pool.fp_k.device
+    _lib.require_device(pool.fp_k, f"compact INT{bits} K flush block")
+    prefix = ck.active_length // ck.superblock_size * ck.superblock_size
+    p = _lib.RingFlush(
+        recent_k=pool.fp_k.data_ptr(), recent_v=pool.fp_v.data_ptr(), dtype=_lib.dtype_code(pool.fp_k.dtype),
+        hkv=int(pool.fp_k.shape[0]), capacity=int(pool.capacity), flush=flush, active=int(pool.active_length),
+        global_buf=pool.global_index_buffer.data_ptr(), logical_buf=pool.logical_position_buffer.data_ptr(),
+        length=pool.length_device.data_ptr(), page_lengths=pool.page_index.lengths.data_ptr(), page_size=cache.page_size,
+        k_packed=ck.packed.data_ptr(), k_scale=ck.scale.data_ptr(), k_zero=ck.zero_point.data_ptr(),
+        k_operands=_lib.ptr(ck.kernel_operands), k_bits=bits, superblock=ck.superblock_size, k_capacity=ck.capacity,
+        k_superblocks=ck.superblock_count, k_start=prefix, k_tail=ck.active_length - prefix,
+        v_packed=values.packed.data_ptr(), v_scale=values.scale.data_ptr(), v_zero=_lib.ptr(values.zero_point),
+        v_bits=4 if int4_values else 2, v_group=128 if int4_values else values.group_size, v_capacity=values.capacity,
+        v_start=values.active_length)
+    if append is not None:
+        nk, nv, p.new_global, p.new_logical = append
+        p.new_k, p.new_v = nk.data_ptr(), nv.data_ptr()
+    if cache.metadata_arena is not None:  # in place (dynamic_fourq_cache.py:236-243)
+        g, l = cache.metadata_arena._take_pages(target, flush, cache.page_size, "int4" if int4_values else "int2")
+        p.dst_global, p.dst_logical = g.data_ptr(), l.data_ptr()
+    else:
+        _append_lowbit_page_metadata(target, pool.global_index_buffer[:flush], pool.logical_position_buffer[:flush],
+                                     cache.page_size)
+    _lib.call("r2o_ring_flush", p, _lib.stream_of(dev))
+    stats.local_tail_dequant_tokens += p.k_tail
+    if int4_values:  # dynamic_fourq_cache.py:212-219
+        stats.flushed_int4_value_tokens += flush
+    ck.active_length += flush
+    values.active_length += flush
 
 
 def append_generated_token(cache: ThreePrecisionCache, new_key: torch.Tensor, new_value: torch.Tensor, *,
@@ -1294,14 +1342,21 @@ def append_generated_token(cache: ThreePrecisionCache, new_key: torch.Tensor, ne
     if new_key.dtype != pool.fp_k.dtype or new_value.dtype != pool.fp_v.dtype:
         raise ValueError("new K/V dtype must match the Recent-FP ring")
     h, cap = int(pool.fp_k.shape[0]), int(pool.capacity)
-    stream = _lib.stream_of(new_key.device)
-    flushed = flush_full_recent_pool(cache, stats)
     nk = new_key.reshape(h, -1).contiguous()
     nv = new_value.reshape(h, -1).contiguous()
+    position = (int(global_token_index), int(logical_position))
+    if pool.active_length == cap and not cache.matched_fp and cache.bf16_key is None:
+        _flush_compact(cache, stats, (nk, nv, *position))
+        pool.active_length += 1 - flush
+        stats.flushed_superblocks += 1
+        stats.flushed_tokens += flush
+        stats.appended_tokens += 1
+        return True
+    flushed = flush_full_recent_pool(cache, stats)
     _lib.call("r2o_recent_append", _lib.ptr(pool.fp_k), _lib.ptr(pool.fp_v), h, cap, _lib.ptr(nk), _lib.ptr(nv),
-              pool.active_length, int(global_token_index), int(logical_position), _lib.ptr(pool.length_device),
+              pool.active_length, *position, _lib.ptr(pool.length_device),
               _lib.ptr(pool.global_index_buffer), _lib.ptr(pool.logical_position_buffer),
-              _lib.ptr(pool.page_index.lengths), cache.page_size, stream)
+              _lib.ptr(pool.page_index.lengths), cache.page_size, _lib.stream_of(new_key.device))
     pool.active_length += 1
     stats.appended_tokens += 1
     return flushed

@@ -162,3 +162,68 @@ def test_int4_key_packer_at_the_ends_of_the_range():
     np.testing.assert_array_equal(np.stack((got & 15, got >> 4), -1).reshape(1, 64, 128), codes)
     np.testing.assert_array_equal(arena.scale[:, :2].cpu().numpy(), scale)
     np.testing.assert_array_equal(arena.zero_point[:, :2].cpu().numpy(), zero)
+
+
+@pytest.mark.parametrize("append", [False, True])
+@pytest.mark.parametrize("ring,superblock,variant,gen", [
+    (128, 32, "v_fourq_k_int4_compact", "int2"), (256, 128, "v_fourq_k_int2_compact", "int2"),
+    (384, 64, "v_fourq_k_int4_compact", "int4"), (160, 32, "v_fourq_k_int4_compact", "int2")])
+def test_ring_flush_is_its_parts(ring, superblock, variant, gen, append):
+    """Two flushes in one call each, against the arenas' own appends and a ring moved by torch (rings that
+    move nothing, less than a flush, one flush and two)."""
+    import r2omni_amd as ro
+    from r2omni_amd.policy import PageClass, plan_from_pages
+
+    dev = _dev()
+    pages = 9
+    plan = plan_from_pages([32 * i for i in range(pages)], [32] * pages,
+                           [int((PageClass.FP_PAGE, PageClass.INT4_PAGE, PageClass.INT2_PAGE)[i % 3]) for i in range(pages)],
+                           recent_fp_capacity=ring, device=dev)
+    gen_k = torch.Generator().manual_seed(ring)
+    k, v = (torch.randn(3, 32 * pages, 128, generator=gen_k).to(torch.bfloat16).to(dev) for _ in range(2))
+    kw = dict(page_size=32, key_quantization_superblock=superblock, cache_variant=variant, generated_value_precision=gen,
+              compact_key_append_capacity=512)
+    cache, parts = (ro.build_three_precision_cache(k, v, plan, **kw) for _ in range(2))
+    stats, at = ro.DynamicCacheStats(), 32 * pages
+    rows = torch.randn(2, 700, 3, 1, 128, generator=gen_k).to(torch.bfloat16).to(dev)
+    want_ring = []  # (k row, v row, global, logical)
+    for step in range(2):
+        while cache.recent_fp_pool.active_length < ring:
+            i = at - 32 * pages
+            ro.append_generated_token(cache, rows[0, i], rows[1, i], global_token_index=at, logical_position=3 * at, stats=stats)
+            want_ring.append((rows[0, i, :, 0], rows[1, i, :, 0], at, 3 * at))
+            at += 1
+        oldest = want_ring[:128]
+        kb, vb = (torch.stack([r[e] for r in oldest], 1).contiguous() for e in (0, 1))
+        parts.compact_key.append_superblock(kb)
+        if gen == "int4":
+            parts.compact_int4_value.append_block(vb)
+            parts.metadata_arena.append_int4_pages(parts.int4_pool, *(torch.tensor([r[e] for r in oldest], device=dev) for e in (2, 3)), 32)
+        else:
+            parts.compact_value.append_superblock(vb)
+            parts.metadata_arena.append_int2_pages(parts.int2_pool, *(torch.tensor([r[e] for r in oldest], device=dev) for e in (2, 3)), 32)
+        want_ring = want_ring[128:]
+        if append:
+            i = at - 32 * pages
+            assert ro.append_generated_token(cache, rows[0, i], rows[1, i], global_token_index=at, logical_position=3 * at, stats=stats)
+            want_ring.append((rows[0, i, :, 0], rows[1, i, :, 0], at, 3 * at))
+            at += 1
+        else:
+            assert ro.flush_full_recent_pool(cache, stats)
+        n, pool = len(want_ring), cache.recent_fp_pool
+        assert pool.active_length == n == int(pool.length_device)
+        assert pool.page_index.lengths.tolist() == [min(max(n - 32 * p, 0), 32) for p in range(ring // 32)]
+        for e, t in ((0, pool.fp_k), (1, pool.fp_v)):
+            if n:
+                assert torch.equal(t[:, :n], torch.stack([r[e] for r in want_ring], 1))
+        assert pool.global_index_buffer[:n].tolist() == [r[2] for r in want_ring]
+        assert pool.logical_position_buffer[:n].tolist() == [r[3] for r in want_ring]
+        a, b = cache.compact_key, parts.compact_key
+        for x, y in ((a.packed, b.packed), (a.scale, b.scale), (a.zero_point, b.zero_point), (a.kernel_operands, b.kernel_operands)):
+            assert torch.equal(x, y)
+        a, b = (c.compact_int4_value if gen == "int4" else c.compact_value for c in (cache, parts))
+        assert a.active_length == b.active_length and torch.equal(a.packed, b.packed) and torch.equal(a.scale, b.scale)
+        for x, y in zip(cache.pools[:3], parts.pools[:3]):
+            for f in ("original_page_ids", "physical_offsets", "lengths", "global_token_indices", "logical_positions"):
+                assert torch.equal(getattr(x.page_index, f), getattr(y.page_index, f))
+    assert stats.flushed_tokens == 256
