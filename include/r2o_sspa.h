@@ -359,6 +359,62 @@ typedef struct r2o_ring_flush_params {
 
 int r2o_ring_flush(const r2o_ring_flush_params* params, void* stream);
 
+/* Tokens and pages of each tier of a cache plan (host code).  table [3, n_pages]: page classes (PageClass
+ * values), first tokens, lengths; the tiers are FP (with protected and recent pages), INT4, INT2 and
+ * evicted.  R2O_EINVAL for an unknown class or a page outside [0, tokens).  Replaces the sort of
+ * _compact_page_layouts (precision_pool.py:611-669), with r2o_cache_page_words. */
+int r2o_cache_pages(const int64_t* table, int64_t n_pages, int64_t tokens, int64_t* tier_pages, int64_t* tier_tokens);
+
+/* The page words of a cache's metadata arena and the expansion table behind them (host code).  Per tier FP,
+ * INT4, INT2: plan page ids, offsets in the pool and lengths, each followed by its reserved pages' (-1, the
+ * offsets that continue the pool, page_size); the ring's pages (-1, offsets, 0); one word 0 (the ring's
+ * device length).  Then, for every page in tier order (evicted last): first tokens, lengths, and positions
+ * in the tier-ordered token sequence.  reserve4 / reserve2 / ring_capacity are whole pages of tokens; words
+ * holds max_words. */
+int r2o_cache_page_words(const int64_t* table, int64_t n_pages, int64_t page_size, int64_t reserve4, int64_t reserve2,
+                         int64_t ring_capacity, int64_t* words, int64_t max_words);
+
+/* A prompt's packed cache in two launches: the first expands the page table (`pages`, the device copy of
+ * r2o_cache_page_words' words) into the metadata storage (page words; then global and logical indices of
+ * the survivors with each tier's reserve, evicted globals, ring indices; unused entries -1) and the
+ * tier-ordered token index, and zeroes what the payload arenas keep beyond their tokens and the ring's
+ * rows; the second packs every tier (r2o_pack_int4_k / r2o_pack_int2_k or the 16-bit key rows,
+ * r2o_pack_int4_v, r2o_pack_int2_v, r2o_gather_rows).  Replaces the launches of
+ * build_three_precision_cache (precision_pool.py:878-984).  Every payload pointer 16-byte aligned. */
+typedef struct r2o_cache_build_params {
+    const uint16_t* key;          /* [hkv, tokens, 128] */
+    const uint16_t* value;
+    int64_t key_dtype, value_dtype, hkv, tokens;
+    const int64_t* plan_global;   /* [tokens] token indices of the plan */
+    const int64_t* plan_logical;
+    const int64_t* pages;         /* device [page_words + 3 * n_pages] */
+    int64_t page_words, n_pages;
+    int64_t tier_tokens[4];       /* r2o_cache_pages */
+    int64_t reserve4, reserve2;
+    int64_t* storage;             /* device [page_words + 2 * (survivors + reserves) + evicted + 2 * ring_capacity] */
+    int64_t* index;               /* device scratch [survivors] */
+    uint16_t* ring_k;             /* [hkv, ring_capacity, 128] */
+    uint16_t* ring_v;
+    int64_t ring_capacity;
+    int64_t k_bits;               /* 4, 2, or 16 for k_packed as 16-bit rows */
+    int64_t superblock;
+    uint8_t* k_packed;
+    uint16_t* k_scale;
+    void* k_zero;
+    uint32_t* k_operands;
+    int64_t k_capacity, k_superblocks;
+    uint16_t* fp_v;               /* [hkv, FP tokens, 128] */
+    uint8_t* i4_v;                /* [hkv, i4_capacity, 64] */
+    float* i4_scale;
+    int64_t i4_capacity;
+    uint8_t* i2_v;                /* [hkv, i2_capacity, 32] */
+    uint16_t* i2_scale;
+    uint8_t* i2_zero;
+    int64_t i2_capacity, i2_group;
+} r2o_cache_build_params;
+
+int r2o_cache_build(const r2o_cache_build_params* params, void* stream);
+
 /* Orthonormal 128-point FWHT of `rows` rows (in place allowed), dtype in/out.  Replaces
  * triton_fwht_128 (triton_qwen_mrope.py:325-346). */
 int r2o_fwht128(const uint16_t* src, uint16_t* dst, int64_t rows, int64_t dtype, void* stream);

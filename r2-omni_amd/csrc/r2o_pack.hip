@@ -5,6 +5,8 @@
 // to even (__builtin_rintf -> v_rndne_f32), no contraction (the file is built with
 // -ffp-contract=off), fp32 step quantisation with fp16-RNE storage of the step.  Where many values share a
 // divisor its reciprocal is kept and r2o_div_by gives the same correctly rounded quotients.
+#include <initializer_list>
+
 #include "r2o_common.hpp"
 
 namespace {
@@ -605,6 +607,94 @@ void launch_pack_cache(CachePack& a, int key_bits, int64_t superblock, int64_t d
     else launch_pack_cache_of<1>(a, key_bits, superblock, grid, st);
 }
 
+// ------------------------------------------------------------------- a cache's indices in one launch
+// Before the payload: one wave per page writes its tokens' plan index, global and logical index in tier
+// order, and blocks of up to kFillBytes copy the page words and fill what no token reaches (-1 for unused
+// indices, 0 for the arenas' spare capacity and the ring).  In place of ~20 library launches (scan, gathers,
+// fills of whole arenas) that a build spent most of its time queueing.  Measured, with the payload's
+// launch: 4k tokens x 2 heads 5.3 + 5.6 us (357 -> 92 us a build, now the host's), 65k x 4 10.5 + 31 us
+// (391 -> 99), 131k x 8 9.8 + 132 us (572 -> 146, of which the packers' own changes 234).
+constexpr int64_t kFillBytes = 32768;
+constexpr int kMaxFills = 20;
+
+struct Fill {
+    unsigned char* dst;         // of head 0
+    const unsigned char* src;   // nullable: fill with `byte`
+    int64_t head_stride, bytes;
+    int heads, first_block;     // consecutive blocks: heads x chunks of kFillBytes
+    uint32_t byte;              // 0 or 0xff
+};
+
+struct CacheIndex {
+    const int64_t* start;       // [n_pages] first tokens, then lengths, then positions
+    int64_t n_pages;
+    const int64_t* plan_global;
+    const int64_t* plan_logical;
+    int64_t* index;
+    int64_t* global;            // survivors' global indices (each tier followed by its reserve), then logical
+    int64_t* logical;
+    int64_t* evicted;
+    int64_t int2_at, reserve4, survivors;  // positions from int2_at on come after the INT4 reserve
+    int page_blocks, n_fills;
+    Fill fills[kMaxFills];
+};
+
+__global__ __launch_bounds__(256) void cache_index_kernel(CacheIndex a) {
+    const int lane = threadIdx.x & 63;
+    int block = blockIdx.x;
+    if (block < a.page_blocks) {
+        const int64_t page = (int64_t)block * 4 + (threadIdx.x >> 6);
+        if (page >= a.n_pages) return;
+        const int64_t start = a.start[page], len = a.start[a.n_pages + page], position = a.start[2 * a.n_pages + page];
+        for (int64_t j = lane; j < len; j += 64) {
+            const int64_t token = start + j, p = position + j, g = a.plan_global[token];
+            if (p >= a.survivors) {
+                a.evicted[p - a.survivors] = g;
+                continue;
+            }
+            const int64_t slot = p + (p >= a.int2_at ? a.reserve4 : 0);
+            a.index[p] = token;
+            a.global[slot] = g;
+            a.logical[slot] = a.plan_logical[token];
+        }
+        return;
+    }
+    block -= a.page_blocks;
+    int i = 0;
+    while (i + 1 < a.n_fills && block >= a.fills[i + 1].first_block) ++i;
+    const Fill& f = a.fills[i];
+    block -= f.first_block;
+    const int64_t first = (int64_t)(block / f.heads) * kFillBytes, n = min(kFillBytes, f.bytes - first);
+    unsigned char* dst = f.dst + (block % f.heads) * f.head_stride + first;
+    if (f.src) {  // the page words: 8-byte aligned, one head
+        for (int64_t e = threadIdx.x; e < n / 8; e += 256)
+            reinterpret_cast<int64_t*>(dst)[e] = reinterpret_cast<const int64_t*>(f.src + first)[e];
+        return;
+    }
+    const int64_t head = min((int64_t)(-reinterpret_cast<uintptr_t>(dst) & 15), n), body = (n - head) / 16;
+    const uint32_t word = f.byte * 0x01010101u;
+    if (threadIdx.x < head) dst[threadIdx.x] = (unsigned char)f.byte;
+    for (int64_t e = threadIdx.x; e < body; e += 256)
+        reinterpret_cast<r2o_u4*>(dst + head)[e] = r2o_u4{word, word, word, word};
+    const int64_t done = head + 16 * body;
+    if (threadIdx.x < n - done) dst[done + threadIdx.x] = (unsigned char)f.byte;
+}
+
+// Adds the fill of bytes [from, to) of each head's `stride` bytes.
+void add_fill(CacheIndex& a, int64_t& blocks, void* base, const void* src, int64_t heads, int64_t stride, int64_t from,
+              int64_t to, uint32_t byte) {
+    if (to <= from || heads <= 0) return;
+    Fill& f = a.fills[a.n_fills++];
+    f.dst = reinterpret_cast<unsigned char*>(base) + from;
+    f.src = reinterpret_cast<const unsigned char*>(src);
+    f.head_stride = stride;
+    f.bytes = to - from;
+    f.heads = (int)heads;
+    f.first_block = (int)blocks;
+    f.byte = byte;
+    blocks += heads * blocks_of(to - from, kFillBytes);
+}
+
 // ------------------------------------------------------------------------ Recent-FP ring
 __global__ __launch_bounds__(256) void recent_append_kernel(
     uint16_t* rk, uint16_t* rv, int64_t hkv, int64_t capacity, const uint16_t* __restrict__ nk,
@@ -814,6 +904,94 @@ int r2o_ring_flush(const r2o_ring_flush_params* p, void* stream) {
     launch_recent_shift({{p->recent_k, p->recent_v}, {p->new_k, p->new_v}, p->hkv, p->capacity, p->flush,
                          p->active - p->flush, {p->global_buf, p->logical_buf}, {p->new_global, p->new_logical},
                          p->length, p->page_lengths, p->page_size}, st);
+    R2O_CHECK_LAUNCH();
+    return R2O_OK;
+}
+
+int r2o_cache_build(const r2o_cache_build_params* p, void* stream) {
+    if (!p || !p->pages || !p->storage || !p->ring_k || !p->ring_v) return R2O_EINVAL;
+    if (p->tokens > 0 && (!p->key || !p->value || !p->plan_global || !p->plan_logical)) return R2O_EINVAL;
+    if ((p->key_dtype != 0 && p->key_dtype != 1) || (p->value_dtype != 0 && p->value_dtype != 1)) return R2O_EINVAL;
+    if (p->hkv <= 0 || p->tokens < 0 || p->n_pages < 0 || p->page_words <= 0 || p->reserve4 < 0 || p->reserve2 < 0 ||
+        p->ring_capacity < 0)
+        return R2O_EINVAL;
+    const int64_t s_fp = p->tier_tokens[0], s_i4 = p->tier_tokens[1], s_i2 = p->tier_tokens[2], s_ev = p->tier_tokens[3];
+    if (s_fp < 0 || s_i4 < 0 || s_i2 < 0 || s_ev < 0) return R2O_EINVAL;
+    const int64_t n = s_fp + s_i4 + s_i2;
+    if (n > p->k_capacity || n > 0x7fffffff || (n > 0 && !p->index) || !p->k_packed) return R2O_EINVAL;
+    const bool packed_k = p->k_bits == 4 || p->k_bits == 2;
+    if (!packed_k && p->k_bits != 16) return R2O_EINVAL;
+    if (packed_k && (!p->k_scale || !p->k_zero || !(p->superblock == 32 || p->superblock == 64 || p->superblock == 128) ||
+                     p->k_superblocks * p->superblock != p->k_capacity))
+        return R2O_EINVAL;
+    if ((s_fp > 0 && !p->fp_v) || s_i4 > p->i4_capacity || (p->i4_capacity > 0 && (!p->i4_v || !p->i4_scale)) ||
+        s_i2 > p->i2_capacity || p->i4_capacity < 0 || p->i2_capacity < 0 ||
+        (p->i2_capacity > 0 && (!p->i2_v || !p->i2_scale || !p->i2_zero ||
+                                !(p->i2_group == 32 || p->i2_group == 64 || p->i2_group == 128))))
+        return R2O_EINVAL;
+    for (const void* q : {(const void*)p->key, (const void*)p->value, (const void*)p->k_packed, (const void*)p->k_scale,
+                          (const void*)p->fp_v, (const void*)p->i4_v, (const void*)p->i2_v, (const void*)p->ring_k,
+                          (const void*)p->ring_v})
+        if (reinterpret_cast<uintptr_t>(q) % 16) return R2O_EINVAL;
+    const hipStream_t st = (hipStream_t)stream;
+    const int64_t h = p->hkv, span = n + p->reserve4 + p->reserve2, head = s_fp + s_i4, cap = p->ring_capacity;
+    CacheIndex x{};
+    x.start = p->pages + p->page_words;
+    x.n_pages = p->n_pages;
+    x.plan_global = p->plan_global;
+    x.plan_logical = p->plan_logical;
+    x.index = p->index;
+    x.global = p->storage + p->page_words;
+    x.logical = x.global + span;
+    x.evicted = x.logical + span;
+    x.int2_at = head;
+    x.reserve4 = p->reserve4;
+    x.survivors = n;
+    x.page_blocks = (int)blocks_of(p->n_pages, 4);
+    int64_t blocks = 0;
+    add_fill(x, blocks, p->storage, p->pages, 1, 0, 0, 8 * p->page_words, 0);
+    for (int64_t* idx : {x.global, x.logical}) {
+        add_fill(x, blocks, idx, nullptr, 1, 0, 8 * head, 8 * (head + p->reserve4), 0xff);
+        add_fill(x, blocks, idx, nullptr, 1, 0, 8 * (span - p->reserve2), 8 * span, 0xff);
+    }
+    add_fill(x, blocks, x.evicted + s_ev, nullptr, 1, 0, 0, 16 * cap, 0xff);
+    for (uint16_t* ring : {p->ring_k, p->ring_v}) add_fill(x, blocks, ring, nullptr, 1, 0, 0, h * cap * 256, 0);
+    if (packed_k) {
+        const int64_t row = p->k_bits * 16, sb = blocks_of(n, p->superblock), zb = p->k_bits == 4 ? 128 : 256;
+        add_fill(x, blocks, p->k_packed, nullptr, h, p->k_capacity * row, n * row, p->k_capacity * row, 0);
+        add_fill(x, blocks, p->k_scale, nullptr, h, p->k_superblocks * 256, sb * 256, p->k_superblocks * 256, 0);
+        add_fill(x, blocks, p->k_zero, nullptr, h, p->k_superblocks * zb, sb * zb, p->k_superblocks * zb, 0);
+        if (p->k_operands)
+            add_fill(x, blocks, p->k_operands, nullptr, h, p->k_superblocks * 512, sb * 512, p->k_superblocks * 512, 0);
+    } else {
+        add_fill(x, blocks, p->k_packed, nullptr, h, p->k_capacity * 256, n * 256, p->k_capacity * 256, 0);
+    }
+    add_fill(x, blocks, p->i4_v, nullptr, h, p->i4_capacity * 64, s_i4 * 64, p->i4_capacity * 64, 0);
+    add_fill(x, blocks, p->i4_scale, nullptr, h, p->i4_capacity * 4, s_i4 * 4, p->i4_capacity * 4, 0);
+    const int64_t g = p->i2_capacity > 0 ? 128 / p->i2_group : 0;
+    add_fill(x, blocks, p->i2_v, nullptr, h, p->i2_capacity * 32, s_i2 * 32, p->i2_capacity * 32, 0);
+    add_fill(x, blocks, p->i2_scale, nullptr, h, p->i2_capacity * 2 * g, s_i2 * 2 * g, p->i2_capacity * 2 * g, 0);
+    add_fill(x, blocks, p->i2_zero, nullptr, h, p->i2_capacity * g, s_i2 * g, p->i2_capacity * g, 0);
+    static_assert(kMaxFills >= 1 + 4 + 1 + 2 + 4 + 2 + 3, "every fill has a place");
+    if (blocks + x.page_blocks > 0x7fffffff) return R2O_EINVAL;
+    hipLaunchKernelGGL(cache_index_kernel, dim3((unsigned)(x.page_blocks + blocks)), dim3(256), 0, st, x);
+    R2O_CHECK_LAUNCH();
+    CachePack a{};
+    if (packed_k)
+        a.key = {p->key, p->tokens, p->index, n, 0, 0, p->k_packed, p->k_scale, p->k_zero, p->k_operands, p->k_capacity,
+                 p->k_superblocks};
+    else
+        a.rows = {p->key, p->tokens, p->index, n, reinterpret_cast<uint16_t*>(p->k_packed), p->k_capacity};
+    a.fp = {p->value, p->tokens, p->index, s_fp, p->fp_v, s_fp};
+    a.v4 = {p->value, p->tokens, p->index + s_fp, s_i4, 0, p->i4_v, p->i4_scale, nullptr, p->i4_capacity, 128};
+    a.v2 = {p->value, p->tokens, p->index + head, s_i2, 0, p->i2_v, p->i2_scale, p->i2_zero, p->i2_capacity, (int)p->i2_group};
+    int key_bits = packed_k && n > 0 ? (int)p->k_bits : 0;
+    if (key_bits && p->key_dtype != p->value_dtype) {  // one dtype per launch
+        if (key_bits == 4) launch_pack_keys<4>(a.key, p->superblock, p->key_dtype, h, st);
+        else launch_pack_keys<2>(a.key, p->superblock, p->key_dtype, h, st);
+        key_bits = 0;
+    }
+    launch_pack_cache(a, key_bits, p->superblock, p->value_dtype, h, st);
     R2O_CHECK_LAUNCH();
     return R2O_OK;
 }

@@ -185,3 +185,81 @@ extern "C" int r2o_plan_work_items(const r2o_plan_run* runs, int64_t n_runs, con
     *n_items = (int64_t)planned.size();
     return R2O_OK;
 }
+
+// ------------------------------------------------------------------------------ cache page tables
+namespace {
+
+// Tier of a page class (PageClass in policy.py): FP (+protected, recent) 0, INT4 1, INT2 2, evicted 3.
+int tier_of(int64_t cls) {
+    constexpr int kTier[6] = {3, 0, 1, 0, 0, 2};
+    return cls >= 0 && cls < 6 ? kTier[cls] : -1;
+}
+
+}  // namespace
+
+extern "C" int r2o_cache_pages(const int64_t* table, int64_t n_pages, int64_t tokens, int64_t* tier_pages,
+                               int64_t* tier_tokens) {
+    if ((!table && n_pages > 0) || n_pages < 0 || tokens < 0 || !tier_pages || !tier_tokens) return R2O_EINVAL;
+    for (int t = 0; t < 4; ++t) tier_pages[t] = tier_tokens[t] = 0;
+    for (int64_t p = 0; p < n_pages; ++p) {
+        const int t = tier_of(table[p]);
+        const int64_t first = table[n_pages + p], len = table[2 * n_pages + p];
+        if (t < 0 || len < 0 || first < 0 || first > tokens - len) return R2O_EINVAL;
+        tier_pages[t] += 1;
+        tier_tokens[t] += len;
+    }
+    return R2O_OK;
+}
+
+extern "C" int r2o_cache_page_words(const int64_t* table, int64_t n_pages, int64_t page_size, int64_t reserve4,
+                                    int64_t reserve2, int64_t ring_capacity, int64_t* words, int64_t max_words) {
+    if ((!table && n_pages > 0) || n_pages < 0 || !words || page_size <= 0 || reserve4 < 0 || reserve2 < 0 ||
+        ring_capacity < 0 || reserve4 % page_size || reserve2 % page_size || ring_capacity % page_size)
+        return R2O_EINVAL;
+    int64_t pages[4] = {0, 0, 0, 0};
+    for (int64_t p = 0; p < n_pages; ++p) {
+        const int t = tier_of(table[p]);
+        if (t < 0) return R2O_EINVAL;
+        pages[t] += 1;
+    }
+    const int64_t extra[4] = {0, reserve4 / page_size, reserve2 / page_size, 0}, ring = ring_capacity / page_size;
+    const int64_t page_words = 3 * (pages[0] + pages[1] + pages[2] + extra[1] + extra[2] + ring) + 1;
+    if (max_words < page_words + 3 * n_pages) return R2O_EINVAL;
+    int64_t* start = words + page_words;  // first tokens, lengths, positions of every page in tier order
+    int64_t at = 0, position = 0;
+    int64_t* w = words;
+    for (int t = 0; t < 4; ++t) {
+        const int64_t span = pages[t] + extra[t];
+        int64_t k = 0, offset = 0;
+        for (int64_t p = 0; p < n_pages; ++p) {
+            if (tier_of(table[p]) != t) continue;
+            const int64_t len = table[2 * n_pages + p];
+            if (t < 3) {
+                w[k] = p;
+                w[span + k] = offset;
+                w[2 * span + k] = len;
+            }
+            start[at] = table[n_pages + p];
+            start[n_pages + at] = len;
+            start[2 * n_pages + at] = position;
+            ++k;
+            ++at;
+            offset += len;
+            position += len;
+        }
+        if (t == 3) break;
+        for (int64_t e = 0; e < extra[t]; ++e, ++k) {
+            w[k] = -1;
+            w[span + k] = offset + page_size * e;
+            w[2 * span + k] = page_size;
+        }
+        w += 3 * span;
+    }
+    for (int64_t e = 0; e < ring; ++e) {
+        w[e] = -1;
+        w[ring + e] = page_size * e;
+        w[2 * ring + e] = 0;
+    }
+    w[3 * ring] = 0;
+    return R2O_OK;
+}

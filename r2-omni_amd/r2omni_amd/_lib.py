@@ -122,6 +122,19 @@ class RingFlush(ctypes.Structure):  # r2o_ring_flush_params
     ]
 
 
+class CacheBuild(ctypes.Structure):  # r2o_cache_build_params
+    _fields_ = [
+        ("key", c_vp), ("value", c_vp), ("key_dtype", c_i64), ("value_dtype", c_i64), ("hkv", c_i64), ("tokens", c_i64),
+        ("plan_global", c_vp), ("plan_logical", c_vp), ("pages", c_vp), ("page_words", c_i64), ("n_pages", c_i64),
+        ("tier_tokens", c_i64 * 4), ("reserve4", c_i64), ("reserve2", c_i64), ("storage", c_vp), ("index", c_vp),
+        ("ring_k", c_vp), ("ring_v", c_vp), ("ring_capacity", c_i64),
+        ("k_bits", c_i64), ("superblock", c_i64), ("k_packed", c_vp), ("k_scale", c_vp), ("k_zero", c_vp),
+        ("k_operands", c_vp), ("k_capacity", c_i64), ("k_superblocks", c_i64),
+        ("fp_v", c_vp), ("i4_v", c_vp), ("i4_scale", c_vp), ("i4_capacity", c_i64),
+        ("i2_v", c_vp), ("i2_scale", c_vp), ("i2_zero", c_vp), ("i2_capacity", c_i64), ("i2_group", c_i64),
+    ]
+
+
 _SIGNATURES = {
     "r2o_plan_work_items": (ctypes.POINTER(PlanRun), c_i64, ctypes.POINTER(PlanConfig), c_vp, c_i64, c_i64, c_i64,
                             c_vp, c_i64, c_vp, c_i64, ctypes.POINTER(c_i64)),
@@ -139,6 +152,9 @@ _SIGNATURES = {
     "r2o_gather_rows": (c_vp, c_i64, c_i64, c_vp, c_i64, c_vp, c_i64, c_vp),
     "r2o_recent_append": (c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_i64, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp),
     "r2o_recent_shift": (c_vp, c_vp, c_i64, c_i64, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp),
+    "r2o_cache_pages": (c_vp, c_i64, c_i64, c_vp, c_vp),
+    "r2o_cache_page_words": (c_vp, c_i64, c_i64, c_i64, c_i64, c_i64, c_vp, c_i64),
+    "r2o_cache_build": (ctypes.POINTER(CacheBuild), c_vp),
     "r2o_ring_flush": (ctypes.POINTER(RingFlush), c_vp),
     "r2o_fwht128": (c_vp, c_vp, c_i64, c_i64, c_vp),
     "r2o_qk_mrope": (c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_i64, c_i64, c_vp, c_vp, c_i64, c_vp, c_vp,

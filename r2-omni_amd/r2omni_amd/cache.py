@@ -464,8 +464,12 @@ def fused_gather_pack_int4_value(value: torch.Tensor, token_indices: torch.Tenso
         idx = token_indices.to(torch.long).contiguous()
         _lib.call("r2o_pack_int4_v", _lib.ptr(value), _lib.dtype_code(value.dtype), h, s, _lib.ptr(idx), n, 0,
                   _lib.ptr(packed), _lib.ptr(scale), n, _lib.stream_of(value.device))
-    return PackedTensor(packed=packed.flatten(), scale=scale, zero_point=None, num_bits=4, original_shape=(h, n, d),
-                        dtype=value.dtype, quant_scheme="per_token",
+    return _packed_int4(packed.flatten(), scale, h, n, value.dtype)
+
+
+def _packed_int4(packed: torch.Tensor, scale: torch.Tensor, h: int, n: int, dtype: torch.dtype) -> PackedTensor:
+    return PackedTensor(packed=packed, scale=scale, zero_point=None, num_bits=4, original_shape=(h, n, 128),
+                        dtype=dtype, quant_scheme="per_token",
                         pack_metadata={"pack_axis": "flatten_c_order", "fused_gather": True},
                         quant_metadata={"dim": 2, "fused_gather": True})
 
@@ -866,17 +870,22 @@ for _c, _t in ((PageClass.EVICTED_PAGE, 3), (PageClass.FP_PAGE, 0), (PageClass.P
     _TIER_OF_CLASS[int(_c)] = _t
 
 
-def _tier_page_table(plan: LayerCompressionPlan) -> _TierTable:
-    """Pages stably sorted by tier, each keeping its token order (precision_pool.py:611-669).
-
-    The page table is small: it is sorted on the host, from the plan's host copy or one copy from
-    the device when the plan lives there.
-    """
+def _host_page_table(plan: LayerCompressionPlan) -> torch.Tensor:
+    """(page classes, offsets, lengths) as contiguous int64 [3, pages] on the host: the plan's own host copy or
+    one copy from the device when the plan lives there."""
     table = plan.host_page_table
     if table is None:
         table = torch.stack((plan.page_classes.detach().to(torch.long), plan.page_offsets.detach().to(torch.long),
-                             plan.page_lengths.detach().to(torch.long))).to("cpu")
-    classes, starts, lens = table.numpy()
+                             plan.page_lengths.detach().to(torch.long)))
+    return table.to("cpu", torch.long).contiguous()
+
+
+def _tier_page_table(plan: LayerCompressionPlan) -> _TierTable:
+    """Pages stably sorted by tier, each keeping its token order (precision_pool.py:611-669).
+
+    The page table is small: it is sorted on the host.
+    """
+    classes, starts, lens = _host_page_table(plan).numpy()
     if classes.size and (int(classes.min()) < 0 or int(classes.max()) >= _TIER_OF_CLASS.size):
         raise ValueError("page_classes holds a value that is not a PageClass")
     cat = _TIER_OF_CLASS[classes]
@@ -906,93 +915,80 @@ def _expand_tier_tokens(tab: _TierTable, device) -> torch.Tensor:
                                                                                   dtype=torch.long)
 
 
+def _metadata_views(storage: torch.Tensor, tier_pages, tier_tokens, *, page_size: int, recent_capacity: int,
+                    int2_reserve: int, int4_reserve: int):
+    """The views of a metadata arena's int64 ``storage`` (precision_pool.py:400-585): the arena, the four
+    pools' page indexes, the evicted indices and the ring's (global, logical, length) buffers.
+
+    Layout: per tier FP, INT4, INT2 and for the ring the page fields (ids, offsets, lengths), the length word,
+    then the token fields: global [FP INT4 INT4-reserve INT2 INT2-reserve], logical [the same], evicted, ring
+    global, ring logical.  ``int4_reserve`` / ``int2_reserve`` tokens (whole pages) follow the INT4 / INT2
+    pool's own in every field."""
+    ps = int(page_size)
+    extra = (0, int(int4_reserve), int(int2_reserve))
+    pages, tokens = [int(n) for n in tier_pages[:3]], [int(n) for n in tier_tokens[:3]]
+    ring_pages = int(recent_capacity) // ps
+    page_spans = [n + e // ps for n, e in zip(pages, extra)]
+    token_spans = [n + e for n, e in zip(tokens, extra)]
+    parts = storage.split_with_sizes([n for n in page_spans for _ in range(3)] + [ring_pages] * 3 + [1] + token_spans * 2
+                                     + [int(tier_tokens[3]), int(recent_capacity), int(recent_capacity)])
+    length = parts[12].view(torch.int32)[0]
+    evicted, ring_g, ring_l = parts[19:]
+    pools, fields = [], {}
+    for t, name in enumerate(("fp", "int4", "int2")):
+        ids, offs, lens = parts[3 * t:3 * t + 3]
+        g, l = parts[13 + t], parts[16 + t]
+        if name != "fp":
+            fields.update({f"{name}_original_page_ids_buffer": ids, f"{name}_physical_offsets_buffer": offs,
+                           f"{name}_lengths_buffer": lens, f"{name}_global_index_buffer": g,
+                           f"{name}_logical_position_buffer": l, f"{name}_page_count": pages[t],
+                           f"{name}_token_count": tokens[t]})
+        if extra[t]:
+            ids, offs, lens, g, l = ids[:pages[t]], offs[:pages[t]], lens[:pages[t]], g[:tokens[t]], l[:tokens[t]]
+        pools.append(PhysicalPageIndex(original_page_ids=ids, physical_offsets=offs, lengths=lens,
+                                       global_token_indices=g, logical_positions=l))
+    pools.append(PhysicalPageIndex(*parts[9:12], global_token_indices=ring_g, logical_positions=ring_l))
+    return CompactMetadataArena(storage=storage, **fields), pools, evicted, (ring_g, ring_l, length)
+
+
+def _metadata_words(tier_pages, tier_tokens, *, page_size: int, recent_capacity: int, int2_reserve: int,
+                    int4_reserve: int) -> tuple[int, int]:
+    """(page words, all words) of a metadata arena's storage."""
+    if int2_reserve % page_size or int4_reserve % page_size or recent_capacity % page_size:
+        raise ValueError("metadata reserves must be whole pages")
+    pages = sum(int(n) for n in tier_pages[:3]) + (int4_reserve + int2_reserve + recent_capacity) // page_size
+    span = sum(int(n) for n in tier_tokens[:3]) + int4_reserve + int2_reserve
+    words = 3 * pages + 1
+    return words, words + 2 * span + int(tier_tokens[3]) + 2 * recent_capacity
+
+
 def _build_metadata_arena(tab: _TierTable, tokens: torch.Tensor, gi: torch.Tensor, lp: torch.Tensor, *,
                           page_size: int, recent_capacity: int, int2_reserve: int, int4_reserve: int = 0):
-    """One int64 allocation holding the page index of every pool, the evicted global indices, the
-    Recent-FP ring's index buffers and its device length (precision_pool.py:400-585).
-
-    ``tokens`` are the tier-ordered token indices of ``_expand_tier_tokens``; ``gi`` / ``lp`` the
-    plan's global / logical token indices on the same device.  ``int4_reserve`` / ``int2_reserve``
-    tokens (whole pages) are reserved after the INT4 / INT2 pool's fields.  Layout: the page fields
-    of every pool and the length slot (built on the host, one copy), then the token fields: global
-    [FP INT4 INT4-reserve INT2 INT2-reserve], logical [the same], evicted, ring global, ring logical.
-    Returns the arena, the four pools' page indexes, the evicted indices and the ring's (global,
-    logical, length) buffers.
-    """
-    ps = int(page_size)
-    cap = int(recent_capacity)
-    if int2_reserve % ps or int4_reserve % ps or cap % ps:
-        raise ValueError("metadata reserves must be whole pages")
-    dev = tokens.device
-    tiers = [slice(int(tab.first_page[t]), int(tab.first_page[t + 1])) for t in range(3)]
-    reserve_pages = (0, int(int4_reserve) // ps, int(int2_reserve) // ps)
+    """The metadata arena of ``_metadata_views`` filled by torch on any device, from the tier-ordered token
+    indices of ``_expand_tier_tokens`` and the plan's global / logical token indices (a cache build fills
+    its arena by ``r2o_cache_build``)."""
+    ps, cap = int(page_size), int(recent_capacity)
+    sizes = dict(page_size=ps, recent_capacity=cap, int2_reserve=int(int2_reserve), int4_reserve=int(int4_reserve))
+    tier_pages = np.diff(tab.first_page)
+    page_words, total = _metadata_words(tier_pages, tab.tier_tokens, **sizes)
+    storage = torch.full((total,), -1, device=tokens.device, dtype=torch.long)
+    arena, pools, evicted, ring = _metadata_views(storage, tier_pages, tab.tier_tokens, **sizes)
+    parts = []
+    for t, extra in enumerate((0, int(int4_reserve) // ps, int(int2_reserve) // ps)):
+        sl, n_tok = slice(int(tab.first_page[t]), int(tab.first_page[t + 1])), int(tab.tier_tokens[t])
+        parts += [tab.pages[sl], np.full(extra, -1), tab.offsets[sl], n_tok + ps * np.arange(extra), tab.lengths[sl],
+                  np.full(extra, ps)]
     ring_pages = cap // ps
-
-    page_parts = []
-    for t, extra in zip(tiers, reserve_pages):
-        n_tok = int(tab.tier_tokens[len(page_parts)])
-        page_parts.append(np.concatenate((tab.pages[t], np.full(extra, -1), tab.offsets[t],
-                                          n_tok + ps * np.arange(extra), tab.lengths[t], np.full(extra, ps))))
-    page_parts.append(np.concatenate((np.full(ring_pages, -1), ps * np.arange(ring_pages),
-                                      np.zeros(ring_pages, np.int64))))
-    page_parts.append(np.zeros(1, np.int64))  # the ring's device length (int32 in the low half)
-    page_block = torch.from_numpy(np.concatenate(page_parts).astype(np.int64))
-    n_pages_total = int(page_block.numel())
-    n_surv = int(tab.tier_tokens[:3].sum())
-    n_ev = int(tab.tier_tokens[3])
-    n_head = int(tab.tier_tokens[:2].sum())  # FP + INT4 tokens, before the INT4 reserve
-    surv_span = n_surv + int(int4_reserve) + int(int2_reserve)
-    storage = torch.empty(n_pages_total + 2 * surv_span + n_ev + 2 * cap, device=dev, dtype=torch.long)
-    if dev.type != "cpu":
-        page_block = page_block.pin_memory()
-    storage[:n_pages_total].copy_(page_block, non_blocking=True)
-    tok = storage[n_pages_total:]
-    tok.fill_(-1)
-    g_all, l_all = tok[:surv_span], tok[surv_span:2 * surv_span]
-    evicted = tok[2 * surv_span:2 * surv_span + n_ev]
-    ring_g = tok[2 * surv_span + n_ev:2 * surv_span + n_ev + cap]
-    ring_l = tok[2 * surv_span + n_ev + cap:]
-    i2_at = n_head + int(int4_reserve)
-    for dst, lo, hi in ((0, 0, n_head), (i2_at, n_head, n_surv)):
-        if hi > lo:
-            torch.index_select(gi, 0, tokens[lo:hi], out=g_all[dst:dst + hi - lo])
-            torch.index_select(lp, 0, tokens[lo:hi], out=l_all[dst:dst + hi - lo])
-    if n_ev:
-        torch.index_select(gi, 0, tokens[n_surv:], out=evicted)
-
-    cursor = 0
-
-    def take(n):
-        nonlocal cursor
-        v = storage[cursor:cursor + n]
-        cursor += n
-        return v
-
-    indexes = []
-    tok_start = 0
-    for t, extra in zip(tiers, reserve_pages):
-        npg = t.stop - t.start + extra
-        ids, offs, lens = take(npg), take(npg), take(npg)
-        nt = int(tab.tier_tokens[len(indexes)])
-        span = nt + extra * ps
-        g, l = g_all[tok_start:tok_start + span], l_all[tok_start:tok_start + span]
-        tok_start += span
-        indexes.append((ids, offs, lens, g, l, npg - extra, nt))
-    ring_ids, ring_offs, ring_lens = take(ring_pages), take(ring_pages), take(ring_pages)
-    length = take(1).view(torch.int32)[0]
-    pools = [PhysicalPageIndex(original_page_ids=ids[:np_], physical_offsets=offs[:np_], lengths=lens[:np_],
-                               global_token_indices=g[:nt], logical_positions=l[:nt])
-             for ids, offs, lens, g, l, np_, nt in indexes]
-    pools.append(PhysicalPageIndex(original_page_ids=ring_ids, physical_offsets=ring_offs, lengths=ring_lens,
-                                   global_token_indices=ring_g, logical_positions=ring_l))
-    tier_fields = {}
-    for name, (ids, offs, lens, g, l, np_, nt) in (("int4", indexes[1]), ("int2", indexes[2])):
-        tier_fields.update({f"{name}_original_page_ids_buffer": ids, f"{name}_physical_offsets_buffer": offs,
-                            f"{name}_lengths_buffer": lens, f"{name}_global_index_buffer": g,
-                            f"{name}_logical_position_buffer": l, f"{name}_page_count": np_,
-                            f"{name}_token_count": nt})
-    arena = CompactMetadataArena(storage=storage, **tier_fields)
-    return arena, pools, evicted, (ring_g, ring_l, length)
+    parts += [np.full(ring_pages, -1), ps * np.arange(ring_pages), np.zeros(ring_pages + 1, np.int64)]
+    storage[:page_words].copy_(torch.from_numpy(np.concatenate(parts).astype(np.int64)))
+    at = 0
+    for pool, n in zip(pools, tab.tier_tokens[:3]):
+        ix = tokens[at:at + int(n)]
+        pool.global_token_indices.copy_(gi[ix])
+        pool.logical_positions.copy_(lp[ix])
+        at += int(n)
+    evicted.copy_(gi[tokens[at:]])
+    return arena, pools, evicted, ring
 
 
 def _survivor_layout(plan: LayerCompressionPlan, device):
@@ -1034,32 +1030,24 @@ def _make_page_index(layout, gi: torch.Tensor, lp: torch.Tensor) -> PhysicalPage
                              lengths=lengths.to(dev), global_token_indices=gi[tokens], logical_positions=lp[tokens])
 
 
-def _preallocate_recent_pool(name: str, key: torch.Tensor, *, page_size: int, capacity: int,
-                             metadata=None) -> PrecisionPool:
-    """The Recent-FP ring: bf16/fp16 K and V rows of ``capacity`` tokens and its index buffers.
-    ``metadata`` = (page index, global buffer, logical buffer, int32 length) views of a metadata arena;
-    without it they are allocated here (the matched-FP cache has no arena)."""
-    if capacity < page_size or capacity % page_size:
-        raise ValueError("Recent-FP capacity must be positive and page aligned")
+def _preallocate_recent_pool(name: str, key: torch.Tensor, *, page_size: int, capacity: int) -> PrecisionPool:
+    """The Recent-FP ring of a cache without a metadata arena: 16-bit K and V rows of ``capacity`` tokens and
+    its index buffers."""
     h, _, d = map(int, key.shape)
     dev = key.device
-    if metadata is None:
-        gbuf = torch.full((capacity,), -1, device=dev, dtype=torch.long)
-        lbuf = torch.full((capacity,), -1, device=dev, dtype=torch.long)
-        pages = capacity // page_size
-        index = PhysicalPageIndex(
-            original_page_ids=torch.full((pages,), -1, device=dev, dtype=torch.long),
-            physical_offsets=torch.arange(pages, device=dev, dtype=torch.long) * page_size,
-            lengths=torch.zeros(pages, device=dev, dtype=torch.long),
-            global_token_indices=gbuf, logical_positions=lbuf)
-        length = torch.zeros((), device=dev, dtype=torch.int32)
-    else:
-        index, gbuf, lbuf, length = metadata
+    gbuf = torch.full((capacity,), -1, device=dev, dtype=torch.long)
+    lbuf = torch.full((capacity,), -1, device=dev, dtype=torch.long)
+    pages = capacity // page_size
+    index = PhysicalPageIndex(
+        original_page_ids=torch.full((pages,), -1, device=dev, dtype=torch.long),
+        physical_offsets=torch.arange(pages, device=dev, dtype=torch.long) * page_size,
+        lengths=torch.zeros(pages, device=dev, dtype=torch.long),
+        global_token_indices=gbuf, logical_positions=lbuf)
     return PrecisionPool(
         name=name, page_index=index,
         fp_k=torch.zeros((h, capacity, d), device=dev, dtype=key.dtype),
         fp_v=torch.zeros((h, capacity, d), device=dev, dtype=key.dtype),
-        active_length=0, capacity=capacity, length_device=length,
+        active_length=0, capacity=capacity, length_device=torch.zeros((), device=dev, dtype=torch.int32),
         global_index_buffer=gbuf, logical_position_buffer=lbuf,
     )
 
@@ -1106,91 +1094,157 @@ def build_three_precision_cache(
         raise ValueError("the SSPA decode path requires head_dim 128")
     _lib.require_device(key, "key")
     _lib.dtype_code(key.dtype)
-    bf16_keys = matched_fp or cache_variant == "v_fourq_k_bf16"  # key rows in the model dtype (bf16 or fp16)
     key = key.contiguous()
     value = value.contiguous()
-    dev = key.device
-    tab = _tier_page_table(plan)
-    if int(tab.tier_tokens.sum()) != int(key.shape[1]):
-        raise ValueError("compact physical pools must cover every logical token")
     if plan.recent_fp_capacity < page_size or plan.recent_fp_capacity % page_size:
         raise ValueError("Recent-FP capacity must be positive and page aligned")
-    h = int(key.shape[0])
-    stream = _lib.stream_of(dev)
     append_capacity = plan.recent_fp_capacity if compact_key_append_capacity is None \
         else int(compact_key_append_capacity)
-    gi = plan.global_token_indices.detach().to(dev, torch.long)
-    lp = plan.logical_positions.detach().to(dev, torch.long)
-    tokens = _expand_tier_tokens(tab, dev)
-    s_fp, s_i4, s_i2 = (int(n) for n in tab.tier_tokens[:3])
-    n_surv = s_fp + s_i4 + s_i2
     common = dict(page_size=int(page_size), quantization_superblock=int(quantization_superblock),
                   cache_variant=cache_variant, recent_flush_size=int(recent_flush_size),
                   generated_value_precision=str(generated_value_precision))
-    if matched_fp:  # every surviving page, K and V in bf16, in one FP pool (precision_pool.py:834-876)
-        surv = _survivor_layout(plan, dev)
-        n = int(surv[0].numel())
-        arena = _gather_key_rows(key, surv[0], append_capacity, (0, n, n))
-        fp_pool = PrecisionPool(name="fp", page_index=_make_page_index(surv, gi, lp), fp_k=arena.view(0, n))
-        fp_pool.fp_v = torch.empty((h, n, 128), device=dev, dtype=value.dtype)
-        if n:
-            _lib.call("r2o_gather_rows", _lib.ptr(value), h, int(value.shape[1]), _lib.ptr(surv[0]), n,
-                      _lib.ptr(fp_pool.fp_v), n, stream)
-        empty = (surv[0][:0], surv[1][:0], surv[2][:0], surv[3][:0])
-        recent = _preallocate_recent_pool("recent_fp", key, page_size=page_size, capacity=plan.recent_fp_capacity)
-        return ThreePrecisionCache(
-            fp_pool=fp_pool, int4_pool=PrecisionPool(name="int4", page_index=_make_page_index(empty, gi, lp)),
-            int2_pool=PrecisionPool(name="int2", page_index=_make_page_index(empty, gi, lp)),
-            recent_fp_pool=recent, matched_fp=True, bf16_key=arena, generated_k_offset=n,
-            evicted_global_indices=gi[tokens[n_surv:]], **common)
-    fp_tokens, i4_tokens, i2_tokens = tokens[:s_fp], tokens[s_fp:s_fp + s_i4], tokens[s_fp + s_i4:n_surv]
+    if matched_fp:
+        return _build_matched_cache(key, value, plan, append_capacity, common)
+    return _build_tiered_cache(key, value, plan, append_capacity, int(key_quantization_superblock), int(int2_group_size),
+                               common)
 
-    fp_v = int4_v = compact_int4_value = None
-    if s_fp:
-        fp_v = torch.empty((h, s_fp, 128), device=dev, dtype=value.dtype)
-        _lib.call("r2o_gather_rows", _lib.ptr(value), h, int(value.shape[1]), _lib.ptr(fp_tokens), s_fp,
-                  _lib.ptr(fp_v), s_fp, stream)
-    int4_generated = generated_value_precision == "int4"
+
+def _build_matched_cache(key, value, plan: LayerCompressionPlan, append_capacity: int, common: dict) -> ThreePrecisionCache:
+    """Every surviving page, K and V in the model dtype, in one FP pool (precision_pool.py:834-876)."""
+    dev, h, page_size = key.device, int(key.shape[0]), common["page_size"]
+    tab = _tier_page_table(plan)
+    if int(tab.tier_tokens.sum()) != int(key.shape[1]):
+        raise ValueError("compact physical pools must cover every logical token")
+    gi = plan.global_token_indices.detach().to(dev, torch.long)
+    lp = plan.logical_positions.detach().to(dev, torch.long)
+    tokens = _expand_tier_tokens(tab, dev)
+    surv = _survivor_layout(plan, dev)
+    n = int(surv[0].numel())
+    arena = _gather_key_rows(key, surv[0], append_capacity, (0, n, n))
+    fp_pool = PrecisionPool(name="fp", page_index=_make_page_index(surv, gi, lp), fp_k=arena.view(0, n))
+    fp_pool.fp_v = torch.empty((h, n, 128), device=dev, dtype=value.dtype)
+    if n:
+        _lib.call("r2o_gather_rows", _lib.ptr(value), h, int(value.shape[1]), _lib.ptr(surv[0]), n,
+                  _lib.ptr(fp_pool.fp_v), n, _lib.stream_of(dev))
+    empty = (surv[0][:0], surv[1][:0], surv[2][:0], surv[3][:0])
+    recent = _preallocate_recent_pool("recent_fp", key, page_size=page_size, capacity=plan.recent_fp_capacity)
+    return ThreePrecisionCache(
+        fp_pool=fp_pool, int4_pool=PrecisionPool(name="int4", page_index=_make_page_index(empty, gi, lp)),
+        int2_pool=PrecisionPool(name="int2", page_index=_make_page_index(empty, gi, lp)),
+        recent_fp_pool=recent, matched_fp=True, bf16_key=arena, generated_k_offset=n,
+        evicted_global_indices=gi[tokens[int(tab.tier_tokens[:3].sum()):]], **common)
+
+
+def _build_tiered_cache(key, value, plan: LayerCompressionPlan, append_capacity: int, superblock: int, group: int,
+                        common: dict) -> ThreePrecisionCache:
+    """The three pools and their metadata arena (precision_pool.py:878-984): every tensor allocated here,
+    unwritten, and filled by the two launches of ``r2o_cache_build`` behind one upload of the page table."""
+    dev, h, s = key.device, int(key.shape[0]), int(key.shape[1])
+    ps, cap = common["page_size"], int(plan.recent_fp_capacity)
+    _lib.require_device(value, "value")
+    value_code = _lib.dtype_code(value.dtype)
+    if group not in (32, 64, 128):
+        raise ValueError("compact INT2 V requires group_size 32, 64, or 128")
+    if append_capacity < 0:
+        raise ValueError("append_capacity must be non-negative")
+    # the kernels move rows in 16-byte pieces; a view may start between them
+    key, value = (t.clone() if t.data_ptr() % 16 else t for t in (key, value))
+    table = _host_page_table(plan)
+    n_pages = int(table.shape[1])
+    counts = np.empty(8, dtype=np.int64)
+    lib = _lib.load()
+    if lib.r2o_cache_pages(table.data_ptr(), n_pages, s, counts.ctypes.data, counts.ctypes.data + 32):
+        _tier_page_table(plan)  # names an unknown class
+        raise ValueError("static plan pages must lie inside the K/V sequence")
+    tier_pages, tier_tokens = counts[:4].tolist(), counts[4:].tolist()
+    if sum(tier_tokens) != s:
+        raise ValueError("compact physical pools must cover every logical token")
+    gi = plan.global_token_indices.detach().to(dev, torch.long).contiguous()
+    lp = plan.logical_positions.detach().to(dev, torch.long).contiguous()
+    if gi.numel() < s:
+        raise ValueError("static plan indices must cover the K/V sequence")
+    s_fp, s_i4, s_i2, _ = tier_tokens
+    n = s_fp + s_i4 + s_i2
+    bf16_keys = common["cache_variant"] == "v_fourq_k_bf16"  # key rows in the model dtype (bf16 or fp16)
+    int4_generated = common["generated_value_precision"] == "int4"
+
+    def empty(shape, dtype):
+        return torch.empty(shape, device=dev, dtype=dtype)
+
+    fp_v = empty((h, s_fp, 128), value.dtype) if s_fp else None
+    int4_v = compact_int4_value = None
+    i4_capacity = 0
     if int4_generated:  # the INT4 pool's V is an arena with room for generated flushes (precision_pool.py:935-942)
-        compact_int4_value = int4_v = build_compact_int4_value_arena(value, i4_tokens, append_capacity=append_capacity)
+        i4_capacity = max(1, s_i4 + append_capacity)
+        compact_int4_value = int4_v = CompactInt4ValueArena(
+            packed=empty((h, i4_capacity, 64), torch.uint8), scale=empty((h, i4_capacity, 1), torch.float32),
+            active_length=s_i4, capacity=i4_capacity, original_dtype=value.dtype)
     elif s_i4:
-        int4_v = fused_gather_pack_int4_value(value, i4_tokens)
-    compact_value = build_compact_int2_value_arena(value, i2_tokens, group_size=int2_group_size,
-                                                   append_capacity=0 if int4_generated else append_capacity)
+        i4_capacity = s_i4
+        int4_v = _packed_int4(empty(h * s_i4 * 64, torch.uint8), empty((h, s_i4, 1), torch.float32), h, s_i4, value.dtype)
+    i2_capacity = max(128, _round_up(s_i2 + (0 if int4_generated else append_capacity), 128))
+    compact_value = CompactInt2ValueArena(
+        packed=empty((h, i2_capacity, 32), torch.uint8), scale=empty((h, i2_capacity, 128 // group, 1), torch.float16),
+        zero_point=empty((h, i2_capacity, 128 // group, 1), torch.uint8), active_length=s_i2, capacity=i2_capacity,
+        original_dtype=value.dtype, group_size=group)
+    capacity = max(128, _round_up(n + append_capacity, 128))
+    segments = (0, s_fp, s_fp + s_i4)
     compact_key = bf16_arena = None
-    if bf16_keys:  # v_fourq_k_bf16: every pool keeps bf16 K rows (precision_pool.py:878-906)
-        bf16_arena = _gather_key_rows(key, tokens[:n_surv], append_capacity, (0, s_fp, s_fp + s_i4))
-        reserve = reserve4 = 0  # no compact K arena to flush into (precision_pool.py:404-408)
+    reserve = reserve4 = 0
+    if bf16_keys:  # no compact K arena to flush into: nothing is reserved (precision_pool.py:404-408, 878-906)
+        bf16_arena = BF16KeyArena(rows=empty((h, capacity, 128), key.dtype), active_length=n, capacity=capacity,
+                                  segment_offsets=segments)
+        k_fields = dict(k_bits=16, k_packed=bf16_arena.rows.data_ptr(), k_capacity=capacity)
     else:
-        build_key = build_compact_int2_key_arena if cache_variant == "v_fourq_k_int2_compact" \
-            else build_compact_int4_key_arena
-        compact_key = build_key(key, (fp_tokens, i4_tokens, i2_tokens), append_capacity=append_capacity,
-                                superblock_size=key_quantization_superblock)
-        key_room = compact_key.capacity - compact_key.active_length
-        reserve = min(compact_value.capacity - compact_value.active_length, key_room) // page_size * page_size
-        reserve4 = 0 if compact_int4_value is None else \
-            min(compact_int4_value.capacity - compact_int4_value.active_length, key_room) // page_size * page_size
-    meta, (fp_pi, i4_pi, i2_pi, ring_pi), evicted, (ring_g, ring_l, ring_len) = _build_metadata_arena(
-        tab, tokens, gi, lp, page_size=page_size, recent_capacity=plan.recent_fp_capacity, int2_reserve=reserve,
-        int4_reserve=reserve4)
+        int2_keys = common["cache_variant"] == "v_fourq_k_int2_compact"
+        blocks = capacity // superblock
+        arena_class = CompactInt2KeyArena if int2_keys else CompactInt4KeyArena
+        compact_key = arena_class(
+            packed=empty((h, capacity, 32 if int2_keys else 64), torch.uint8), scale=empty((h, blocks, 128), torch.float16),
+            zero_point=empty((h, blocks, 128), torch.float16 if int2_keys else torch.uint8), active_length=n,
+            capacity=capacity, segment_offsets=segments, original_dtype=key.dtype, superblock_size=superblock,
+            kernel_operands=empty((h, blocks, 128), torch.int32))
+        room = capacity - n
+        reserve = min(i2_capacity - s_i2, room) // ps * ps
+        reserve4 = min(i4_capacity - s_i4, room) // ps * ps if int4_generated else 0
+        k_fields = dict(k_bits=compact_key.bit_width, superblock=superblock, k_packed=compact_key.packed.data_ptr(),
+                        k_scale=compact_key.scale.data_ptr(), k_zero=compact_key.zero_point.data_ptr(),
+                        k_operands=compact_key.kernel_operands.data_ptr(), k_capacity=capacity, k_superblocks=blocks)
+    ring_k, ring_v = empty((h, cap, 128), key.dtype), empty((h, cap, 128), key.dtype)
+
+    sizes = dict(page_size=ps, recent_capacity=cap, int2_reserve=reserve, int4_reserve=reserve4)
+    page_words, total = _metadata_words(tier_pages, tier_tokens, **sizes)
+    words = torch.empty(page_words + 3 * n_pages, dtype=torch.long, pin_memory=True)
+    _lib.check(lib.r2o_cache_page_words(table.data_ptr(), n_pages, ps, reserve4, reserve, cap, words.data_ptr(),
+                                        words.numel()), "r2o_cache_page_words")
+    pages = words.to(dev, non_blocking=True)  # pinned: a copy from pageable memory would wait for the stream
+    storage, index = empty(total, torch.long), empty(n, torch.long)
+    _lib.call("r2o_cache_build", _lib.CacheBuild(
+        key=key.data_ptr(), value=value.data_ptr(), key_dtype=_lib.dtype_code(key.dtype), value_dtype=value_code, hkv=h,
+        tokens=s, plan_global=gi.data_ptr(), plan_logical=lp.data_ptr(), pages=pages.data_ptr(), page_words=page_words,
+        n_pages=n_pages, tier_tokens=tuple(tier_tokens), reserve4=reserve4, reserve2=reserve, storage=storage.data_ptr(),
+        index=index.data_ptr(), ring_k=ring_k.data_ptr(), ring_v=ring_v.data_ptr(), ring_capacity=cap,
+        fp_v=_lib.ptr(fp_v), i4_v=None if int4_v is None else int4_v.packed.data_ptr(),
+        i4_scale=None if int4_v is None else int4_v.scale.data_ptr(), i4_capacity=i4_capacity,
+        i2_v=compact_value.packed.data_ptr(), i2_scale=compact_value.scale.data_ptr(),
+        i2_zero=compact_value.zero_point.data_ptr(), i2_capacity=i2_capacity, i2_group=group, **k_fields),
+        _lib.stream_of(dev))
+
+    meta, (fp_pi, i4_pi, i2_pi, ring_pi), evicted, (ring_g, ring_l, ring_len) = _metadata_views(
+        storage, tier_pages, tier_tokens, **sizes)
     fp_pool = PrecisionPool(name="fp", page_index=fp_pi, fp_v=fp_v)
     int4_pool = PrecisionPool(name="int4", page_index=i4_pi, packed_v=int4_v)
     int2_pool = PrecisionPool(name="int2", page_index=i2_pi, packed_v=compact_value)
-    recent = _preallocate_recent_pool("recent_fp", key, page_size=page_size, capacity=plan.recent_fp_capacity,
-                                      metadata=(ring_pi, ring_g, ring_l, ring_len))
+    recent = PrecisionPool(name="recent_fp", page_index=ring_pi, fp_k=ring_k, fp_v=ring_v, active_length=0, capacity=cap,
+                           length_device=ring_len, global_index_buffer=ring_g, logical_position_buffer=ring_l)
     if bf16_keys:
         fp_pool.fp_k, int4_pool.fp_k = bf16_arena.view(0, s_fp), bf16_arena.view(s_fp, s_i4)
         int2_pool.fp_k = bf16_arena.view(s_fp + s_i4, s_i2)
-        return ThreePrecisionCache(
-            fp_pool=fp_pool, int4_pool=int4_pool, int2_pool=int2_pool, recent_fp_pool=recent, matched_fp=False,
-            compact_value=compact_value, compact_int4_value=compact_int4_value, static_int4_tokens=s_i4,
-            bf16_key=bf16_arena, metadata_arena=meta, evicted_global_indices=evicted, **common)
     return ThreePrecisionCache(
         fp_pool=fp_pool, int4_pool=int4_pool, int2_pool=int2_pool, recent_fp_pool=recent, matched_fp=False,
         compact_key=compact_key, compact_value=compact_value, compact_int4_value=compact_int4_value,
-        static_int4_tokens=s_i4, generated_k_offset=compact_key.active_length, metadata_arena=meta,
-        evicted_global_indices=evicted,
-        **common)
+        static_int4_tokens=s_i4, generated_k_offset=0 if bf16_keys else n, bf16_key=bf16_arena, metadata_arena=meta,
+        evicted_global_indices=evicted, **common)
 
 
 # ------------------------------------------------------------------------- append / flush
