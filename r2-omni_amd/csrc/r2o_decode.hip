@@ -156,11 +156,11 @@ __device__ __forceinline__ int64_t q_stride(const r2o_decode_params& p) {
     return RO != kRopeNone ? p.query_batch_stride : p.hq * 128;
 }
 
-// The query row of head l16 of the KV group (padded heads read head 0; their operand is zeroed).
+// The query row of a head of the KV group (padded heads read head 0; their operand is zeroed).
 template <int RO>
 __device__ __forceinline__ const uint16_t* query_row(const r2o_decode_params& p, int64_t b, int64_t kvh, int gqa,
-                                                     int l16) {
-    return p.query + b * q_stride<RO>(p) + (kvh * gqa + (l16 < gqa ? l16 : 0)) * 128;
+                                                     int head) {
+    return p.query + b * q_stride<RO>(p) + (kvh * gqa + (head < gqa ? head : 0)) * 128;
 }
 
 // The inputs of a lane's part of a rotation, put out ahead of the work item's first tile DMAs: the cos /
@@ -338,23 +338,23 @@ __device__ __forceinline__ void rot_block_row(const r2o_decode_params& p, int64_
     if (!is_q) *reinterpret_cast<r2o_u4*>((is_v ? p.rotated_v : p.rotated_k) + (b * p.hkv + kvh) * 128 + 8 * c8) = out;
 }
 
-// The lane's rotated query channels 32g .. 32g + 31 of head l16 (zero for the padded heads), after
-// the barrier.
-__device__ __forceinline__ void rot_read_query(const uint16_t* rot, int gqa, int l16, int g, r2o_u4 (&q)[4]) {
-    const r2o_u4* src = reinterpret_cast<const r2o_u4*>(rot + (l16 < gqa ? l16 : 0) * kRotStride + 32 * g);
+// The lane's rotated query channels 32g .. 32g + 31 of `head` (zero for the padded heads), after the
+// barrier.
+__device__ __forceinline__ void rot_read_query(const uint16_t* rot, int gqa, int head, int g, r2o_u4 (&q)[4]) {
+    const r2o_u4* src = reinterpret_cast<const r2o_u4*>(rot + (head < gqa ? head : 0) * kRotStride + 32 * g);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) q[j] = l16 < gqa ? src[j] : r2o_u4{0, 0, 0, 0};
+    for (int j = 0; j < 4; ++j) q[j] = head < gqa ? src[j] : r2o_u4{0, 0, 0, 0};
 }
 
-// Query operand of head l16 of the KV group (padded heads are zero), channels 32g .. 32g+31, in
+// Query operand of a head of the KV group (padded heads are zero), channels 32g .. 32g+31, in
 // the K operand order of the format: f16 pairs (8j+u, 8j+u+4) for INT4-K, f16 pairs
 // (16(j/2) + 4(j%2) + u, +8) for INT2-K, both scaled by D^-1/2 log2(e), or bf16 pairs in channel
 // order for bf16 keys (BF16-K pools and the Recent-FP ring; fp16 pairs for fp16 rows).  With a folded
 // rotation (RO) `qrot` holds the lane's rotated channels (rot_read_query).
 template <int KF, int RF, int RO>
-__device__ __forceinline__ void load_query(const r2o_decode_params& p, int64_t b, int64_t kvh, int gqa, int l16,
+__device__ __forceinline__ void load_query(const r2o_decode_params& p, int64_t b, int64_t kvh, int gqa, int head,
                                            int g, float qscale, uint32_t (&qp)[4][4], const r2o_u4 (&qrot)[4]) {
-    const bool head_ok = l16 < gqa;
+    const bool head_ok = head < gqa;
     float qf[32];
     {
         r2o_u4 raw[4];
@@ -362,7 +362,7 @@ __device__ __forceinline__ void load_query(const r2o_decode_params& p, int64_t b
 #pragma unroll
             for (int j = 0; j < 4; ++j) raw[j] = qrot[j];
         } else {
-            const r2o_u4* q4 = reinterpret_cast<const r2o_u4*>(query_row<RO>(p, b, kvh, gqa, l16) + 32 * g);
+            const r2o_u4* q4 = reinterpret_cast<const r2o_u4*>(query_row<RO>(p, b, kvh, gqa, head) + 32 * g);
 #pragma unroll
             for (int j = 0; j < 4; ++j) raw[j] = head_ok ? r2o_ldg(q4 + j) : r2o_u4{0, 0, 0, 0};
         }
@@ -391,21 +391,27 @@ __device__ __forceinline__ float head_max(float x) {
     return fmaxf(__uint_as_float(c[0]), __uint_as_float(c[1]));
 }
 
-// Online-softmax update for one tile: sv are the lane's 8 logits (log2 domain, -inf = masked).
-// Returns the probabilities in pk.  The running max is raised lazily: only when a tile's max
+// Online-softmax update for one tile whose logits are the lane's N values sv + add (log2 domain, -inf =
+// masked).  Returns the probabilities in pk; with ACC_L false the caller accumulates their sum itself (in
+// one of the `extra` accumulators).  The running max is raised lazily: only when a tile's max
 // exceeds it by more than kRescaleSlack (log2 units) are the state and the NE accumulators at `extra`
 // (4-row accumulators in the PV output layout) rescaled, so p = exp2(s - m) stays below
 // 2^kRescaleSlack while the rescale branch is taken only a few times per work item.  (m, l, acc)
 // always refer to the same m, so the state and its later merges are exact.
 constexpr float kRescaleSlack = 4.f;
 
-template <int N, int NE, bool ACC_L = true>
-__device__ __forceinline__ void softmax_step(WaveState& st, const float (&sv)[N], float (&pk)[N], int g, float add,
-                                             r2o_f4* extra) {
+//
+// N is 8, or 4 for a KV group of at most 8 query heads, whose tiles are held split (kSplitHeads): lane
+// l16 then has the logits of head l16 % 8 and lane l16 ^ 8 the tile's other half for the same head.
+template <int N, int NE = 0, bool ACC_L = true>
+__device__ __forceinline__ void softmax_tile(WaveState& st, const float (&sv)[N], float (&pk)[N], int g,
+                                             float add = 0.f, r2o_f4* extra = nullptr) {
     float tmax = sv[0];
 #pragma unroll
     for (int k = 1; k < N; ++k) tmax = fmaxf(tmax, sv[k]);
-    tmax = head_max(tmax) + add;  // -inf + add = -inf
+    tmax = head_max(tmax);
+    if constexpr (N == 4) tmax = fmaxf(tmax, r2o_lane_xor<8>(tmax));
+    tmax += add;  // -inf + add = -inf
     if (__any(tmax > st.m + kRescaleSlack)) {  // -inf + slack = -inf: the first valid tile rescales
         const float m_new = fmaxf(st.m, tmax);
         // exp2(-inf) = 0 when the state was empty; a head with no valid token keeps alpha = 1
@@ -427,14 +433,6 @@ __device__ __forceinline__ void softmax_step(WaveState& st, const float (&sv)[N]
         pk[k] = __builtin_amdgcn_exp2f(sv[k] - d);  // exp2(-inf) = 0 for masked tokens
         if constexpr (ACC_L) st.l += pk[k];
     }
-}
-
-// Online-softmax update for one tile whose logits are sv + add (log2 domain, -inf = masked).  With
-// ACC_L false the caller accumulates the sum of p itself (in one of the `extra` accumulators).
-template <int NE = 0, bool ACC_L = true>
-__device__ __forceinline__ void softmax_tile(WaveState& st, const float (&sv)[8], float (&pk)[8], int g,
-                                             float add = 0.f, r2o_f4* extra = nullptr) {
-    softmax_step<8, NE, ACC_L>(st, sv, pk, g, add, extra);
 }
 
 // PV for 16-bit V rows held as R[k] = 8 dims (8*l16 ..) of token tile_token(g, k).
@@ -495,7 +493,7 @@ struct VRegs<kFP> {
 template <>
 struct VRegs<kI4> {
     uint32_t v[8];
-    uint32_t vm[8];  // f32 scale bits
+    uint32_t vm[8];  // f32 scale bits of the N tokens whose probabilities the lane holds
 };
 template <>
 struct VRegs<kI2> {
@@ -598,38 +596,63 @@ __device__ __forceinline__ void qk_int2k(const QkOps& o, const VConst& vc, const
     }
 }
 
-// Logits of a tile in the lane's token order (masks only on partial tiles; padded heads have
-// q = 0, so their logits are 0: harmless, and their rows are never written out).
-__device__ __forceinline__ void tile_logits(const SegCtx& c, int a0, int g, const r2o_f4 (&s)[2], float (&sv)[8]) {
+// KV groups of at most this many query heads fill only half the MFMA's 16 columns.  Their query operand is
+// held twice (columns n and n + 8 are head n), so that both 16-token products of a tile have every head in
+// both column halves; taking the first product's rows in columns 0 .. 7 and the second's in 8 .. 15 leaves a
+// lane 4 logits that are all needed, in place of 8 of which half belong to padding.  The exponentials (a
+// quarter-rate instruction), sums and roundings of a tile halve for 4 selects and 2 or 4 DPP moves, which
+// bring the two halves of P together in lanes 0 .. 7 for the PV operand (rows 8 .. 15 of the product are
+// padding).
+constexpr int kSplitHeads = 8;
+
+// Logits of a tile in the lane's token order (masks only on partial tiles; padded heads have q = 0, so
+// their logits are 0: harmless, and their rows are never written out).  N = 8: tokens tile_token(g, k) of
+// head l16; N = 4: tokens 16 (l16 / 8) + 4 g + k of head l16 % 8.
+template <int N>
+__device__ __forceinline__ void tile_logits(const SegCtx& c, int a0, int l16, int g, const r2o_f4 (&s)[2],
+                                            float (&sv)[N]) {
     const bool full = __builtin_amdgcn_readfirstlane(a0 >= c.lo && a0 + 32 <= c.hi);
-    if (full) {
+    const bool second = l16 >= kSplitHeads;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) sv[k] = s[k >> 2][k & 3];
-    } else {
+    for (int k = 0; k < N; ++k) sv[k] = N == 8 ? s[k >> 2][k & 3] : (second ? s[1][k & 3] : s[0][k & 3]);
+    if (!full) {
+        const int first = a0 + (N == 4 && second ? 16 : 0) + 4 * g;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int pos = a0 + tile_token(g, k);
-            sv[k] = ((pos >= c.lo) & (pos < c.hi)) ? s[k >> 2][k & 3] : -INFINITY;
+        for (int k = 0; k < N; ++k) {
+            const int pos = first + (k < 4 ? k : 12 + k);
+            sv[k] = ((pos >= c.lo) & (pos < c.hi)) ? sv[k] : -INFINITY;
         }
     }
 }
 
-// PV of one tile with probabilities pk (the lane's 8 tokens).
-template <int KIND, bool TS, int RF>  // TS: INT2 values with one scale and zero point per token (group 128)
-__device__ __forceinline__ void pv_tile(WaveState& st, SegState<KIND>& ss, const VConst& vc, const float (&pk)[8],
+// The PV operand of a lane's 8 tokens from its own pairs w[0 .. N / 2 - 1]: split tiles take the second half
+// from lane l16 ^ 8.
+template <int N>
+__device__ __forceinline__ r2o_u4 pv_operand(const uint32_t (&w)[N / 2]) {
+    if constexpr (N == 8) return r2o_u4{w[0], w[1], w[2], w[3]};
+    else
+        return r2o_u4{w[0], w[1], __float_as_uint(r2o_lane_xor<8>(__uint_as_float(w[0]))),
+                      __float_as_uint(r2o_lane_xor<8>(__uint_as_float(w[1])))};
+}
+
+// PV of one tile with probabilities pk (the lane's N tokens).
+template <int KIND, bool TS, int RF, int N>  // TS: INT2 values with one scale and zero point per token (group 128)
+__device__ __forceinline__ void pv_tile(WaveState& st, SegState<KIND>& ss, const VConst& vc, const float (&pk)[N],
                                         const VRegs<KIND>& cur) {
     r2o_u4 ap;
+    uint32_t w[N / 2];
     if constexpr (KIND == kFP) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) ap[u] = pack_row2<RF>(pk[2 * u], pk[2 * u + 1]);
-        pv_rows<RF>(st, ap, cur.v);
+        for (int u = 0; u < N / 2; ++u) w[u] = pack_row2<RF>(pk[2 * u], pk[2 * u + 1]);
+        pv_rows<RF>(st, pv_operand<N>(w), cur.v);
     } else if constexpr (KIND == kI4) {
         // P' = p * s_t; the signed codes (xor 8) enter as 1032 + c (low nibble) and, read in
         // place, 1152 + 16 c (high nibble).  sum_k P'_k is accumulated by one more MFMA on the
         // same A operand (so both see identical f16 inputs) and the offsets are removed at the end.
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            ap[u] = r2o_pack_h2(pk[2 * u] * __uint_as_float(cur.vm[2 * u]), pk[2 * u + 1] * __uint_as_float(cur.vm[2 * u + 1]));
+        for (int u = 0; u < N / 2; ++u)
+            w[u] = r2o_pack_h2(pk[2 * u] * __uint_as_float(cur.vm[2 * u]), pk[2 * u + 1] * __uint_as_float(cur.vm[2 * u + 1]));
+        ap = pv_operand<N>(w);
         ss.bias[0] = r2o_mfma_f16(ap, r2o_u4{0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u}, ss.bias[0]);
         uint32_t X[8];
 #pragma unroll
@@ -656,12 +679,14 @@ __device__ __forceinline__ void pv_tile(WaveState& st, SegState<KIND>& ss, const
         // removed after the last tile.
         // p in f16 pairs, P' = p * s in packed f16 against the tokens' scale pairs; sum_k p_k accumulates
         // by one more MFMA (the softmax leaves l to it)
-        r2o_u4 p2;
+        uint32_t ws[N / 2];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            p2[u] = r2o_pack_h2(pk[2 * u], pk[2 * u + 1]);
-            ap[u] = r2o_h2_mul(p2[u], cur.vm[u]);
+        for (int u = 0; u < N / 2; ++u) {
+            w[u] = r2o_pack_h2(pk[2 * u], pk[2 * u + 1]);
+            ws[u] = r2o_h2_mul(w[u], cur.vm[u]);
         }
+        const r2o_u4 p2 = pv_operand<N>(w);
+        ap = pv_operand<N>(ws);
         const r2o_u4 ones = {0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
         ss.bias[2] = r2o_mfma_f16(p2, ones, ss.bias[2]);
         uint32_t yp[4], y8[4];
@@ -684,7 +709,8 @@ __device__ __forceinline__ void pv_tile(WaveState& st, SegState<KIND>& ss, const
         }
     } else {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) ap[u] = r2o_pack_h2(pk[2 * u], pk[2 * u + 1]);
+        for (int u = 0; u < N / 2; ++u) w[u] = r2o_pack_h2(pk[2 * u], pk[2 * u + 1]);
+        ap = pv_operand<N>(w);
         uint32_t yp[4], zp[4], sp[4];
 #pragma unroll
         for (int pr = 0; pr < 4; ++pr) {
@@ -721,9 +747,9 @@ __device__ __forceinline__ void qk_bf16k(const uint32_t (&qp)[4][4], float qscal
 }
 
 // One tile: QK, masks, online softmax, PV.
-template <int KIND, int KF, bool TS, int RF>
+template <int KIND, int KF, bool TS, int RF, int N>
 __device__ __forceinline__ void seg_compute(const SegCtx& c, WaveState& st, SegState<KIND>& ss, const VConst& vc,
-                                            int a0, int g, float qscale, const QkOps& qo,
+                                            int a0, int l16, int g, float qscale, const QkOps& qo,
                                             const TileRegs<KIND, KF>& cur) {
     r2o_f4 s[2];
     float corr = 0.f;
@@ -731,10 +757,10 @@ __device__ __forceinline__ void seg_compute(const SegCtx& c, WaveState& st, SegS
     else if constexpr (KF == kKInt4) qk_int4k(qo, vc, cur.kx, s);
     else qk_int2k(qo, vc, cur.kx, s);
     if constexpr (KF != kKBf16) corr = qo.corr;
-    float sv[8], pk[8];
-    tile_logits(c, a0, g, s, sv);
-    softmax_tile<TS ? 3 : (KIND == kI4 ? 1 : 0), !TS>(st, sv, pk, g, corr, ss.bias);
-    pv_tile<KIND, TS, RF>(st, ss, vc, pk, cur);
+    float sv[N], pk[N];
+    tile_logits<N>(c, a0, l16, g, s, sv);
+    softmax_tile<N, TS ? 3 : (KIND == kI4 ? 1 : 0), !TS>(st, sv, pk, g, corr, ss.bias);
+    pv_tile<KIND, TS, RF, N>(st, ss, vc, pk, cur);
 }
 
 // ------------------------------------------------------------------ pool tiles via LDS DMA
@@ -870,7 +896,7 @@ __device__ __forceinline__ void read_ops(const unsigned char* stage, int g, r2o_
         ko[j] = *reinterpret_cast<const r2o_u4*>(stage + StageLayout<KIND, KF>::kOps + g * 128 + 16 * j);
 }
 
-template <int KIND, int KF, bool TS = false>
+template <int KIND, int KF, bool TS, int N>
 __device__ __forceinline__ void read_tile(const unsigned char* stage, int l16, int g, int gamma, int groups,
                                           TileRegs<KIND, KF>& tr) {
     using Lay = StageLayout<KIND, KF>;
@@ -899,19 +925,34 @@ __device__ __forceinline__ void read_tile(const unsigned char* stage, int l16, i
             tr.v[k] = *reinterpret_cast<const r2o_u4*>(stage + Lay::kV + 256 * t + 16 * l16);
         } else if constexpr (KIND == kI4) {
             tr.v[k] = *reinterpret_cast<const uint32_t*>(stage + Lay::kV + 16 * v4_slot(t, l16 >> 2) + 4 * (l16 & 3));
-            tr.vm[k] = *reinterpret_cast<const uint32_t*>(stage + Lay::kScale + 4 * t);
-        } else if constexpr (TS) {  // one group per token: scales and zeros of tokens t, t + 1 (t even) together
+        } else if constexpr (TS) {
             tr.v[k] = *reinterpret_cast<const uint16_t*>(stage + Lay::kV + 16 * v2_slot(t, l16 >> 3) + 2 * (l16 & 7));
-            if ((k & 1) == 0) {  // one dword slot per token: the 8 bytes at 4t hold both tokens' slots
-                const uint2 sc = *reinterpret_cast<const uint2*>(stage + Lay::kScale + 4 * t);
-                const uint2 zr = *reinterpret_cast<const uint2*>(stage + Lay::kZero + 4 * t);
-                tr.vm[k >> 1] = r2o_perm(sc.y, sc.x, 0x05040100u);  // (s_t, s_t+1) as an f16 pair
-                tr.vz[k >> 1] = r2o_perm(zr.y, zr.x, 0x0C040C00u);  // z_t | z_t+1 << 16
-            }
         } else {  // scale rows: 8 bytes (G = 32) or one dword slot; zero rows: one dword slot
             tr.v[k] = *reinterpret_cast<const uint16_t*>(stage + Lay::kV + 16 * v2_slot(t, l16 >> 3) + 2 * (l16 & 7));
             tr.vm[k] = *reinterpret_cast<const uint16_t*>(stage + Lay::kScale + t * (groups == 4 ? 8 : 4) + 2 * gamma);
             tr.vz[k] = *(stage + Lay::kZero + 4 * t + gamma);
+        }
+    }
+    // per-token metadata in one dword slot per token, 4 adjacent tokens a read: the scales of the N tokens whose
+    // probabilities the lane holds (split tiles: of one half), the zero points of all 8
+    const unsigned char* mine = stage + Lay::kScale + 16 * g + (N == 4 ? 64 * (l16 >> 3) : 0);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        if constexpr (KIND == kI4) {
+            if (e < N / 4) {
+                const r2o_u4 sc = *reinterpret_cast<const r2o_u4*>(mine + 64 * e);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) tr.vm[4 * e + k] = sc[k];
+            }
+        } else if constexpr (TS) {  // pairs of tokens: (s_t, s_t+1) as f16, z_t | z_t+1 << 16
+            if (e < N / 4) {
+                const r2o_u4 sc = *reinterpret_cast<const r2o_u4*>(mine + 64 * e);
+                tr.vm[2 * e] = r2o_perm(sc[1], sc[0], 0x05040100u);
+                tr.vm[2 * e + 1] = r2o_perm(sc[3], sc[2], 0x05040100u);
+            }
+            const r2o_u4 zr = *reinterpret_cast<const r2o_u4*>(stage + Lay::kZero + 16 * g + 64 * e);
+            tr.vz[2 * e] = r2o_perm(zr[1], zr[0], 0x0C040C00u);
+            tr.vz[2 * e + 1] = r2o_perm(zr[3], zr[2], 0x0C040C00u);
         }
     }
 }
@@ -938,7 +979,8 @@ __device__ __forceinline__ void touch_combine_kernarg(const r2o_decode_params& p
                  "s"(p.output_hadamard), "s"(ca.gqa), "s"(ca.n_groups), "s"(range_begin), "s"(range_end));
 }
 
-template <int KIND, int KF, bool TS, int RF, int RO>
+// N: logits per lane and tile, 4 for groups of at most kSplitHeads query heads, else 8.
+template <int KIND, int KF, bool TS, int RF, int RO, int N>
 __device__ __forceinline__ void run_segment(const r2o_decode_params& p, const r2o_work_item& it,
                                             unsigned char* smem, WaveState& st, Stamps& ts) {
     using Cfg = KernelCfg<KF>;
@@ -1000,6 +1042,7 @@ __device__ __forceinline__ void run_segment(const r2o_decode_params& p, const r2
     for (int j = 0; j < kDmaStages; ++j)
         if (j < n) dma_tile<KIND, KF>(c, a_first + 32 * j, ring + j * Cfg::kStage, lane, true);
     stamp(ts, 2);
+    const int head = N == 4 ? l16 & (kSplitHeads - 1) : l16;  // of the lane's query operand and logits
     r2o_u4 qrot[4];
     if constexpr (RO != kRopeNone) {  // the waves share the rotation while their first tiles are in flight
         uint16_t* rot = reinterpret_cast<uint16_t*>(smem + Cfg::kSmem);
@@ -1011,13 +1054,13 @@ __device__ __forceinline__ void run_segment(const r2o_decode_params& p, const r2
         }
         __syncthreads();
         if (n <= 0) return;
-        rot_read_query(rot, gqa, l16, g, qrot);
+        rot_read_query(rot, gqa, head, g, qrot);
     }
 
     const VConst vc = make_vconst();
     const float qscale = p.sm_scale * kLog2e;
     SegState<KIND> ss;
-    load_query<KF, RF, RO>(p, b, kvh, gqa, l16, g, qscale, ss.qp, qrot);  // BF16-K: row-type pairs, scaled after the MFMA
+    load_query<KF, RF, RO>(p, b, kvh, gqa, head, g, qscale, ss.qp, qrot);  // BF16-K: row-type pairs, scaled after the MFMA
 #pragma unroll
     for (int e = 0; e < (KIND == kI2 ? 3 : 2); ++e) ss.bias[e] = r2o_f4{0, 0, 0, 0};
     const SegCtx sc = {c.lo, c.hi};
@@ -1029,7 +1072,7 @@ __device__ __forceinline__ void run_segment(const r2o_decode_params& p, const r2
         if (i == n - 1) stamp(ts, 4);
         unsigned char* stage = ring + (i % kDmaStages) * Cfg::kStage;
         TileRegs<KIND, KF> cur;
-        read_tile<KIND, KF, TS>(stage, l16, g, gamma, c.groups, cur);
+        read_tile<KIND, KF, TS, N>(stage, l16, g, gamma, c.groups, cur);
         const bool fresh = __builtin_amdgcn_readfirstlane(needs_ops(i));  // wave-uniform
         r2o_u4 ko[8];
         if constexpr (KF != kKBf16)
@@ -1044,7 +1087,7 @@ __device__ __forceinline__ void run_segment(const r2o_decode_params& p, const r2
         } else if constexpr (KF == kKInt2) {
             if (fresh) qk_ops_int2k(ss.qp, ko, qo);
         }
-        seg_compute<KIND, KF, TS, RF>(sc, st, ss, vc, a_first + 32 * i, g, qscale, qo, cur);
+        seg_compute<KIND, KF, TS, RF, N>(sc, st, ss, vc, a_first + 32 * i, l16, g, qscale, qo, cur);
     }
     if constexpr (TS) {  // column q = 4^-u (sum P' (1024 + 4^u c)) - sum P' (1024 + z) + 1024 (1 - 4^-u) sum P'
 #pragma unroll
@@ -1057,7 +1100,7 @@ __device__ __forceinline__ void run_segment(const r2o_decode_params& p, const r2
         const int r = l16 & 3;
         const float mine = r == 0 ? ss.bias[2][0] : (r == 1 ? ss.bias[2][1] : (r == 2 ? ss.bias[2][2] : ss.bias[2][3]));
         const float head_l = __shfl(mine, 16 * (l16 >> 2) + l16, R2O_WAVE);
-        st.l = g == 0 ? head_l : 0.f;
+        st.l = g == 0 && (N == 8 || l16 < kSplitHeads) ? head_l : 0.f;
     }
     if constexpr (KIND == kI4) {  // remove the code offsets: lo dims 1032 * sum P', hi dims (1152 * sum P') / 16
 #pragma unroll
@@ -1159,7 +1202,7 @@ __device__ __forceinline__ void run_recent(const r2o_decode_params& p, const r2o
         float sv[8], pk[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) sv[k] = ((a0 + tile_token(g, k) < valid_end) & head_ok) ? s[k >> 2][k & 3] : -INFINITY;
-        softmax_tile(st, sv, pk, g);
+        softmax_tile<8>(st, sv, pk, g);
         r2o_u4 ap;
 #pragma unroll
         for (int u = 0; u < 4; ++u) ap[u] = pack_row2<RF>(pk[2 * u], pk[2 * u + 1]);
@@ -1167,9 +1210,23 @@ __device__ __forceinline__ void run_recent(const r2o_decode_params& p, const r2o
     }
 }
 
-template <int KF, int RF, int RO>
-__global__ __launch_bounds__(KernelCfg<KF>::kThreads, KernelCfg<KF>::kWavesPerSimd) void decode_partial_kernel(
-        r2o_decode_params p) {
+// The tiles of a pool segment, by its kind.
+template <int KF, int RF, int RO, int N>
+__device__ __forceinline__ void run_pool(const r2o_decode_params& p, const r2o_work_item& it, unsigned char* smem,
+                                         WaveState& st, Stamps& ts) {
+    switch (it.kind) {
+        case kFP: run_segment<kFP, KF, false, RF, RO, N>(p, it, smem, st, ts); break;
+        case kI4: run_segment<kI4, KF, false, RF, RO, N>(p, it, smem, st, ts); break;
+        default:  // INT2 values: one scale and zero point per token when a group spans all 128 dims
+            if (it.v_group == 128) run_segment<kI2, KF, true, RF, RO, N>(p, it, smem, st, ts);
+            else run_segment<kI2, KF, false, RF, RO, N>(p, it, smem, st, ts);
+            break;
+    }
+}
+
+// One work item; the whole partial kernel.  N: see kSplitHeads.
+template <int KF, int RF, int RO, int N>
+__device__ __forceinline__ void decode_item(const r2o_decode_params& p) {
     constexpr int kWaves = KernelCfg<KF>::kWaves;
     __shared__ __align__(16) unsigned char smem[KernelCfg<KF>::kSmem + (RO != kRopeNone ? kRotBytes : 0)];
     Stamps ts{};
@@ -1195,20 +1252,14 @@ __global__ __launch_bounds__(KernelCfg<KF>::kThreads, KernelCfg<KF>::kWavesPerSi
 #pragma unroll
     for (int q = 0; q < 8; ++q) st.acc[q] = r2o_f4{0, 0, 0, 0};
 
-    switch (it.kind) {
-        case kFP: run_segment<kFP, KF, false, RF, RO>(p, it, smem, st, ts); break;
-        case kI4: run_segment<kI4, KF, false, RF, RO>(p, it, smem, st, ts); break;
-        case kI2:  // INT2 values: one scale and zero point per token when a group spans all 128 dims
-            if (it.v_group == 128) run_segment<kI2, KF, true, RF, RO>(p, it, smem, st, ts);
-            else run_segment<kI2, KF, false, RF, RO>(p, it, smem, st, ts);
-            break;
-        default: run_recent<KF, RF, RO>(p, it, smem, st); break;
-    }
+    if (it.kind == kRecent) run_recent<KF, RF, RO>(p, it, smem, st);
+    else run_pool<KF, RF, RO, N>(p, it, smem, st, ts);
 
     // ---- per-wave epilogue: reduce l (and u) over the 4 lane groups of each head
     float l_h = st.l;
     l_h = r2o_sum_lane_pair<16>(l_h);
     l_h = r2o_sum_lane_pair<32>(l_h);
+    if constexpr (N == 4) l_h += r2o_lane_xor<8>(l_h);  // split tiles (ring items: lanes 8 .. 15 are padding, l = 0)
     stamp(ts, 5);
     // each wave's state goes to the start of its own DMA ring, whose tiles it has all read: no wave
     // waits for the others before writing (one barrier less than a shared merge area)
@@ -1266,6 +1317,22 @@ __global__ __launch_bounds__(KernelCfg<KF>::kThreads, KernelCfg<KF>::kWavesPerSi
 #ifdef R2O_TIMELINE
     stamps_store(g_timeline_partial, blockIdx.x, wave, kTimelineWaves, ts);
 #endif
+}
+
+// Split tiles (see kSplitHeads) are for INT2-K, the one key format whose loop is bound by VALU issue: measured
+// on 131k tokens, 32 / 8 heads, its call falls from 25.3 to 24.4 us, while INT4-K and 16-bit keys, which
+// wait for their tiles, stay where they are (+-0.4 % on the 7B and MiniCPM shapes, the folded rotation
+// 0.4 % slower).  INT2-K groups of more heads have a kernel of their own, so that neither carries the
+// other's code.
+template <int KF, int RF, int RO>
+__global__ __launch_bounds__(KernelCfg<KF>::kThreads, KernelCfg<KF>::kWavesPerSimd) void decode_partial_kernel(
+        r2o_decode_params p) {
+    decode_item<KF, RF, RO, KF == kKInt2 ? 4 : 8>(p);
+}
+template <int RF, int RO>
+__global__ __launch_bounds__(KernelCfg<kKInt2>::kThreads, KernelCfg<kKInt2>::kWavesPerSimd) void decode_partial_wide_kernel(
+        r2o_decode_params p) {
+    decode_item<kKInt2, RF, RO, 8>(p);
 }
 
 // Fused Recent-FP append (triton_fourq_splitk.py:1007-1020) of every KV head of request b, by one
@@ -1571,24 +1638,32 @@ float* scratch_address(int dev) {
     return ptr;
 }
 
+template <int KF, int RF, int RO>
+void launch_partial_of(const r2o_decode_params& p, hipStream_t stream) {
+    const dim3 grid((unsigned)p.n_items), block(KernelCfg<KF>::kThreads);
+    if constexpr (KF == kKInt2)
+        if (p.hq / p.hkv > kSplitHeads) {
+            hipLaunchKernelGGL((decode_partial_wide_kernel<RF, RO>), grid, block, 0, stream, p);
+            return;
+        }
+    hipLaunchKernelGGL((decode_partial_kernel<KF, RF, RO>), grid, block, 0, stream, p);
+}
+
 template <int RO>
 void launch_partial(const r2o_decode_params& p, hipStream_t stream) {
-    const dim3 grid((unsigned)p.n_items);
-    const dim3 block(KernelCfg<kKInt4>::kThreads), block_bf16(KernelCfg<kKBf16>::kThreads);
-    static_assert(KernelCfg<kKInt4>::kThreads == KernelCfg<kKInt2>::kThreads, "one workgroup size for the low-bit K formats");
     const bool f16 = p.row_dtype == kRowF16;
     switch (p.k_format) {
         case kKInt4:
-            if (f16) hipLaunchKernelGGL((decode_partial_kernel<kKInt4, kRowF16, RO>), grid, block, 0, stream, p);
-            else hipLaunchKernelGGL((decode_partial_kernel<kKInt4, kRowBf16, RO>), grid, block, 0, stream, p);
+            if (f16) launch_partial_of<kKInt4, kRowF16, RO>(p, stream);
+            else launch_partial_of<kKInt4, kRowBf16, RO>(p, stream);
             break;
         case kKBf16:
-            if (f16) hipLaunchKernelGGL((decode_partial_kernel<kKBf16, kRowF16, RO>), grid, block_bf16, 0, stream, p);
-            else hipLaunchKernelGGL((decode_partial_kernel<kKBf16, kRowBf16, RO>), grid, block_bf16, 0, stream, p);
+            if (f16) launch_partial_of<kKBf16, kRowF16, RO>(p, stream);
+            else launch_partial_of<kKBf16, kRowBf16, RO>(p, stream);
             break;
         default:
-            if (f16) hipLaunchKernelGGL((decode_partial_kernel<kKInt2, kRowF16, RO>), grid, block, 0, stream, p);
-            else hipLaunchKernelGGL((decode_partial_kernel<kKInt2, kRowBf16, RO>), grid, block, 0, stream, p);
+            if (f16) launch_partial_of<kKInt2, kRowF16, RO>(p, stream);
+            else launch_partial_of<kKInt2, kRowBf16, RO>(p, stream);
             break;
     }
 }

@@ -11,6 +11,7 @@ import os
 import shutil
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 ROOT_DIR = os.path.dirname(PKG_DIR)                 # r2-omni_amd/
@@ -52,35 +53,35 @@ def common_flags() -> list[str]:
 def build_library(verbose: bool = False) -> str:
     """Compile every source and link ``libr2o_sspa.so`` (and bench.py's ``libr2o_bench.so`` and
     ``libr2o_timeline.so``) next to this file; returns the decode library's path."""
-    _link(SOURCES, LIB_PATH, verbose)
-    _link(BENCH_SOURCES, BENCH_LIB_PATH, verbose)
-    _link(SOURCES, TIMELINE_LIB_PATH, verbose, defines=("R2O_TIMELINE",), rebuild=("r2o_decode.hip",))
+    timeline = ("R2O_TIMELINE",)
+    jobs = [(src, ()) for src in SOURCES + BENCH_SOURCES] + [("r2o_decode.hip", timeline)]
+    with ThreadPoolExecutor() as pool:  # one compiler process each; the decode kernels take most of the time
+        objects = dict(zip(jobs, pool.map(lambda job: _compile(*job, verbose), jobs)))
+    _link([objects[src, ()] for src in SOURCES], LIB_PATH, verbose)
+    _link([objects[src, ()] for src in BENCH_SOURCES], BENCH_LIB_PATH, verbose)
+    _link([objects.get((src, timeline), objects[src, ()]) for src in SOURCES], TIMELINE_LIB_PATH, verbose)
     return LIB_PATH
 
 
-def _link(sources, path: str, verbose: bool, defines=(), rebuild=None) -> None:
-    """Compile ``sources`` (only those in ``rebuild`` when given, reusing the other objects of the
-    plain build) with ``defines`` and link them into ``path``."""
-    hipcc = _hipcc()
+def _compile(src: str, defines: tuple, verbose: bool) -> str:
+    """The object of one source, built with ``defines``; a HIP source's kernels are checked for scratch use."""
     build_dir = os.path.join(ROOT_DIR, "_build")
     os.makedirs(build_dir, exist_ok=True)
     suffix = "".join("_" + d.lower() for d in defines)
-    objects = []
-    for src in sources:
-        stem = os.path.splitext(src)[0]
-        if rebuild is not None and src not in rebuild:
-            objects.append(os.path.join(build_dir, stem + ".o"))
-            continue
-        obj = os.path.join(build_dir, stem + suffix + ".o")
-        cmd = [hipcc, *common_flags(), *[f"-D{d}" for d in defines], "-c", os.path.join(CSRC, src), "-o", obj]
-        if src.endswith(".hip"):
-            cmd.append("-Rpass-analysis=kernel-resource-usage")
-        stderr = _run(cmd, verbose)
-        if src.endswith(".hip"):
-            _check_resources(src + suffix, stderr, os.path.join(build_dir, stem + suffix + ".resources.txt"))
-        objects.append(obj)
+    stem = os.path.splitext(src)[0]
+    obj = os.path.join(build_dir, stem + suffix + ".o")
+    cmd = [_hipcc(), *common_flags(), *[f"-D{d}" for d in defines], "-c", os.path.join(CSRC, src), "-o", obj]
+    if src.endswith(".hip"):
+        cmd.append("-Rpass-analysis=kernel-resource-usage")
+    stderr = _run(cmd, verbose)
+    if src.endswith(".hip"):
+        _check_resources(src + suffix, stderr, os.path.join(build_dir, stem + suffix + ".resources.txt"))
+    return obj
+
+
+def _link(objects: list[str], path: str, verbose: bool) -> None:
     tmp = path + ".tmp"
-    _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objects, "-o", tmp], verbose)
+    _run([_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objects, "-o", tmp], verbose)
     os.replace(tmp, path)
 
 
