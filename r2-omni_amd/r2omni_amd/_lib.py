@@ -191,6 +191,27 @@ def load() -> ctypes.CDLL:
     return _LIB
 
 
+_HOST = None
+
+
+def host():
+    """The package's native host module (r2o_host.cpp), loaded on first use like the library and as loudly."""
+    global _HOST
+    if _HOST is None:
+        try:
+            from . import _r2o_host
+        except ImportError as e:
+            raise RuntimeError("the native host module _r2o_host.so is missing or does not load: build it with "
+                               f"`python -m r2omni_amd.build` ({e})") from e
+        _HOST = _r2o_host
+    return _HOST
+
+
+def address(name: str) -> int:
+    """Address of one of the library's functions, for the host module."""
+    return ctypes.cast(getattr(load(), name), ctypes.c_void_p).value
+
+
 def check(rc: int, name: str) -> None:
     if rc == 0:
         return

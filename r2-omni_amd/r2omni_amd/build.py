@@ -26,6 +26,9 @@ BENCH_LIB_PATH = os.path.join(PKG_DIR, "libr2o_bench.so")
 BENCH_SOURCES = ("bench_read.hip",)
 # the same decode library built with per-wave phase stamps (-DR2O_TIMELINE), for bench.py --timeline only
 TIMELINE_LIB_PATH = os.path.join(PKG_DIR, "libr2o_timeline.so")
+# the package's native host module (a CPython extension over torch's C++ API; no GPU code)
+HOST_SOURCE = "r2o_host.cpp"
+HOST_PATH = os.path.join(PKG_DIR, "_r2o_host.so")
 ARCH = "gfx950"
 
 
@@ -51,16 +54,38 @@ def common_flags() -> list[str]:
 
 
 def build_library(verbose: bool = False) -> str:
-    """Compile every source and link ``libr2o_sspa.so`` (and bench.py's ``libr2o_bench.so`` and
-    ``libr2o_timeline.so``) next to this file; returns the decode library's path."""
+    """Compile every source and link ``libr2o_sspa.so`` (and the host module ``_r2o_host.so``, bench.py's
+    ``libr2o_bench.so`` and ``libr2o_timeline.so``) next to this file; returns the decode library's path."""
     timeline = ("R2O_TIMELINE",)
-    jobs = [(src, ()) for src in SOURCES + BENCH_SOURCES] + [("r2o_decode.hip", timeline)]
+    jobs = [(src, ()) for src in SOURCES + BENCH_SOURCES + (HOST_SOURCE,)] + [("r2o_decode.hip", timeline)]
     with ThreadPoolExecutor() as pool:  # one compiler process each; the decode kernels take most of the time
         objects = dict(zip(jobs, pool.map(lambda job: _compile(*job, verbose), jobs)))
     _link([objects[src, ()] for src in SOURCES], LIB_PATH, verbose)
     _link([objects[src, ()] for src in BENCH_SOURCES], BENCH_LIB_PATH, verbose)
     _link([objects.get((src, timeline), objects[src, ()]) for src in SOURCES], TIMELINE_LIB_PATH, verbose)
+    _link([objects[HOST_SOURCE, ()]], HOST_PATH, verbose, _torch_libraries())
     return LIB_PATH
+
+
+def _host_flags() -> list[str]:
+    """Flags of the host module: torch's C++ API and CPython's, host code only."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    return ["-x", "c++", "-O2", "-fPIC", "-std=c++17", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", INCLUDE,
+            "-I", sysconfig.get_paths()["include"],
+            *[a for p in [*include_paths(), os.path.join(os.path.dirname(os.path.dirname(_hipcc())), "include")]
+              for a in ("-isystem", p)]]
+
+
+def _torch_libraries() -> list[str]:
+    import torch
+
+    path = os.path.join(os.path.dirname(torch.__file__), "lib")
+    return ["-L", path, f"-Wl,-rpath,{path}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
 
 
 def _compile(src: str, defines: tuple, verbose: bool) -> str:
@@ -70,7 +95,8 @@ def _compile(src: str, defines: tuple, verbose: bool) -> str:
     suffix = "".join("_" + d.lower() for d in defines)
     stem = os.path.splitext(src)[0]
     obj = os.path.join(build_dir, stem + suffix + ".o")
-    cmd = [_hipcc(), *common_flags(), *[f"-D{d}" for d in defines], "-c", os.path.join(CSRC, src), "-o", obj]
+    flags = _host_flags() if src == HOST_SOURCE else common_flags()
+    cmd = [_hipcc(), *flags, *[f"-D{d}" for d in defines], "-c", os.path.join(CSRC, src), "-o", obj]
     if src.endswith(".hip"):
         cmd.append("-Rpass-analysis=kernel-resource-usage")
     stderr = _run(cmd, verbose)
@@ -79,9 +105,9 @@ def _compile(src: str, defines: tuple, verbose: bool) -> str:
     return obj
 
 
-def _link(objects: list[str], path: str, verbose: bool) -> None:
+def _link(objects: list[str], path: str, verbose: bool, libraries=()) -> None:
     tmp = path + ".tmp"
-    _run([_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objects, "-o", tmp], verbose)
+    _run([_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objects, *libraries, "-o", tmp], verbose)
     os.replace(tmp, path)
 
 

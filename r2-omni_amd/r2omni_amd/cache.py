@@ -17,6 +17,7 @@ cache; generated (flushed) values INT2 (released) or INT4 (``generated_value_pre
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass, field
 from typing import Any, Literal, NamedTuple
 
@@ -965,8 +966,8 @@ def _metadata_words(tier_pages, tier_tokens, *, page_size: int, recent_capacity:
 def _build_metadata_arena(tab: _TierTable, tokens: torch.Tensor, gi: torch.Tensor, lp: torch.Tensor, *,
                           page_size: int, recent_capacity: int, int2_reserve: int, int4_reserve: int = 0):
     """The metadata arena of ``_metadata_views`` filled by torch on any device, from the tier-ordered token
-    indices of ``_expand_tier_tokens`` and the plan's global / logical token indices (a cache build fills
-    its arena by ``r2o_cache_build``)."""
+    indices of ``_expand_tier_tokens`` and the plan's global / logical token indices: what ``r2o_cache_build``
+    writes, restated (a cache build fills its arena there)."""
     ps, cap = int(page_size), int(recent_capacity)
     sizes = dict(page_size=ps, recent_capacity=cap, int2_reserve=int(int2_reserve), int4_reserve=int(int4_reserve))
     tier_pages = np.diff(tab.first_page)
@@ -1137,12 +1138,12 @@ def _build_matched_cache(key, value, plan: LayerCompressionPlan, append_capacity
 
 def _build_tiered_cache(key, value, plan: LayerCompressionPlan, append_capacity: int, superblock: int, group: int,
                         common: dict) -> ThreePrecisionCache:
-    """The three pools and their metadata arena (precision_pool.py:878-984): every tensor allocated here,
-    unwritten, and filled by the two launches of ``r2o_cache_build`` behind one upload of the page table."""
-    dev, h, s = key.device, int(key.shape[0]), int(key.shape[1])
+    """The three pools and their metadata arena (precision_pool.py:878-984): one native call allocates every
+    tensor, uploads the page table and makes the two launches of ``r2o_cache_build``."""
+    dev, s = key.device, int(key.shape[1])
     ps, cap = common["page_size"], int(plan.recent_fp_capacity)
     _lib.require_device(value, "value")
-    value_code = _lib.dtype_code(value.dtype)
+    _lib.dtype_code(value.dtype)
     if group not in (32, 64, 128):
         raise ValueError("compact INT2 V requires group_size 32, 64, or 128")
     if append_capacity < 0:
@@ -1150,13 +1151,12 @@ def _build_tiered_cache(key, value, plan: LayerCompressionPlan, append_capacity:
     # the kernels move rows in 16-byte pieces; a view may start between them
     key, value = (t.clone() if t.data_ptr() % 16 else t for t in (key, value))
     table = _host_page_table(plan)
-    n_pages = int(table.shape[1])
-    counts = np.empty(8, dtype=np.int64)
+    counts = (ctypes.c_int64 * 8)()
     lib = _lib.load()
-    if lib.r2o_cache_pages(table.data_ptr(), n_pages, s, counts.ctypes.data, counts.ctypes.data + 32):
+    if lib.r2o_cache_pages(table.data_ptr(), int(table.shape[1]), s, counts, ctypes.byref(counts, 32)):
         _tier_page_table(plan)  # names an unknown class
         raise ValueError("static plan pages must lie inside the K/V sequence")
-    tier_pages, tier_tokens = counts[:4].tolist(), counts[4:].tolist()
+    tier_pages, tier_tokens = tuple(counts[:4]), tuple(counts[4:])
     if sum(tier_tokens) != s:
         raise ValueError("compact physical pools must cover every logical token")
     gi = plan.global_token_indices.detach().to(dev, torch.long).contiguous()
@@ -1165,86 +1165,47 @@ def _build_tiered_cache(key, value, plan: LayerCompressionPlan, append_capacity:
         raise ValueError("static plan indices must cover the K/V sequence")
     s_fp, s_i4, s_i2, _ = tier_tokens
     n = s_fp + s_i4 + s_i2
+    int2_keys = common["cache_variant"] == "v_fourq_k_int2_compact"
     bf16_keys = common["cache_variant"] == "v_fourq_k_bf16"  # key rows in the model dtype (bf16 or fp16)
     int4_generated = common["generated_value_precision"] == "int4"
+    rc, payload, meta = _lib.host().cache_build(
+        key, value, gi, lp, table, _lib.address("r2o_cache_page_words"), _lib.address("r2o_cache_build"), tier_pages,
+        tier_tokens, ps, cap, append_capacity, superblock, group, 16 if bf16_keys else (2 if int2_keys else 4), int4_generated)
+    _lib.check(rc, "r2o_cache_build")
+    fp_v, i4_packed, i4_scale, i2_packed, i2_scale, i2_zero, k_packed, k_scale, k_zero, k_ops, ring_k, ring_v = payload
 
-    def empty(shape, dtype):
-        return torch.empty(shape, device=dev, dtype=dtype)
-
-    fp_v = empty((h, s_fp, 128), value.dtype) if s_fp else None
-    int4_v = compact_int4_value = None
-    i4_capacity = 0
+    int4_v = compact_int4_value = compact_key = bf16_arena = None
     if int4_generated:  # the INT4 pool's V is an arena with room for generated flushes (precision_pool.py:935-942)
-        i4_capacity = max(1, s_i4 + append_capacity)
-        compact_int4_value = int4_v = CompactInt4ValueArena(
-            packed=empty((h, i4_capacity, 64), torch.uint8), scale=empty((h, i4_capacity, 1), torch.float32),
-            active_length=s_i4, capacity=i4_capacity, original_dtype=value.dtype)
+        compact_int4_value = int4_v = CompactInt4ValueArena(packed=i4_packed, scale=i4_scale, active_length=s_i4,
+                                                            capacity=int(i4_packed.shape[1]), original_dtype=value.dtype)
     elif s_i4:
-        i4_capacity = s_i4
-        int4_v = _packed_int4(empty(h * s_i4 * 64, torch.uint8), empty((h, s_i4, 1), torch.float32), h, s_i4, value.dtype)
-    i2_capacity = max(128, _round_up(s_i2 + (0 if int4_generated else append_capacity), 128))
-    compact_value = CompactInt2ValueArena(
-        packed=empty((h, i2_capacity, 32), torch.uint8), scale=empty((h, i2_capacity, 128 // group, 1), torch.float16),
-        zero_point=empty((h, i2_capacity, 128 // group, 1), torch.uint8), active_length=s_i2, capacity=i2_capacity,
-        original_dtype=value.dtype, group_size=group)
-    capacity = max(128, _round_up(n + append_capacity, 128))
-    segments = (0, s_fp, s_fp + s_i4)
-    compact_key = bf16_arena = None
-    reserve = reserve4 = 0
-    if bf16_keys:  # no compact K arena to flush into: nothing is reserved (precision_pool.py:404-408, 878-906)
-        bf16_arena = BF16KeyArena(rows=empty((h, capacity, 128), key.dtype), active_length=n, capacity=capacity,
-                                  segment_offsets=segments)
-        k_fields = dict(k_bits=16, k_packed=bf16_arena.rows.data_ptr(), k_capacity=capacity)
+        int4_v = _packed_int4(i4_packed, i4_scale, int(key.shape[0]), s_i4, value.dtype)
+    compact_value = CompactInt2ValueArena(packed=i2_packed, scale=i2_scale, zero_point=i2_zero, active_length=s_i2,
+                                          capacity=int(i2_packed.shape[1]), original_dtype=value.dtype, group_size=group)
+    segments, capacity = (0, s_fp, s_fp + s_i4), int(k_packed.shape[1])
+    if bf16_keys:  # every pool keeps 16-bit K rows, and nothing is reserved (precision_pool.py:404-408, 878-906)
+        bf16_arena = BF16KeyArena(rows=k_packed, active_length=n, capacity=capacity, segment_offsets=segments)
     else:
-        int2_keys = common["cache_variant"] == "v_fourq_k_int2_compact"
-        blocks = capacity // superblock
-        arena_class = CompactInt2KeyArena if int2_keys else CompactInt4KeyArena
-        compact_key = arena_class(
-            packed=empty((h, capacity, 32 if int2_keys else 64), torch.uint8), scale=empty((h, blocks, 128), torch.float16),
-            zero_point=empty((h, blocks, 128), torch.float16 if int2_keys else torch.uint8), active_length=n,
-            capacity=capacity, segment_offsets=segments, original_dtype=key.dtype, superblock_size=superblock,
-            kernel_operands=empty((h, blocks, 128), torch.int32))
-        room = capacity - n
-        reserve = min(i2_capacity - s_i2, room) // ps * ps
-        reserve4 = min(i4_capacity - s_i4, room) // ps * ps if int4_generated else 0
-        k_fields = dict(k_bits=compact_key.bit_width, superblock=superblock, k_packed=compact_key.packed.data_ptr(),
-                        k_scale=compact_key.scale.data_ptr(), k_zero=compact_key.zero_point.data_ptr(),
-                        k_operands=compact_key.kernel_operands.data_ptr(), k_capacity=capacity, k_superblocks=blocks)
-    ring_k, ring_v = empty((h, cap, 128), key.dtype), empty((h, cap, 128), key.dtype)
-
-    sizes = dict(page_size=ps, recent_capacity=cap, int2_reserve=reserve, int4_reserve=reserve4)
-    page_words, total = _metadata_words(tier_pages, tier_tokens, **sizes)
-    words = torch.empty(page_words + 3 * n_pages, dtype=torch.long, pin_memory=True)
-    _lib.check(lib.r2o_cache_page_words(table.data_ptr(), n_pages, ps, reserve4, reserve, cap, words.data_ptr(),
-                                        words.numel()), "r2o_cache_page_words")
-    pages = words.to(dev, non_blocking=True)  # pinned: a copy from pageable memory would wait for the stream
-    storage, index = empty(total, torch.long), empty(n, torch.long)
-    _lib.call("r2o_cache_build", _lib.CacheBuild(
-        key=key.data_ptr(), value=value.data_ptr(), key_dtype=_lib.dtype_code(key.dtype), value_dtype=value_code, hkv=h,
-        tokens=s, plan_global=gi.data_ptr(), plan_logical=lp.data_ptr(), pages=pages.data_ptr(), page_words=page_words,
-        n_pages=n_pages, tier_tokens=tuple(tier_tokens), reserve4=reserve4, reserve2=reserve, storage=storage.data_ptr(),
-        index=index.data_ptr(), ring_k=ring_k.data_ptr(), ring_v=ring_v.data_ptr(), ring_capacity=cap,
-        fp_v=_lib.ptr(fp_v), i4_v=None if int4_v is None else int4_v.packed.data_ptr(),
-        i4_scale=None if int4_v is None else int4_v.scale.data_ptr(), i4_capacity=i4_capacity,
-        i2_v=compact_value.packed.data_ptr(), i2_scale=compact_value.scale.data_ptr(),
-        i2_zero=compact_value.zero_point.data_ptr(), i2_capacity=i2_capacity, i2_group=group, **k_fields),
-        _lib.stream_of(dev))
-
-    meta, (fp_pi, i4_pi, i2_pi, ring_pi), evicted, (ring_g, ring_l, ring_len) = _metadata_views(
-        storage, tier_pages, tier_tokens, **sizes)
-    fp_pool = PrecisionPool(name="fp", page_index=fp_pi, fp_v=fp_v)
-    int4_pool = PrecisionPool(name="int4", page_index=i4_pi, packed_v=int4_v)
-    int2_pool = PrecisionPool(name="int2", page_index=i2_pi, packed_v=compact_value)
-    recent = PrecisionPool(name="recent_fp", page_index=ring_pi, fp_k=ring_k, fp_v=ring_v, active_length=0, capacity=cap,
-                           length_device=ring_len, global_index_buffer=ring_g, logical_position_buffer=ring_l)
+        compact_key = (CompactInt2KeyArena if int2_keys else CompactInt4KeyArena)(
+            packed=k_packed, scale=k_scale, zero_point=k_zero, active_length=n, capacity=capacity, segment_offsets=segments,
+            original_dtype=key.dtype, superblock_size=superblock, kernel_operands=k_ops)
+    arena = CompactMetadataArena(
+        meta[0], *meta[7:10], meta[16], meta[19], tier_pages[2], s_i2, *meta[4:7], meta[15], meta[18], tier_pages[1], s_i4)
+    ring_g, ring_l = meta[21:23]
+    fp_pool = PrecisionPool(name="fp", page_index=PhysicalPageIndex(*meta[1:4], meta[14], meta[17]), fp_v=fp_v)
+    int4_pool = PrecisionPool(name="int4", page_index=PhysicalPageIndex(*meta[23:28]), packed_v=int4_v)
+    int2_pool = PrecisionPool(name="int2", page_index=PhysicalPageIndex(*meta[28:33]), packed_v=compact_value)
+    recent = PrecisionPool(name="recent_fp", page_index=PhysicalPageIndex(*meta[10:13], ring_g, ring_l), fp_k=ring_k,
+                           fp_v=ring_v, active_length=0, capacity=cap, length_device=meta[13], global_index_buffer=ring_g,
+                           logical_position_buffer=ring_l)
     if bf16_keys:
         fp_pool.fp_k, int4_pool.fp_k = bf16_arena.view(0, s_fp), bf16_arena.view(s_fp, s_i4)
         int2_pool.fp_k = bf16_arena.view(s_fp + s_i4, s_i2)
     return ThreePrecisionCache(
         fp_pool=fp_pool, int4_pool=int4_pool, int2_pool=int2_pool, recent_fp_pool=recent, matched_fp=False,
         compact_key=compact_key, compact_value=compact_value, compact_int4_value=compact_int4_value,
-        static_int4_tokens=s_i4, generated_k_offset=0 if bf16_keys else n, bf16_key=bf16_arena, metadata_arena=meta,
-        evicted_global_indices=evicted, **common)
+        static_int4_tokens=s_i4, generated_k_offset=0 if bf16_keys else n, bf16_key=bf16_arena, metadata_arena=arena,
+        evicted_global_indices=meta[20], **common)
 
 
 # ------------------------------------------------------------------------- append / flush

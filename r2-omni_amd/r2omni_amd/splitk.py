@@ -313,6 +313,10 @@ class SplitKExecutor:
         t = self._template
         if t is not None and t[0] is self.workspace and t[1] == self.output_hadamard:
             return t[2]
+        return self._prepare_static()[2]
+
+    def _prepare_static(self) -> tuple:
+        """(workspace, output transform, launch arguments, the host module's copy of them)."""
         p = _lib.DecodeParams()
         ws = self.workspace
         p.reqs, p.items, p.group_begin = self.reqs.data_ptr(), self.items.data_ptr(), self.group_begin.data_ptr()
@@ -329,8 +333,11 @@ class SplitKExecutor:
         p.output_hadamard = int(self.output_hadamard)
         p.k_format = _k_format(self.caches[0])
         p.sm_scale = float(self.head_dim ** -0.5)
-        self._template = (ws, self.output_hadamard, p)
-        return p
+        device = self.reqs.device
+        handle = _lib.host().decode_handle(ctypes.addressof(p), _lib.address("r2o_decode"), device.index) \
+            if device.type == "cuda" else None
+        self._template = (ws, self.output_hadamard, p, handle)
+        return self._template
 
     def _params(self, query: torch.Tensor, out: torch.Tensor, append, *,
                 step_positions: torch.Tensor | None = None, rotary=None) -> _lib.DecodeParams:
@@ -379,10 +386,22 @@ class SplitKExecutor:
         and the appended rows are the raw projections and the launch applies the decode step's mRoPE
         (and FWHT) itself, in place of a separate ``qwen_qk_mrope`` launch (an extension of the
         reference's call, which takes rotated rows)."""
-        p, query, fused = self._prepare_call(query, append, self.workspace.output, rotary)
+        ws = self.workspace
+        if rotary is None:
+            # a step's usual forms (contiguous 16-byte-aligned rows, plain positions, room in the ring) are
+            # checked and launched by the host module; None: any other form, or an error to be raised
+            t = self._template
+            if t is None or t[0] is not ws or t[1] != self.output_hadamard:
+                t = self._prepare_static()
+            if t[3] is not None:
+                rc = _lib.host().decode(t[3], query, append, ws.output, self.caches, self.batched_recent_lengths)
+                if rc is not None:
+                    _lib.check(rc, "r2o_decode")
+                    return ws.output
+        p, query, fused = self._prepare_call(query, append, ws.output, rotary)
         self._launch(p, query.device)
         self._finish_call(fused)
-        return self.workspace.output
+        return ws.output
 
     def call_noalloc(self, query: torch.Tensor, append=None, *, out: torch.Tensor | None = None,
                      rotary=None) -> torch.Tensor:
