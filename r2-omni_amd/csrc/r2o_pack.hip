@@ -612,8 +612,10 @@ void launch_pack_cache(CachePack& a, int key_bits, int64_t superblock, int64_t d
 // order, and blocks of up to kFillBytes copy the page words and fill what no token reaches (-1 for unused
 // indices, 0 for the arenas' spare capacity and the ring).  In place of ~20 library launches (scan, gathers,
 // fills of whole arenas) that a build spent most of its time queueing.  Measured, with the payload's
-// launch: 4k tokens x 2 heads 5.3 + 5.6 us (357 -> 92 us a build, now the host's), 65k x 4 10.5 + 31 us
-// (391 -> 99), 131k x 8 9.8 + 132 us (572 -> 146, of which the packers' own changes 234).
+// launch: 4k tokens x 2 heads 3.6 + 5.4 us (a build 357 -> 65 us, the host's), 65k x 4 6.8 + 32 us (391 -> 71,
+// the host's), 131k x 8 5.5 + 129 us (572 -> 142, of which the packers' own changes 234).  Latency-bound: each
+// block's loads go out together (a fill's search through the arguments and a copy of 16 loads one after
+// another took 5.3, 10.5 and 9.8 us in place of 3.6, 6.8 and 5.5).
 constexpr int64_t kFillBytes = 32768;
 constexpr int kMaxFills = 20;
 
@@ -647,7 +649,7 @@ __global__ __launch_bounds__(256) void cache_index_kernel(CacheIndex a) {
         if (page >= a.n_pages) return;
         const int64_t start = a.start[page], len = a.start[a.n_pages + page], position = a.start[2 * a.n_pages + page];
         for (int64_t j = lane; j < len; j += 64) {
-            const int64_t token = start + j, p = position + j, g = a.plan_global[token];
+            const int64_t token = start + j, p = position + j, g = a.plan_global[token], l = a.plan_logical[token];
             if (p >= a.survivors) {
                 a.evicted[p - a.survivors] = g;
                 continue;
@@ -655,20 +657,26 @@ __global__ __launch_bounds__(256) void cache_index_kernel(CacheIndex a) {
             const int64_t slot = p + (p >= a.int2_at ? a.reserve4 : 0);
             a.index[p] = token;
             a.global[slot] = g;
-            a.logical[slot] = a.plan_logical[token];
+            a.logical[slot] = l;
         }
         return;
     }
     block -= a.page_blocks;
-    int i = 0;
-    while (i + 1 < a.n_fills && block >= a.fills[i + 1].first_block) ++i;
-    const Fill& f = a.fills[i];
+    // all first blocks in one load: a search from fill to fill waited on the launch arguments at every step
+    const bool begun = lane < a.n_fills && block >= a.fills[min(lane, kMaxFills - 1)].first_block;
+    const Fill& f = a.fills[__builtin_amdgcn_readfirstlane(__popcll(__ballot(begun)) - 1)];
     block -= f.first_block;
     const int64_t first = (int64_t)(block / f.heads) * kFillBytes, n = min(kFillBytes, f.bytes - first);
     unsigned char* dst = f.dst + (block % f.heads) * f.head_stride + first;
-    if (f.src) {  // the page words: 8-byte aligned, one head
-        for (int64_t e = threadIdx.x; e < n / 8; e += 256)
-            reinterpret_cast<int64_t*>(dst)[e] = reinterpret_cast<const int64_t*>(f.src + first)[e];
+    if (f.src) {  // the page words: 8-byte aligned, one head; every load first
+        const int64_t* src = reinterpret_cast<const int64_t*>(f.src + first);
+        constexpr int kEach = kFillBytes / 8 / 256;
+        int64_t w[kEach];
+#pragma unroll
+        for (int k = 0; k < kEach; ++k) w[k] = src[min((int64_t)threadIdx.x + 256 * k, n / 8 - 1)];
+#pragma unroll
+        for (int k = 0; k < kEach; ++k)
+            if (threadIdx.x + 256 * k < n / 8) reinterpret_cast<int64_t*>(dst)[threadIdx.x + 256 * k] = w[k];
         return;
     }
     const int64_t head = min((int64_t)(-reinterpret_cast<uintptr_t>(dst) & 15), n), body = (n - head) / 16;
