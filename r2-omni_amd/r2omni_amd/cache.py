@@ -9,8 +9,8 @@ Drop-in for the reference runtime (same names, fields, layouts and error message
   PrecisionPool, ThreePrecisionCache, build_three_precision_cache  precision_pool.py:152-274, 787-984
   CompactMetadataArena       precision_pool.py:45-145, 400-585
   append_generated_token, DynamicCacheStats  dynamic_fourq_cache.py:16-24, 172-267
-All payload bytes are produced by the gfx950 kernels of libr2o_sspa.so (r2o_pack_int4_k,
-r2o_pack_int4_v, r2o_pack_int2_v, r2o_gather_rows, r2o_recent_append, r2o_recent_shift);
+All payload bytes are produced by the gfx950 kernels of libr2o_sspa.so (r2o_cache_build, r2o_ring_flush,
+r2o_pack_int4_k, r2o_pack_int4_v, r2o_pack_int2_v, r2o_gather_rows, r2o_recent_append, r2o_recent_shift);
 torch only allocates the tensors and keeps small index vectors.  Variants: the released
 ``v_fourq_k_int4_compact`` cache, ``v_fourq_k_int2_compact``, ``v_fourq_k_bf16`` and the matched-FP
 cache; generated (flushed) values INT2 (released) or INT4 (``generated_value_precision="int4"``).
