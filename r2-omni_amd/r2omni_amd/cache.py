@@ -76,14 +76,12 @@ class CompactMetadataArena:
     int4_page_count: int
     int4_token_count: int
 
-    def _take_pages(self, pool: "PrecisionPool", n: int, page_size: int, tier: str) -> tuple[torch.Tensor, torch.Tensor]:
-        """Add ``n`` tokens of whole pages to the tier and return its (global, logical) index slots for them,
-        which the caller fills on the pool's stream."""
+    def _next_pages(self, n: int, page_size: int, tier: str) -> tuple[tuple[int, int], torch.Tensor, torch.Tensor]:
+        """Room for ``n`` more tokens of whole pages in the tier: its (pages, tokens) with them, and their (global,
+        logical) index slots, which the caller fills on the pool's stream before ``_commit_pages``."""
         if n <= 0 or n % int(page_size):
             raise ValueError(f"compact {tier.upper()} metadata append requires matching complete pages")
-        ids, offs, lens, g, l = (getattr(self, f"{tier}_{name}_buffer") for name in
-                                 ("original_page_ids", "physical_offsets", "lengths", "global_index",
-                                  "logical_position"))
+        lens, g, l = (getattr(self, f"{tier}_{name}_buffer") for name in ("lengths", "global_index", "logical_position"))
         pages, tokens = getattr(self, f"{tier}_page_count"), getattr(self, f"{tier}_token_count")
         page_end = pages + n // int(page_size)
         token_end = tokens + n
@@ -91,12 +89,19 @@ class CompactMetadataArena:
             raise RuntimeError(f"compact {tier.upper()} page metadata capacity exhausted")
         if token_end > g.numel():
             raise RuntimeError(f"compact {tier.upper()} token metadata capacity exhausted")
+        return (page_end, token_end), g[tokens:token_end], l[tokens:token_end]
+
+    def _commit_pages(self, pool: "PrecisionPool", ends: tuple[int, int], tier: str) -> None:
+        """Make ``ends`` = (pages, tokens) of ``_next_pages`` the tier's own: its counts and its pool's page index."""
+        ids, offs, lens, g, l = (getattr(self, f"{tier}_{name}_buffer") for name in
+                                 ("original_page_ids", "physical_offsets", "lengths", "global_index",
+                                  "logical_position"))
+        page_end, token_end = ends
         setattr(self, f"{tier}_page_count", page_end)
         setattr(self, f"{tier}_token_count", token_end)
         pool.page_index = PhysicalPageIndex(original_page_ids=ids[:page_end], physical_offsets=offs[:page_end],
                                             lengths=lens[:page_end], global_token_indices=g[:token_end],
                                             logical_positions=l[:token_end])
-        return g[tokens:token_end], l[tokens:token_end]
 
     def _append_pages(self, pool: "PrecisionPool", global_indices: torch.Tensor, logical_positions: torch.Tensor,
                       page_size: int, tier: str) -> None:
@@ -106,9 +111,10 @@ class CompactMetadataArena:
         if global_indices.dtype != torch.long or logical_positions.dtype != torch.long \
                 or global_indices.device != self.storage.device or logical_positions.device != self.storage.device:
             raise ValueError(f"compact {tier.upper()} metadata append requires same-device int64 indices")
-        g, l = self._take_pages(pool, n, page_size, tier)
+        ends, g, l = self._next_pages(n, page_size, tier)
         g.copy_(global_indices)
         l.copy_(logical_positions)
+        self._commit_pages(pool, ends, tier)
 
     def append_int2_pages(self, pool: "PrecisionPool", global_indices: torch.Tensor,
                           logical_positions: torch.Tensor, page_size: int) -> None:
@@ -1220,8 +1226,9 @@ class DynamicCacheStats:
     full_dequant_tensor_count: int = 0
 
 
-def _append_lowbit_page_metadata(pool: PrecisionPool, global_block: torch.Tensor, logical_block: torch.Tensor,
-                                 page_size: int) -> None:
+def _extended_page_index(pool: PrecisionPool, global_block: torch.Tensor, logical_block: torch.Tensor,
+                         page_size: int) -> PhysicalPageIndex:
+    """The page index of a pool without a metadata arena and of one more block of whole pages."""
     n = int(global_block.numel())
     if n <= 0 or n % page_size:
         raise ValueError("low-bit metadata append must contain complete pages")
@@ -1229,7 +1236,7 @@ def _append_lowbit_page_metadata(pool: PrecisionPool, global_block: torch.Tensor
     old = pool.page_index
     dev = global_block.device
     start = pool.token_count
-    pool.page_index = PhysicalPageIndex(
+    return PhysicalPageIndex(
         original_page_ids=torch.cat((old.original_page_ids, torch.full((pages,), -1, device=dev, dtype=torch.long))),
         physical_offsets=torch.cat((old.physical_offsets,
                                     start + torch.arange(pages, device=dev, dtype=torch.long) * page_size)),
@@ -1267,14 +1274,15 @@ def _flush_matched(cache: ThreePrecisionCache) -> None:
     """_append_matched_fp_block (dynamic_fourq_cache.py:145-170) and the ring's shift."""
     pool, flush = cache.recent_fp_pool, int(cache.recent_flush_size)
     # Views of the ring's oldest slots: every consumer copies them on this stream before the ring shift is
-    # launched, so no snapshot is needed.
-    _append_lowbit_page_metadata(cache.fp_pool, pool.global_index_buffer[:flush], pool.logical_position_buffer[:flush],
+    # launched, so no snapshot is needed.  What can fail (the pool's copies, key rows that
+    # have to grow) comes before its fields change.
+    index = _extended_page_index(cache.fp_pool, pool.global_index_buffer[:flush], pool.logical_position_buffer[:flush],
                                  cache.page_size)
+    values = torch.cat((cache.fp_pool.fp_v, pool.fp_v[:, :flush]), dim=1)
     cache.bf16_key.append_block(pool.fp_k[:, :flush])
     n = cache.bf16_key.active_length
     cache.bf16_key.segment_offsets = (0, n, n)
-    cache.fp_pool.fp_k = cache.bf16_key.view(0, n)
-    cache.fp_pool.fp_v = torch.cat((cache.fp_pool.fp_v, pool.fp_v[:, :flush]), dim=1)
+    cache.fp_pool.page_index, cache.fp_pool.fp_k, cache.fp_pool.fp_v = index, cache.bf16_key.view(0, n), values
     cache.generated_k_offset = n
     _lib.call("r2o_recent_shift", _lib.ptr(pool.fp_k), _lib.ptr(pool.fp_v), int(pool.fp_k.shape[0]), int(pool.capacity),
               flush, pool.active_length, _lib.ptr(pool.global_index_buffer), _lib.ptr(pool.logical_position_buffer),
@@ -1285,7 +1293,8 @@ def _flush_matched(cache: ThreePrecisionCache) -> None:
 def _flush_compact(cache: ThreePrecisionCache, stats: DynamicCacheStats, append) -> None:
     """The flush of a full ring into the compact arenas and its page metadata, the ring's shift and, with
     ``append`` = (K rows, V rows [Hkv, D], global index, logical position), the token that follows: one
-    host call of two launches (r2o_ring_flush).  Every refusal comes before the first launch."""
+    host call of two launches (r2o_ring_flush).  Every refusal comes before the first launch, and the cache's
+    counts and page index change after the launches were taken."""
     pool, flush, ck = cache.recent_fp_pool, int(cache.recent_flush_size), cache.compact_key
     if ck is None:
         raise RuntimeError("compact K cache is missing its compact K arena")
@@ -1327,13 +1336,18 @@ def _flush_compact(cache: ThreePrecisionCache, stats: DynamicCacheStats, append)
     if append is not None:
         nk, nv, p.new_global, p.new_logical = append
         p.new_k, p.new_v = nk.data_ptr(), nv.data_ptr()
-    if cache.metadata_arena is not None:  # in place (dynamic_fourq_cache.py:236-243)
-        g, l = cache.metadata_arena._take_pages(target, flush, cache.page_size, "int4" if int4_values else "int2")
+    arena, tier = cache.metadata_arena, "int4" if int4_values else "int2"
+    if arena is not None:  # in place (dynamic_fourq_cache.py:236-243)
+        ends, g, l = arena._next_pages(flush, cache.page_size, tier)
         p.dst_global, p.dst_logical = g.data_ptr(), l.data_ptr()
     else:
-        _append_lowbit_page_metadata(target, pool.global_index_buffer[:flush], pool.logical_position_buffer[:flush],
+        index = _extended_page_index(target, pool.global_index_buffer[:flush], pool.logical_position_buffer[:flush],
                                      cache.page_size)
     _lib.call("r2o_ring_flush", p, _lib.stream_of(dev))
+    if arena is not None:
+        arena._commit_pages(target, ends, tier)
+    else:
+        target.page_index = index
     stats.local_tail_dequant_tokens += p.k_tail
     if int4_values:  # dynamic_fourq_cache.py:212-219
         stats.flushed_int4_value_tokens += flush
