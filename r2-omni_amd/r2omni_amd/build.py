@@ -1,6 +1,7 @@
 """Compile the gfx950 HIP sources into the in-tree C-ABI library ``libr2o_sspa.so``.
 
-Usage: ``python -m r2omni_amd.build`` (from ``r2-omni_amd/``) or ``build_library()``.
+Usage: ``python -m r2omni_amd.build`` (from ``r2-omni_amd/``) or ``build()``;
+``build_library()`` leaves out the host module, and with it torch's headers.
 Every HIP translation unit is compiled for gfx950 only, with packed-FP32 instruction
 selection disabled and FP contraction off (the quantisers must round exactly like the
 reference's torch CPU path).
@@ -53,18 +54,34 @@ def common_flags() -> list[str]:
     ]
 
 
+def build(verbose: bool = False) -> str:
+    """The libraries and the host module, side by side; returns the decode library's path.  A host module that
+    does not build (no torch headers) raises after the libraries are in place."""
+    with ThreadPoolExecutor(1) as pool:
+        host = pool.submit(build_host_module, verbose)
+        path = build_library(verbose)
+        host.result()
+    return path
+
+
 def build_library(verbose: bool = False) -> str:
-    """Compile every source and link ``libr2o_sspa.so`` (and the host module ``_r2o_host.so``, bench.py's
-    ``libr2o_bench.so`` and ``libr2o_timeline.so``) next to this file; returns the decode library's path."""
+    """Compile every source of the C library and link ``libr2o_sspa.so`` (and bench.py's ``libr2o_bench.so`` and
+    ``libr2o_timeline.so``) next to this file; returns the decode library's path.  Needs hipcc alone."""
     timeline = ("R2O_TIMELINE",)
-    jobs = [(src, ()) for src in SOURCES + BENCH_SOURCES + (HOST_SOURCE,)] + [("r2o_decode.hip", timeline)]
+    jobs = [(src, ()) for src in SOURCES + BENCH_SOURCES] + [("r2o_decode.hip", timeline)]
     with ThreadPoolExecutor() as pool:  # one compiler process each; the decode kernels take most of the time
         objects = dict(zip(jobs, pool.map(lambda job: _compile(*job, verbose), jobs)))
     _link([objects[src, ()] for src in SOURCES], LIB_PATH, verbose)
     _link([objects[src, ()] for src in BENCH_SOURCES], BENCH_LIB_PATH, verbose)
     _link([objects.get((src, timeline), objects[src, ()]) for src in SOURCES], TIMELINE_LIB_PATH, verbose)
-    _link([objects[HOST_SOURCE, ()]], HOST_PATH, verbose, _torch_libraries())
     return LIB_PATH
+
+
+def build_host_module(verbose: bool = False) -> str:
+    """Compile and link ``_r2o_host.so`` next to this file, against the Python and the torch that run this; it
+    loads into those alone."""
+    _link([_compile(HOST_SOURCE, (), verbose)], HOST_PATH, verbose, _torch_libraries())
+    return HOST_PATH
 
 
 def _host_flags() -> list[str]:
@@ -164,4 +181,4 @@ def _check_resources(what: str, stderr: str, path: str) -> None:
 
 
 if __name__ == "__main__":
-    print(build_library(verbose=True))
+    print(build(verbose=True))
