@@ -267,6 +267,9 @@ def _request_desc(cache: ThreePrecisionCache) -> list[int]:
     return [words[f] for f in _lib.REQUEST_FIELDS]
 
 
+_UNPREPARED = object()  # the host module's copy of the launch arguments, before the first call that uses it
+
+
 @dataclass
 class SplitKExecutor:
     caches: list
@@ -316,7 +319,8 @@ class SplitKExecutor:
         return self._prepare_static()[2]
 
     def _prepare_static(self) -> tuple:
-        """(workspace, output transform, launch arguments, the host module's copy of them)."""
+        """(workspace, output transform, launch arguments, the host module's copy of them).  The copy is made by
+        the first plain call: every other form does without the module."""
         p = _lib.DecodeParams()
         ws = self.workspace
         p.reqs, p.items, p.group_begin = self.reqs.data_ptr(), self.items.data_ptr(), self.group_begin.data_ptr()
@@ -333,10 +337,12 @@ class SplitKExecutor:
         p.output_hadamard = int(self.output_hadamard)
         p.k_format = _k_format(self.caches[0])
         p.sm_scale = float(self.head_dim ** -0.5)
-        device = self.reqs.device
-        handle = _lib.host().decode_handle(ctypes.addressof(p), _lib.address("r2o_decode"), device.index) \
-            if device.type == "cuda" else None
-        self._template = (ws, self.output_hadamard, p, handle)
+        self._template = (ws, self.output_hadamard, p, _UNPREPARED if self.reqs.is_cuda else None)
+        return self._template
+
+    def _prepare_native(self, t: tuple) -> tuple:
+        handle = _lib.host().decode_handle(ctypes.addressof(t[2]), _lib.address("r2o_decode"), self.reqs.device.index)
+        self._template = t[:3] + (handle,)
         return self._template
 
     def _params(self, query: torch.Tensor, out: torch.Tensor, append, *,
@@ -393,6 +399,8 @@ class SplitKExecutor:
             t = self._template
             if t is None or t[0] is not ws or t[1] != self.output_hadamard:
                 t = self._prepare_static()
+            if t[3] is _UNPREPARED:
+                t = self._prepare_native(t)
             if t[3] is not None:
                 rc = _lib.host().decode(t[3], query, append, ws.output, self.caches, self.batched_recent_lengths)
                 if rc is not None:

@@ -43,3 +43,31 @@ def test_the_host_module_loads_into_this_python():
     from r2omni_amd import _lib
 
     assert all(callable(getattr(_lib.host(), f)) for f in ("decode_handle", "decode", "cache_build"))
+
+
+def test_only_the_plain_call_asks_for_the_host_module(monkeypatch):
+    """The launch arguments of rotary, graph and workspace-free calls are made without it."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from r2omni_amd import _lib
+    from r2omni_amd.splitk import SplitKExecutor, SplitKWorkspace
+
+    def missing():
+        raise RuntimeError("no host module")
+
+    class OnDevice(torch.Tensor):
+        is_cuda = True
+
+    monkeypatch.setattr(_lib, "host", missing)
+    f32 = torch.zeros(1)
+    cache = SimpleNamespace(recent_fp_pool=SimpleNamespace(fp_k=torch.zeros(1, dtype=torch.bfloat16)), bf16_key=f32)
+    ws = SplitKWorkspace(partial_max=f32, partial_sum=f32, partial_output=f32, output=f32, total_blocks=1, block_n=128,
+                         hierarchical_group_blocks=64, empty_bf16=f32)
+    reqs = torch.zeros(1, dtype=torch.int64).as_subclass(OnDevice)
+    ex = SplitKExecutor(caches=[cache], workspace=ws, reqs=reqs, items=f32, group_begin=f32, n_items=1, num_query_heads=2,
+                        num_key_value_heads=1)
+    assert ex._static_params().batch == 1
+    with pytest.raises(RuntimeError, match="no host module"):
+        ex(f32)
