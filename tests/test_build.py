@@ -58,7 +58,7 @@ def test_only_the_plain_call_asks_for_the_host_module(monkeypatch):
         raise RuntimeError("no host module")
 
     class OnDevice(torch.Tensor):
-        is_cuda = True
+        is_cuda, device = True, torch.device("cuda", 0)
 
     monkeypatch.setattr(_lib, "host", missing)
     f32 = torch.zeros(1)
