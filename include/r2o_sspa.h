@@ -306,7 +306,8 @@ int r2o_pack_int2_v(const uint16_t* src, int64_t dtype, int64_t hkv, int64_t src
                     void* stream);
 
 /* Row gather dst[h, i, :] = src[h, index[i], :] of 16-bit elements (FP-V pool build,
- * replaces value.index_select(1, tokens) at precision_pool.py:697-698). */
+ * replaces value.index_select(1, tokens) at precision_pool.py:697-698).  index NULL: src[h, i].
+ * Rows that start off a 16-byte boundary move element by element. */
 int r2o_gather_rows(const uint16_t* src, int64_t hkv, int64_t src_tokens, const int64_t* index,
                     int64_t n, uint16_t* dst, int64_t dst_stride, void* stream);
 

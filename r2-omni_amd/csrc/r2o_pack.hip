@@ -496,6 +496,7 @@ void launch_pack_keys(const KeyPack& a, int64_t superblock, int64_t dtype, int64
 
 // ---------------------------------------------------------------------------- gather rows
 // 64 rows per 256-thread block: thread t moves 16-byte chunk t % 16 of rows t / 16 + 16 k, all loads first.
+// Rows that start off 16 bytes move element by element.
 constexpr int kGatherRows = 64;
 
 struct RowGather {
@@ -507,6 +508,7 @@ struct RowGather {
     int64_t dst_stride;    // rows per head
 };
 
+template <bool VEC>
 __device__ __forceinline__ void gather_rows(const RowGather& a, int64_t block, int64_t h) {
     const int c = threadIdx.x & 15;
     const int64_t i0 = block * kGatherRows + (threadIdx.x >> 4);
@@ -519,18 +521,19 @@ __device__ __forceinline__ void gather_rows(const RowGather& a, int64_t block, i
     r2o_u4 v[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k)
-        v[k] = r2o_ldg(reinterpret_cast<const r2o_u4*>(a.src + (h * a.src_tokens + rows[k]) * 128 + 8 * c));
+        v[k] = r2o_load8<VEC>(a.src + (h * a.src_tokens + rows[k]) * 128 + 8 * c);
 #pragma unroll
     for (int k = 0; k < 4; ++k)  // keeps the four loads together (not sunk into the guarded stores)
         asm volatile("" ::"v"(v[k].x), "v"(v[k].y), "v"(v[k].z), "v"(v[k].w));
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         const int64_t i = i0 + 16 * k;
-        if (i < a.n) *reinterpret_cast<r2o_u4*>(a.dst + (h * a.dst_stride + i) * 128 + 8 * c) = v[k];
+        if (i < a.n) r2o_store8<VEC>(a.dst + (h * a.dst_stride + i) * 128 + 8 * c, v[k]);
     }
 }
 
-__global__ __launch_bounds__(256) void gather_rows_kernel(RowGather a) { gather_rows(a, blockIdx.x, blockIdx.y); }
+template <bool VEC>
+__global__ __launch_bounds__(256) void gather_rows_kernel(RowGather a) { gather_rows<VEC>(a, blockIdx.x, blockIdx.y); }
 
 // ------------------------------------------------------------------- a cache's payload in one launch
 // The keys, both packed value tiers and the 16-bit rows of a cache build, or the keys and values of a
@@ -565,9 +568,9 @@ __global__ __launch_bounds__(256) void pack_cache_kernel(CachePack a) {
     block -= a.v4_blocks;
     if (block < a.v2_blocks) return pack_values<2, DT, true>(a.v2, block, h);
     block -= a.v2_blocks;
-    if (block < a.fp_blocks) return gather_rows(a.fp, block, h);
+    if (block < a.fp_blocks) return gather_rows<true>(a.fp, block, h);
     block -= a.fp_blocks;
-    if (block < a.row_blocks) return gather_rows(a.rows, block, h);
+    if (block < a.row_blocks) return gather_rows<true>(a.rows, block, h);
     if (h != 0) return;
     for (int i = threadIdx.x; i < a.index_copies; i += blockDim.x) {
         a.index_dst[0][i] = a.index_src[0][i];
@@ -833,8 +836,12 @@ int r2o_gather_rows(const uint16_t* src, int64_t hkv, int64_t src_tokens, const 
     if (hkv <= 0 || n < 0 || n > dst_stride || n > 0x7fffffff) return R2O_EINVAL;
     if (n == 0) return R2O_OK;
     if (!src || !dst) return R2O_EINVAL;
-    hipLaunchKernelGGL(gather_rows_kernel, dim3((unsigned)blocks_of(n, kGatherRows), (unsigned)hkv), dim3(256), 0,
-                       (hipStream_t)stream, RowGather{src, src_tokens, index, n, dst, dst_stride});
+    const RowGather a{src, src_tokens, index, n, dst, dst_stride};
+    const dim3 grid((unsigned)blocks_of(n, kGatherRows), (unsigned)hkv);
+    const hipStream_t st = (hipStream_t)stream;
+    if ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) % 16 == 0)
+        hipLaunchKernelGGL(gather_rows_kernel<true>, grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(gather_rows_kernel<false>, grid, dim3(256), 0, st, a);
     R2O_CHECK_LAUNCH();
     return R2O_OK;
 }

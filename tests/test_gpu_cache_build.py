@@ -102,3 +102,21 @@ def test_build_refuses_plans_outside_the_sequence():
                                global_token_indices=torch.arange(63, device=dev))
     with pytest.raises(ValueError, match="cover the K/V sequence"):
         ro.build_three_precision_cache(k, k, plan)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 130])
+@pytest.mark.parametrize("src_off,dst_off", [(0, 0), (1, 0), (0, 3), (4, 8)])
+def test_gather_moves_rows_that_start_anywhere(n, src_off, dst_off):
+    from r2omni_amd import _lib
+
+    if not torch.cuda.is_available():
+        pytest.skip("needs an MI355X")
+    g = torch.Generator().manual_seed(n)
+    at = lambda rows, off: torch.zeros(2 * rows * 128 + off, dtype=torch.int16, device="cuda:0")[off:].view(2, rows, 128)  # noqa: E731
+    src, dst = at(n + 3, src_off), at(n + 2, dst_off)
+    src.copy_(torch.randint(-2 ** 15, 2 ** 15, src.shape, generator=g, dtype=torch.int32).to(torch.int16))
+    for index in (torch.randperm(n + 3, generator=g)[:n].to(src.device), None):
+        dst.fill_(5)
+        _lib.call("r2o_gather_rows", _lib.ptr(src), 2, n + 3, _lib.ptr(index), n, _lib.ptr(dst), n + 2,
+                  _lib.stream_of(src.device))
+        assert torch.equal(dst[:, :n], src[:, :n] if index is None else src[:, index]) and (dst[:, n:] == 5).all()
