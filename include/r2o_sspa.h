@@ -263,7 +263,7 @@ int r2o_decode_noalloc_init(int device);
  * Arena positions [dst_start, dst_start + tail + n) are (re)written; dst_start must be a
  * multiple of `superblock`.  The first `tail` positions are read back from the arena itself
  * (dequantised, rounded to `dtype`) — the flush rule of CompactInt4KeyArena.append_superblock
- * (compact_int4_key.py:210-220); the next n come from src[h, index[i]] (index NULL: i).
+ * (compact_int4_key.py:210-220); the next n come from src[h, index[i]] (index NULL: i, n <= src_tokens).
  * `operands` (nullable) receives, per superblock, the QK MFMA operands derived from the
  * stored scale/zero: for lane group g (channels 32g..32g+31), MFMA j and pair u, with
  * c = 32g + 8j + u, dword g*32 + 4j + u = fp16 (s[c], s[c+4]) and dword g*32 + 16 + 4j + u =
@@ -306,8 +306,8 @@ int r2o_pack_int2_v(const uint16_t* src, int64_t dtype, int64_t hkv, int64_t src
                     void* stream);
 
 /* Row gather dst[h, i, :] = src[h, index[i], :] of 16-bit elements (FP-V pool build,
- * replaces value.index_select(1, tokens) at precision_pool.py:697-698).  index NULL: src[h, i].
- * Rows that start off a 16-byte boundary move element by element. */
+ * replaces value.index_select(1, tokens) at precision_pool.py:697-698).  index NULL: src[h, i],
+ * n <= src_tokens.  Rows that start off a 16-byte boundary move element by element. */
 int r2o_gather_rows(const uint16_t* src, int64_t hkv, int64_t src_tokens, const int64_t* index,
                     int64_t n, uint16_t* dst, int64_t dst_stride, void* stream);
 

@@ -785,7 +785,7 @@ int r2o_pack_int4_k(const uint16_t* src, int64_t dtype, int64_t hkv, int64_t src
     if (!(superblock == 32 || superblock == 64 || superblock == 128) || (dtype != 0 && dtype != 1)) return R2O_EINVAL;
     if (hkv <= 0 || n < 0 || tail < 0 || tail >= superblock || dst_start < 0 || dst_start % superblock) return R2O_EINVAL;
     if (dst_start + tail + n > capacity || capacity % superblock || superblocks * superblock != capacity) return R2O_EINVAL;
-    if (n > 0 && (!src || src_tokens <= 0)) return R2O_EINVAL;
+    if (n > 0 && (!src || src_tokens <= 0 || (!index && n > src_tokens))) return R2O_EINVAL;
     if (tail + n == 0) return R2O_OK;
     launch_pack_keys<4>({src, src_tokens, index, n, tail, dst_start, packed, scale, zero, operands, capacity, superblocks},
                         superblock, dtype, hkv, (hipStream_t)stream);
@@ -799,7 +799,7 @@ int r2o_pack_int2_k(const uint16_t* src, int64_t dtype, int64_t hkv, int64_t src
     if (!(superblock == 32 || superblock == 64 || superblock == 128) || (dtype != 0 && dtype != 1)) return R2O_EINVAL;
     if (hkv <= 0 || n < 0 || tail < 0 || tail >= superblock || dst_start < 0 || dst_start % superblock) return R2O_EINVAL;
     if (dst_start + tail + n > capacity || capacity % superblock || superblocks * superblock != capacity) return R2O_EINVAL;
-    if (n > 0 && (!src || src_tokens <= 0)) return R2O_EINVAL;
+    if (n > 0 && (!src || src_tokens <= 0 || (!index && n > src_tokens))) return R2O_EINVAL;
     if (tail + n == 0) return R2O_OK;
     launch_pack_keys<2>({src, src_tokens, index, n, tail, dst_start, packed, scale, offset, operands, capacity, superblocks},
                         superblock, dtype, hkv, (hipStream_t)stream);
@@ -835,7 +835,7 @@ int r2o_gather_rows(const uint16_t* src, int64_t hkv, int64_t src_tokens, const 
                     uint16_t* dst, int64_t dst_stride, void* stream) {
     if (hkv <= 0 || n < 0 || n > dst_stride || n > 0x7fffffff) return R2O_EINVAL;
     if (n == 0) return R2O_OK;
-    if (!src || !dst) return R2O_EINVAL;
+    if (!src || !dst || src_tokens <= 0 || (!index && n > src_tokens)) return R2O_EINVAL;
     const RowGather a{src, src_tokens, index, n, dst, dst_stride};
     const dim3 grid((unsigned)blocks_of(n, kGatherRows), (unsigned)hkv);
     const hipStream_t st = (hipStream_t)stream;

@@ -244,3 +244,14 @@ def test_resource_check_rejects_a_kernel_with_scratch(tmp_path):
     _check_resources("x.hip", remarks("k_clean", 0), str(tmp_path / "ok.txt"))
     with pytest.raises(RuntimeError, match="k_stack"):
         _check_resources("x.hip", text, str(tmp_path / "bad.txt"))
+
+
+def test_row_counts_past_the_source_are_refused_before_any_launch():
+    """Without an index the packers and the gather read source rows 0 .. n - 1 (the pointers are never read here)."""
+    lib, at = _lib.load(), 4096
+    assert lib.r2o_gather_rows(at, 2, 10, None, 11, at, 16, None) == 1
+    assert lib.r2o_gather_rows(at, 2, 0, at, 1, at, 16, None) == 1
+    for pack in (lib.r2o_pack_int4_k, lib.r2o_pack_int2_k):
+        assert pack(at, 0, 2, 10, None, 11, 0, 0, at, at, at, None, 128, 4, 32, None) == 1
+    assert lib.r2o_pack_int4_v(at, 0, 2, 10, None, 11, 0, at, at, 128, None) == 1
+    assert lib.r2o_pack_int2_v(at, 0, 2, 10, None, 11, 0, 32, at, at, at, 128, None) == 1
