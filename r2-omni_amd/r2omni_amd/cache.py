@@ -887,12 +887,27 @@ def _host_page_table(plan: LayerCompressionPlan) -> torch.Tensor:
     return table.to("cpu", torch.long).contiguous()
 
 
-def _tier_page_table(plan: LayerCompressionPlan) -> _TierTable:
+def _plan_pages(plan: LayerCompressionPlan, s: int) -> tuple[torch.Tensor, tuple, tuple]:
+    """The host page table of a plan over ``s`` tokens and its (pages, tokens) of each tier.  The kernels read K, V
+    and the plan's indices at what it names: refuses pages and index vectors that do not fit the sequence."""
+    table = _host_page_table(plan)
+    counts = (ctypes.c_int64 * 8)()
+    if _lib.load().r2o_cache_pages(table.data_ptr(), int(table.shape[1]), s, counts, ctypes.byref(counts, 32)):
+        _tier_page_table(plan, table)  # names an unknown class
+        raise ValueError("static plan pages must lie inside the K/V sequence")
+    if sum(counts[4:]) != s:
+        raise ValueError("compact physical pools must cover every logical token")
+    if plan.global_token_indices.numel() < s:  # logical_positions: checked with the K/V shapes
+        raise ValueError("static plan indices must cover the K/V sequence")
+    return table, tuple(counts[:4]), tuple(counts[4:])
+
+
+def _tier_page_table(plan: LayerCompressionPlan, table: torch.Tensor | None = None) -> _TierTable:
     """Pages stably sorted by tier, each keeping its token order (precision_pool.py:611-669).
 
-    The page table is small: it is sorted on the host.
+    The page table is small: it is sorted on the host.  ``table``: the plan's ``_host_page_table``, if at hand.
     """
-    classes, starts, lens = _host_page_table(plan).numpy()
+    classes, starts, lens = (_host_page_table(plan) if table is None else table).numpy()
     if classes.size and (int(classes.min()) < 0 or int(classes.max()) >= _TIER_OF_CLASS.size):
         raise ValueError("page_classes holds a value that is not a PageClass")
     cat = _TIER_OF_CLASS[classes]
@@ -1101,6 +1116,8 @@ def build_three_precision_cache(
         raise ValueError("the SSPA decode path requires head_dim 128")
     _lib.require_device(key, "key")
     _lib.dtype_code(key.dtype)
+    _lib.require_device(value, "value")
+    _lib.dtype_code(value.dtype)
     key = key.contiguous()
     value = value.contiguous()
     if plan.recent_fp_capacity < page_size or plan.recent_fp_capacity % page_size:
@@ -1119,9 +1136,7 @@ def build_three_precision_cache(
 def _build_matched_cache(key, value, plan: LayerCompressionPlan, append_capacity: int, common: dict) -> ThreePrecisionCache:
     """Every surviving page, K and V in the model dtype, in one FP pool (precision_pool.py:834-876)."""
     dev, h, page_size = key.device, int(key.shape[0]), common["page_size"]
-    tab = _tier_page_table(plan)
-    if int(tab.tier_tokens.sum()) != int(key.shape[1]):
-        raise ValueError("compact physical pools must cover every logical token")
+    tab = _tier_page_table(plan, _plan_pages(plan, int(key.shape[1]))[0])
     gi = plan.global_token_indices.detach().to(dev, torch.long)
     lp = plan.logical_positions.detach().to(dev, torch.long)
     tokens = _expand_tier_tokens(tab, dev)
@@ -1146,29 +1161,17 @@ def _build_tiered_cache(key, value, plan: LayerCompressionPlan, append_capacity:
                         common: dict) -> ThreePrecisionCache:
     """The three pools and their metadata arena (precision_pool.py:878-984): one native call allocates every
     tensor, uploads the page table and makes the two launches of ``r2o_cache_build``."""
-    dev, s = key.device, int(key.shape[1])
+    dev = key.device
     ps, cap = common["page_size"], int(plan.recent_fp_capacity)
-    _lib.require_device(value, "value")
-    _lib.dtype_code(value.dtype)
     if group not in (32, 64, 128):
         raise ValueError("compact INT2 V requires group_size 32, 64, or 128")
     if append_capacity < 0:
         raise ValueError("append_capacity must be non-negative")
     # the kernels move rows in 16-byte pieces; a view may start between them
     key, value = (t.clone() if t.data_ptr() % 16 else t for t in (key, value))
-    table = _host_page_table(plan)
-    counts = (ctypes.c_int64 * 8)()
-    lib = _lib.load()
-    if lib.r2o_cache_pages(table.data_ptr(), int(table.shape[1]), s, counts, ctypes.byref(counts, 32)):
-        _tier_page_table(plan)  # names an unknown class
-        raise ValueError("static plan pages must lie inside the K/V sequence")
-    tier_pages, tier_tokens = tuple(counts[:4]), tuple(counts[4:])
-    if sum(tier_tokens) != s:
-        raise ValueError("compact physical pools must cover every logical token")
+    table, tier_pages, tier_tokens = _plan_pages(plan, int(key.shape[1]))
     gi = plan.global_token_indices.detach().to(dev, torch.long).contiguous()
     lp = plan.logical_positions.detach().to(dev, torch.long).contiguous()
-    if gi.numel() < s:
-        raise ValueError("static plan indices must cover the K/V sequence")
     s_fp, s_i4, s_i2, _ = tier_tokens
     n = s_fp + s_i4 + s_i2
     int2_keys = common["cache_variant"] == "v_fourq_k_int2_compact"
