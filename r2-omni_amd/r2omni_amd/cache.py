@@ -1358,6 +1358,18 @@ def _flush_compact(cache: ThreePrecisionCache, stats: DynamicCacheStats, append)
     values.active_length += flush
 
 
+def _ring_rows(pool: PrecisionPool, new_key: torch.Tensor, new_value: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """A token's K and V as the ring's [Hkv, D] rows, which is what the kernels read."""
+    _lib.require_device(new_key, "new_key")
+    _lib.require_device(new_value, "new_value")
+    if new_key.dtype != pool.fp_k.dtype or new_value.dtype != pool.fp_v.dtype:
+        raise ValueError("new K/V dtype must match the Recent-FP ring")
+    h, d = int(pool.fp_k.shape[0]), int(pool.fp_k.shape[2])
+    if new_key.numel() != h * d or new_value.numel() != h * d:
+        raise ValueError("new K/V must match the Recent-FP ring's heads")
+    return new_key.reshape(h, d).contiguous(), new_value.reshape(h, d).contiguous()
+
+
 def append_generated_token(cache: ThreePrecisionCache, new_key: torch.Tensor, new_value: torch.Tensor, *,
                            global_token_index: int, logical_position: int, stats: DynamicCacheStats) -> bool:
     """Append one token to the Recent-FP ring; when it is full, flush its oldest chunk first
@@ -1370,12 +1382,8 @@ def append_generated_token(cache: ThreePrecisionCache, new_key: torch.Tensor, ne
         new_key, new_value = new_key[0], new_value[0]
     if new_key.shape != new_value.shape or new_key.ndim != 3 or int(new_key.shape[1]) != 1:
         raise ValueError("new K/V must be [Hkv,1,D] or [1,Hkv,1,D]")
-    _lib.require_device(new_key, "new_key")
-    if new_key.dtype != pool.fp_k.dtype or new_value.dtype != pool.fp_v.dtype:
-        raise ValueError("new K/V dtype must match the Recent-FP ring")
     h, cap = int(pool.fp_k.shape[0]), int(pool.capacity)
-    nk = new_key.reshape(h, -1).contiguous()
-    nv = new_value.reshape(h, -1).contiguous()
+    nk, nv = _ring_rows(pool, new_key, new_value)
     position = (int(global_token_index), int(logical_position))
     if pool.active_length == cap and not cache.matched_fp and cache.bf16_key is None:
         _flush_compact(cache, stats, (nk, nv, *position))

@@ -21,7 +21,7 @@ from typing import Sequence
 import torch
 
 from . import _lib
-from .cache import ThreePrecisionCache
+from .cache import ThreePrecisionCache, _ring_rows
 
 TILE = 32
 _WAVES_PER_ITEM = 4          # waves of the partial kernel's workgroup (each takes a contiguous share)
@@ -725,11 +725,8 @@ def append_recent_fp_triton(cache: ThreePrecisionCache, new_key: torch.Tensor, n
     if any(v is None for v in (pool.fp_k, pool.fp_v, pool.global_index_buffer, pool.logical_position_buffer,
                                pool.length_device)):
         raise RuntimeError("Recent-FP staging buffers are incomplete")
-    _lib.require_device(new_key, "new_key")
-    h = int(new_key.shape[0])
-    nk = new_key.reshape(h, -1).contiguous()
-    nv = new_value.reshape(h, -1).contiguous()
-    _lib.call("r2o_recent_append", _lib.ptr(pool.fp_k), _lib.ptr(pool.fp_v), h, pool.capacity, _lib.ptr(nk),
+    nk, nv = _ring_rows(pool, new_key, new_value)
+    _lib.call("r2o_recent_append", _lib.ptr(pool.fp_k), _lib.ptr(pool.fp_v), int(pool.fp_k.shape[0]), pool.capacity, _lib.ptr(nk),
               _lib.ptr(nv), pool.active_length, int(global_token_index), int(logical_position),
               _lib.ptr(pool.length_device), _lib.ptr(pool.global_index_buffer),
               _lib.ptr(pool.logical_position_buffer), _lib.ptr(pool.page_index.lengths), cache.page_size,

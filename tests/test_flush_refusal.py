@@ -1,5 +1,6 @@
 """CPU checks that a flush which is refused, or whose launch fails, leaves the cache's counts and page indexes
-as they were: a pool never names tokens that were not packed, and a later flush takes the same places."""
+as they were: a pool never names tokens that were not packed, and a later flush takes the same places; and that
+rows which are not the ring's are refused."""
 import pytest
 import torch
 
@@ -90,3 +91,47 @@ def test_a_matched_flush_that_cannot_grow_leaves_the_cache_as_it_was(host_only, 
     with pytest.raises(torch.OutOfMemoryError):
         rc.flush_full_recent_pool(cache, stats)
     assert not host_only and _state(cache) == before and stats == rc.DynamicCacheStats()
+
+
+BAD_ROWS = {
+    "fewer heads": lambda k: (k[:1], k[:1]),
+    "more heads": lambda k: (torch.cat([k, k]), torch.cat([k, k])),
+    "narrow rows": lambda k: (k[..., :64], k[..., :64]),
+    "other type": lambda k: (k.half(), k.half()),
+    "host value": lambda k: (k, k.clone()),
+    "host key": lambda k: (k.clone(), k),
+}
+
+
+@pytest.mark.parametrize("form", BAD_ROWS)
+@pytest.mark.parametrize("length", [0, RING])
+def test_rows_that_are_not_the_rings_are_refused(monkeypatch, form, length):
+    """The append kernels read [Hkv, 128] rows of the ring's type on its GPU, with and without a flush before."""
+    from r2omni_amd.splitk import append_recent_fp_triton
+
+    def launched(name, *args):
+        raise AssertionError(f"{name} was launched")
+
+    def require(t, what):
+        if what.startswith("new_") and not hasattr(t, "on_device"):
+            raise RuntimeError(f"{what} must live on the GPU")
+
+    monkeypatch.setattr(_lib, "call", launched)
+    monkeypatch.setattr(_lib, "require_device", require)
+    monkeypatch.setattr(_lib, "stream_of", lambda device: 0)
+    key = torch.zeros(HEADS, 1, 128, dtype=torch.bfloat16)
+    key.on_device = True
+    rows = BAD_ROWS[form](key)
+    if not form.startswith("host"):
+        for t in rows:
+            t.on_device = True
+    cache, stats = _cache("int2"), rc.DynamicCacheStats()
+    cache.recent_fp_pool.active_length = length
+    before = _state(cache)
+    kw = dict(global_token_index=1, logical_position=1)
+    with pytest.raises((ValueError, RuntimeError), match="ring|GPU"):
+        rc.append_generated_token(cache, *rows, stats=stats, **kw)
+    if length < RING:
+        with pytest.raises((ValueError, RuntimeError), match="ring|GPU"):
+            append_recent_fp_triton(cache, *rows, **kw)
+    assert _state(cache) == before and stats == rc.DynamicCacheStats()
