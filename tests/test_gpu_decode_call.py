@@ -129,3 +129,35 @@ def test_replaced_workspace_other_streams_and_capture():
         torch.cuda.synchronize()
         got = ex.workspace.output.clone()
         assert torch.equal(got, ex(query))
+
+
+NATIVE = {"plain", "token axis", "ints", "lists", "other query type"}
+
+
+@pytest.mark.parametrize("dtype,batch,stacked", [("bfloat16", 1, False), ("float16", 1, False), ("bfloat16", 3, True)])
+@pytest.mark.parametrize("form", FORMS)
+def test_each_form_takes_its_route(form, dtype, batch, stacked, monkeypatch):
+    """The forms of a model's step are launched by the host module without reaching the Python path; it leaves
+    every other form to that path."""
+    from r2omni_amd import _lib
+
+    ex, q = _executor(dtype, batch=batch, stacked=stacked)
+    query, append = FORMS[form](q, *_rows(batch, dtype))
+    ex(q)  # prepares the handle
+    ex.workspace.output.zero_()
+    own = None if ex.batched_recent_lengths is None else list(ex.batched_recent_lengths)
+    rc = _lib.host().decode(ex._template[3], query, append, ex.workspace.output, ex.caches, own)
+    torch.cuda.synchronize()
+    assert rc == (0 if form in NATIVE else None)
+    assert bool(ex.workspace.output.any()) == (form in NATIVE)
+
+    def python_path(*args):
+        raise NotImplementedError("the Python path")
+
+    monkeypatch.setattr(ex, "_prepare_call", python_path)
+    if form in NATIVE:
+        ex(query, append)
+    else:
+        with pytest.raises(NotImplementedError):
+            ex(query, append)
+    torch.cuda.synchronize()
