@@ -19,6 +19,17 @@ CASES = [
 ]
 
 
+def _fill_free_memory(dev):
+    """Makes memory that a build may take hold 0x77: requests up to 1 MiB come from a pool of their own, so blocks of
+    many sizes are filled in both, small ones for the gaps between live tensors, and freed together."""
+    torch.cuda.empty_cache()
+    held = [torch.full((size,), 0x77, dtype=torch.uint8, device=dev)
+            for size, count in ((512, 1024), (1 << 12, 256), (1 << 16, 128), (1 << 20, 24), (1 << 22, 8)) for _ in range(count)]
+    del held
+    for t in [torch.empty(size, dtype=torch.uint8, device=dev) for size in (512, 1 << 12, 100_000, 900_000, 2_000_000)]:
+        assert (t == 0x77).all(), t.numel()
+
+
 @pytest.mark.parametrize("case", range(len(CASES)))
 @pytest.mark.parametrize("host_table", [True, False])
 def test_build_is_its_parts(case, host_table):
@@ -42,7 +53,7 @@ def test_build_is_its_parts(case, host_table):
                                logical_positions=plan.logical_positions + 11)
     k, v = (torch.empty(3 * s * 128 + offset, dtype=dtype, device=dev)[offset:].view(3, s, 128) for _ in range(2))
     k.copy_(torch.randn(3, s, 128, generator=g)), v.copy_(torch.randn(3, s, 128, generator=g))
-    torch.full((1 << 22,), 7, dtype=torch.uint8, device=dev)  # memory that a build may take is not zero
+    _fill_free_memory(dev)
     c = ro.build_three_precision_cache(k, v, plan, page_size=ps, key_quantization_superblock=sb, int2_group_size=group,
                                        generated_value_precision=gen, cache_variant=variant,
                                        compact_key_append_capacity=append)
@@ -120,3 +131,51 @@ def test_gather_moves_rows_that_start_anywhere(n, src_off, dst_off):
         _lib.call("r2o_gather_rows", _lib.ptr(src), 2, n + 3, _lib.ptr(index), n, _lib.ptr(dst), n + 2,
                   _lib.stream_of(src.device))
         assert torch.equal(dst[:, :n], src[:, :n] if index is None else src[:, index]) and (dst[:, n:] == 5).all()
+
+
+@pytest.mark.parametrize("variant", ["v_fourq_k_int4_compact", "v_fourq_k_int2_compact"])
+@pytest.mark.parametrize("types", [(torch.bfloat16, torch.float16), (torch.float16, torch.bfloat16)])
+def test_keys_and_values_of_different_types(variant, types):
+    """Two packing launches in place of one: the same arenas as the builders of each."""
+    import r2omni_amd as ro
+    from r2omni_amd.policy import plan_from_pages
+
+    if not torch.cuda.is_available():
+        pytest.skip("needs an MI355X")
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(2)
+    k, v = (torch.randn(3, 32 * 11, 128, generator=g).to(t).to(dev) for t in types)
+    cls = [(FP, I4, I2, EV)[i % 4] for i in range(11)]
+    plan = plan_from_pages([32 * i for i in range(11)], [32] * 11, cls, device=dev)
+    _fill_free_memory(dev)
+    c = ro.build_three_precision_cache(k, v, plan, cache_variant=variant)
+    fp, i4, i2 = (torch.cat([torch.arange(32 * i, 32 * i + 32) for i in range(11) if cls[i] == t]).to(dev) for t in (FP, I4, I2))
+    build = ro.build_compact_int4_key_arena if "int4" in variant else ro.build_compact_int2_key_arena
+    for x, y in zip(c.compact_key.allocation_tensors(),
+                    build(k, (fp, i4, i2), append_capacity=128, superblock_size=32).allocation_tensors()):
+        assert torch.equal(x, y)
+    for x, y in zip(c.compact_value.allocation_tensors(),
+                    ro.build_compact_int2_value_arena(v, i2, append_capacity=128, group_size=32).allocation_tensors()):
+        assert torch.equal(x, y)
+    four = ro.fused_gather_pack_int4_value(v, i4)
+    assert torch.equal(c.int4_pool.packed_v.packed, four.packed) and torch.equal(c.int4_pool.packed_v.scale, four.scale)
+    assert torch.equal(c.fp_pool.fp_v, v[:, fp])
+
+
+@pytest.mark.parametrize("offset", [0, 1, 4])
+def test_matched_build_of_rows_that_start_anywhere(offset):
+    import r2omni_amd as ro
+    from r2omni_amd.policy import plan_from_pages
+
+    if not torch.cuda.is_available():
+        pytest.skip("needs an MI355X")
+    dev = torch.device("cuda:0")
+    lens, cls = [32, 7, 32, 20, 32], [FP, I2, EV, I4, FP]
+    offs, s = [sum(lens[:i]) for i in range(5)], sum(lens)
+    g = torch.Generator().manual_seed(offset)
+    k, v = (torch.empty(3 * s * 128 + offset, dtype=torch.bfloat16, device=dev)[offset:].view(3, s, 128) for _ in range(2))
+    k.copy_(torch.randn(3, s, 128, generator=g)), v.copy_(torch.randn(3, s, 128, generator=g))
+    c = ro.build_three_precision_cache(k, v, plan_from_pages(offs, lens, cls, device=dev), matched_fp=True)
+    kept = torch.cat([torch.arange(o, o + n) for o, n, t in zip(offs, lens, cls) if t != EV]).to(dev)
+    assert torch.equal(c.fp_pool.fp_k, k[:, kept]) and torch.equal(c.fp_pool.fp_v, v[:, kept])
+    assert c.fp_pool.page_index.global_token_indices.tolist() == kept.tolist()
