@@ -227,3 +227,45 @@ def test_ring_flush_is_its_parts(ring, superblock, variant, gen, append):
             for f in ("original_page_ids", "physical_offsets", "lengths", "global_token_indices", "logical_positions"):
                 assert torch.equal(getattr(x.page_index, f), getattr(y.page_index, f))
     assert stats.flushed_tokens == 256
+
+
+@pytest.mark.parametrize("variant,gen,superblock", [("v_fourq_k_int4_compact", "int2", 32), ("v_fourq_k_int2_compact", "int4", 128)])
+@pytest.mark.parametrize("row,ring,arena", [(1, 0, 0), (4, 0, 0), (0, 1, 0), (0, 0, 1), (0, 0, 4), (3, 4, 1)])
+def test_a_flush_of_buffers_off_16_bytes(row, ring, arena, variant, gen, superblock):
+    """The appended row, the ring's rows or the arenas start ``row``, ``ring``, ``arena`` elements into their memory:
+    the flush that ends with an append moves and packs them in smaller pieces, to the same bytes."""
+    import r2omni_amd as ro
+    from r2omni_amd.policy import PageClass, plan_from_pages
+
+    dev = _dev()
+    cls = [int((PageClass.FP_PAGE, PageClass.INT4_PAGE, PageClass.INT2_PAGE)[i % 3]) for i in range(5)]
+    plan = plan_from_pages([32 * i for i in range(5)], [32] * 5, cls, recent_fp_capacity=256, device=dev)
+    g = torch.Generator().manual_seed(row + 10 * ring + 100 * arena)
+    k, v = (torch.randn(3, 160, 128, generator=g).to(torch.bfloat16).to(dev) for _ in range(2))
+    kw = dict(page_size=32, key_quantization_superblock=superblock, cache_variant=variant, generated_value_precision=gen,
+              compact_key_append_capacity=512)
+    want, cache = (ro.build_three_precision_cache(k, v, plan, **kw) for _ in range(2))
+    pool, key = cache.recent_fp_pool, cache.compact_key
+    value = cache.compact_int4_value if gen == "int4" else cache.compact_value
+    if ring:
+        pool.fp_k, pool.fp_v = _offset(pool.fp_k, ring), _offset(pool.fp_v, ring)
+    if arena:
+        for a, names in ((key, ("packed", "scale", "zero_point")), (value, ("packed", "scale") + ("zero_point",) * (gen == "int2"))):
+            for name in names:
+                setattr(a, name, _offset(getattr(a, name), arena))
+    rows = torch.randn(2, 257, 3, 1, 128, generator=g).to(torch.bfloat16).to(dev)
+    for c, off in ((want, 0), (cache, row)):
+        stats = ro.DynamicCacheStats()
+        for i in range(257):
+            flushed = ro.append_generated_token(c, _offset(rows[0, i], off), _offset(rows[1, i], off), global_token_index=160 + i,
+                                                logical_position=7 * i, stats=stats)
+        assert flushed and stats.flushed_tokens == 128
+
+    def tensors(c):
+        p, a = c.recent_fp_pool, c.compact_int4_value if gen == "int4" else c.compact_value
+        return [*c.compact_key.allocation_tensors(), *a.allocation_tensors(), p.fp_k[:, :129], p.fp_v[:, :129],
+                p.global_index_buffer[:129], p.logical_position_buffer[:129], p.length_device, p.page_index.lengths,
+                c.metadata_arena.storage]
+
+    for x, y in zip(tensors(cache), tensors(want)):
+        assert torch.equal(x, y)
