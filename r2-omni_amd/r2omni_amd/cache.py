@@ -76,12 +76,14 @@ class CompactMetadataArena:
     int4_page_count: int
     int4_token_count: int
 
-    def _next_pages(self, n: int, page_size: int, tier: str) -> tuple[tuple[int, int], torch.Tensor, torch.Tensor]:
-        """Room for ``n`` more tokens of whole pages in the tier: its (pages, tokens) with them, and their (global,
+    def _next_pages(self, n: int, page_size: int, tier: str) -> tuple[PhysicalPageIndex, torch.Tensor, torch.Tensor]:
+        """Room for ``n`` more tokens of whole pages in the tier: its page index with them, and their (global,
         logical) index slots, which the caller fills on the pool's stream before ``_commit_pages``."""
         if n <= 0 or n % int(page_size):
             raise ValueError(f"compact {tier.upper()} metadata append requires matching complete pages")
-        lens, g, l = (getattr(self, f"{tier}_{name}_buffer") for name in ("lengths", "global_index", "logical_position"))
+        ids, offs, lens, g, l = (getattr(self, f"{tier}_{name}_buffer") for name in
+                                 ("original_page_ids", "physical_offsets", "lengths", "global_index",
+                                  "logical_position"))
         pages, tokens = getattr(self, f"{tier}_page_count"), getattr(self, f"{tier}_token_count")
         page_end = pages + n // int(page_size)
         token_end = tokens + n
@@ -89,19 +91,16 @@ class CompactMetadataArena:
             raise RuntimeError(f"compact {tier.upper()} page metadata capacity exhausted")
         if token_end > g.numel():
             raise RuntimeError(f"compact {tier.upper()} token metadata capacity exhausted")
-        return (page_end, token_end), g[tokens:token_end], l[tokens:token_end]
+        index = PhysicalPageIndex(original_page_ids=ids[:page_end], physical_offsets=offs[:page_end],
+                                  lengths=lens[:page_end], global_token_indices=g[:token_end],
+                                  logical_positions=l[:token_end])
+        return index, g[tokens:token_end], l[tokens:token_end]
 
-    def _commit_pages(self, pool: "PrecisionPool", ends: tuple[int, int], tier: str) -> None:
-        """Make ``ends`` = (pages, tokens) of ``_next_pages`` the tier's own: its counts and its pool's page index."""
-        ids, offs, lens, g, l = (getattr(self, f"{tier}_{name}_buffer") for name in
-                                 ("original_page_ids", "physical_offsets", "lengths", "global_index",
-                                  "logical_position"))
-        page_end, token_end = ends
-        setattr(self, f"{tier}_page_count", page_end)
-        setattr(self, f"{tier}_token_count", token_end)
-        pool.page_index = PhysicalPageIndex(original_page_ids=ids[:page_end], physical_offsets=offs[:page_end],
-                                            lengths=lens[:page_end], global_token_indices=g[:token_end],
-                                            logical_positions=l[:token_end])
+    def _commit_pages(self, pool: "PrecisionPool", index: PhysicalPageIndex, tier: str) -> None:
+        """Make the page index of ``_next_pages`` the pool's, and its counts the tier's."""
+        setattr(self, f"{tier}_page_count", index.lengths.numel())
+        setattr(self, f"{tier}_token_count", index.global_token_indices.numel())
+        pool.page_index = index
 
     def _append_pages(self, pool: "PrecisionPool", global_indices: torch.Tensor, logical_positions: torch.Tensor,
                       page_size: int, tier: str) -> None:
@@ -111,10 +110,10 @@ class CompactMetadataArena:
         if global_indices.dtype != torch.long or logical_positions.dtype != torch.long \
                 or global_indices.device != self.storage.device or logical_positions.device != self.storage.device:
             raise ValueError(f"compact {tier.upper()} metadata append requires same-device int64 indices")
-        ends, g, l = self._next_pages(n, page_size, tier)
+        index, g, l = self._next_pages(n, page_size, tier)
         g.copy_(global_indices)
         l.copy_(logical_positions)
-        self._commit_pages(pool, ends, tier)
+        self._commit_pages(pool, index, tier)
 
     def append_int2_pages(self, pool: "PrecisionPool", global_indices: torch.Tensor,
                           logical_positions: torch.Tensor, page_size: int) -> None:
@@ -1311,9 +1310,10 @@ def _flush_compact(cache: ThreePrecisionCache, stats: DynamicCacheStats, append)
     values = cache.compact_int4_value if int4_values else cache.compact_value
     target = cache.int4_pool if int4_values else cache.int2_pool
     bits = ck.bit_width
-    if (int(pool.fp_k.shape[0]), int(pool.fp_k.shape[2])) != (ck.head_count, ck.head_dim):
+    h, _, d = pool.fp_k.shape
+    if (h, d) != (ck.head_count, ck.head_dim):
         raise ValueError(f"compact INT{bits} K flush requires 128 matching tokens")
-    if (int(pool.fp_v.shape[0]), int(pool.fp_v.shape[2])) != values.original_shape[::2]:
+    if pool.fp_v.shape[::2] != values.original_shape[::2]:
         raise ValueError(f"compact INT{4 if int4_values else 2} V flush must contain matching tokens")
     if not (pool.fp_k.is_contiguous() and pool.fp_v.is_contiguous()):
         raise ValueError(f"compact INT{bits} K flush block must have contiguous rows")
@@ -1327,7 +1327,7 @@ def _flush_compact(cache: ThreePrecisionCache, stats: DynamicCacheStats, append)
     prefix = ck.active_length // ck.superblock_size * ck.superblock_size
     p = _lib.RingFlush(
         recent_k=pool.fp_k.data_ptr(), recent_v=pool.fp_v.data_ptr(), dtype=_lib.dtype_code(pool.fp_k.dtype),
-        hkv=int(pool.fp_k.shape[0]), capacity=int(pool.capacity), flush=flush, active=int(pool.active_length),
+        hkv=h, capacity=int(pool.capacity), flush=flush, active=int(pool.active_length),
         global_buf=pool.global_index_buffer.data_ptr(), logical_buf=pool.logical_position_buffer.data_ptr(),
         length=pool.length_device.data_ptr(), page_lengths=pool.page_index.lengths.data_ptr(), page_size=cache.page_size,
         k_packed=ck.packed.data_ptr(), k_scale=ck.scale.data_ptr(), k_zero=ck.zero_point.data_ptr(),
@@ -1341,14 +1341,14 @@ def _flush_compact(cache: ThreePrecisionCache, stats: DynamicCacheStats, append)
         p.new_k, p.new_v = nk.data_ptr(), nv.data_ptr()
     arena, tier = cache.metadata_arena, "int4" if int4_values else "int2"
     if arena is not None:  # in place (dynamic_fourq_cache.py:236-243)
-        ends, g, l = arena._next_pages(flush, cache.page_size, tier)
+        index, g, l = arena._next_pages(flush, cache.page_size, tier)
         p.dst_global, p.dst_logical = g.data_ptr(), l.data_ptr()
     else:
         index = _extended_page_index(target, pool.global_index_buffer[:flush], pool.logical_position_buffer[:flush],
                                      cache.page_size)
     _lib.call("r2o_ring_flush", p, _lib.stream_of(dev))
     if arena is not None:
-        arena._commit_pages(target, ends, tier)
+        arena._commit_pages(target, index, tier)
     else:
         target.page_index = index
     stats.local_tail_dequant_tokens += p.k_tail
@@ -1364,8 +1364,8 @@ def _ring_rows(pool: PrecisionPool, new_key: torch.Tensor, new_value: torch.Tens
     _lib.require_device(new_value, "new_value")
     if new_key.dtype != pool.fp_k.dtype or new_value.dtype != pool.fp_v.dtype:
         raise ValueError("new K/V dtype must match the Recent-FP ring")
-    h, d = int(pool.fp_k.shape[0]), int(pool.fp_k.shape[2])
-    if new_key.numel() != h * d or new_value.numel() != h * d:
+    h, _, d = pool.fp_k.shape
+    if new_key.numel() != h * d:  # the callers have compared the two shapes
         raise ValueError("new K/V must match the Recent-FP ring's heads")
     return new_key.reshape(h, d).contiguous(), new_value.reshape(h, d).contiguous()
 
@@ -1382,10 +1382,9 @@ def append_generated_token(cache: ThreePrecisionCache, new_key: torch.Tensor, ne
         new_key, new_value = new_key[0], new_value[0]
     if new_key.shape != new_value.shape or new_key.ndim != 3 or int(new_key.shape[1]) != 1:
         raise ValueError("new K/V must be [Hkv,1,D] or [1,Hkv,1,D]")
-    h, cap = int(pool.fp_k.shape[0]), int(pool.capacity)
     nk, nv = _ring_rows(pool, new_key, new_value)
     position = (int(global_token_index), int(logical_position))
-    if pool.active_length == cap and not cache.matched_fp and cache.bf16_key is None:
+    if pool.active_length == pool.capacity and not cache.matched_fp and cache.bf16_key is None:
         _flush_compact(cache, stats, (nk, nv, *position))
         pool.active_length += 1 - flush
         stats.flushed_superblocks += 1
@@ -1393,8 +1392,8 @@ def append_generated_token(cache: ThreePrecisionCache, new_key: torch.Tensor, ne
         stats.appended_tokens += 1
         return True
     flushed = flush_full_recent_pool(cache, stats)
-    _lib.call("r2o_recent_append", _lib.ptr(pool.fp_k), _lib.ptr(pool.fp_v), h, cap, _lib.ptr(nk), _lib.ptr(nv),
-              pool.active_length, *position, _lib.ptr(pool.length_device),
+    _lib.call("r2o_recent_append", _lib.ptr(pool.fp_k), _lib.ptr(pool.fp_v), int(pool.fp_k.shape[0]),
+              int(pool.capacity), _lib.ptr(nk), _lib.ptr(nv), pool.active_length, *position, _lib.ptr(pool.length_device),
               _lib.ptr(pool.global_index_buffer), _lib.ptr(pool.logical_position_buffer),
               _lib.ptr(pool.page_index.lengths), cache.page_size, _lib.stream_of(new_key.device))
     pool.active_length += 1
