@@ -62,11 +62,6 @@ __device__ __forceinline__ uint32_t r2o_f32_to_f16(float x) {
     return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)x);
 }
 
-__device__ __forceinline__ float r2o_load_elem(const uint16_t* p, int64_t i, int dtype) {
-    uint32_t b = p[i];
-    return dtype == 0 ? r2o_bf16_to_f32(b) : r2o_f16_to_f32(b);
-}
-
 __device__ __forceinline__ float r2o_round_dtype(float x, int dtype) {
     return dtype == 0 ? r2o_bf16_to_f32(r2o_f32_to_bf16(x)) : r2o_f16_to_f32(r2o_f32_to_f16(x));
 }

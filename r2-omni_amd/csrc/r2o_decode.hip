@@ -393,16 +393,15 @@ __device__ __forceinline__ float head_max(float x) {
 
 // Online-softmax update for one tile whose logits are the lane's N values sv + add (log2 domain, -inf =
 // masked).  Returns the probabilities in pk; with ACC_L false the caller accumulates their sum itself (in
-// one of the `extra` accumulators).  The running max is raised lazily: only when a tile's max
+// one of the `extra` accumulators).  N is 8, or 4 for a KV group of at most 8 query heads, whose tiles are
+// held split (kSplitHeads): lane l16 then has the logits of head l16 % 8 and lane l16 ^ 8 the tile's other
+// half for the same head.  The running max is raised lazily: only when a tile's max
 // exceeds it by more than kRescaleSlack (log2 units) are the state and the NE accumulators at `extra`
 // (4-row accumulators in the PV output layout) rescaled, so p = exp2(s - m) stays below
 // 2^kRescaleSlack while the rescale branch is taken only a few times per work item.  (m, l, acc)
 // always refer to the same m, so the state and its later merges are exact.
 constexpr float kRescaleSlack = 4.f;
 
-//
-// N is 8, or 4 for a KV group of at most 8 query heads, whose tiles are held split (kSplitHeads): lane
-// l16 then has the logits of head l16 % 8 and lane l16 ^ 8 the tile's other half for the same head.
 template <int N, int NE = 0, bool ACC_L = true>
 __device__ __forceinline__ void softmax_tile(WaveState& st, const float (&sv)[N], float (&pk)[N], int g,
                                              float add = 0.f, r2o_f4* extra = nullptr) {
@@ -803,7 +802,7 @@ __device__ __forceinline__ int v2_slot(int t, int c) { return 8 * (t & 3) + 32 *
 // chunk of 16 consecutive tokens, so tokens 8..15 of a group swap their two chunks.  (Their 16-lane
 // passes still meet 2-way bank conflicts, which a layout cannot remove while 16 lanes read the same
 // half of 16 chunks; reading each chunk once with 16 bytes a lane and two row swaps removes them, but
-// the swaps cost this VALU-bound loop more than the conflicts do.)
+// the swaps cost more than the conflicts do.)
 __device__ __forceinline__ int k2_slot(int t, int c) { return 2 * t + (c ^ ((t >> 3) & 1)); }
 // BF16 V rows stay in natural order: 8 lanes read 8 consecutive chunks of one 256-byte row.
 // BF16 K: token t, chunk c (0..15) of its 256-byte row.  Reads: 8 lanes take one chunk of 8
@@ -1319,11 +1318,16 @@ __device__ __forceinline__ void decode_item(const r2o_decode_params& p) {
 #endif
 }
 
-// Split tiles (see kSplitHeads) are for INT2-K, the one key format whose loop is bound by VALU issue: measured
-// on 131k tokens, 32 / 8 heads, its call falls from 25.3 to 24.4 us, while INT4-K and 16-bit keys, which
-// wait for their tiles, stay where they are (+-0.4 % on the 7B and MiniCPM shapes, the folded rotation
-// 0.4 % slower).  INT2-K groups of more heads have a kernel of their own, so that neither carries the
-// other's code.
+// Split tiles (see kSplitHeads) are for INT2-K, where they were measured to gain: against 8 logits in the same
+// loop, 131k tokens of INT2 values, 32 / 8 heads, 24.45 -> 24.14 us a call at group 128, and 1.3 to 2.6 % at
+// group 32 with 4, 7 and 8 heads a group (22.1 -> 21.7 us, 7 heads).  Mixed value tiers: 0.7 to 3.3 % faster for
+// most (19.69 -> 19.15 us for four 7B requests of 8k to 64k), -0.6 to +1.7 % with superblocks of 32, up to 1.5 %
+// faster with INT4 values alone; on a box whose runs scattered by 1 to 4 % some of them came out 1 to 2 %
+// slower.  Split for the INT2 values' items alone it was up to 1.8 % slower than for all (19.15 -> 19.39 us).
+// INT4-K and 16-bit keys stay where they are (+-0.4 % on the 7B and MiniCPM shapes, the folded rotation 0.4 %
+// slower).  What makes the formats differ is not known: VALU issue takes 62 % of a SIMD's cycles in both, and
+// fewer instructions elsewhere in the loop shortened neither.  INT2-K groups of more heads have a kernel of
+// their own, so that neither carries the other's code.
 template <int KF, int RF, int RO>
 __global__ __launch_bounds__(KernelCfg<KF>::kThreads, KernelCfg<KF>::kWavesPerSimd) void decode_partial_kernel(
         r2o_decode_params p) {

@@ -2,8 +2,8 @@
 // launches.  A decode call's argument checks and launch arguments took ~5.6 us of Python and ctypes next to
 // ~6.8 us for the launches themselves, more than a small cache's time on the GPU: 11.8 -> 9.2 us per call at
 // 3B's heads over 4k tokens, 11.7 -> 10.7 (GPU-bound) over 32k.  A cache build's allocations, launch
-// arguments and ~45 metadata views took ~80 us next to 11 us of kernels: 92 -> 65 us (4k tokens), 99 -> 71
-// (64k, 42 us of kernels).
+// arguments and ~45 metadata views took ~80 us next to 9 us of kernels: 92 -> 68 us (4k tokens), 99 -> 75
+// (64k, 38 us of kernels).
 //
 // The decode entry takes the forms that a model's step uses and returns None for every other (strided or
 // misaligned rows, other types, a full ring, a folded rotation, any error): those keep the Python path and

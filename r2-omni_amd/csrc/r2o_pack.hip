@@ -615,7 +615,7 @@ void launch_pack_cache(CachePack& a, int key_bits, int64_t superblock, int64_t d
 // order, and blocks of up to kFillBytes copy the page words and fill what no token reaches (-1 for unused
 // indices, 0 for the arenas' spare capacity and the ring).  In place of ~20 library launches (scan, gathers,
 // fills of whole arenas) that a build spent most of its time queueing.  Measured, with the payload's
-// launch: 4k tokens x 2 heads 3.6 + 5.4 us (a build 357 -> 65 us, the host's), 65k x 4 6.8 + 32 us (391 -> 71,
+// launch: 4k tokens x 2 heads 3.6 + 5.4 us (a build 361 -> 68 us, the host's), 65k x 4 6.8 + 32 us (399 -> 75,
 // the host's), 131k x 8 5.5 + 129 us (572 -> 142, of which the packers' own changes 234).  Latency-bound: each
 // block's loads go out together (a fill's search through the arguments and a copy of 16 loads one after
 // another took 5.3, 10.5 and 9.8 us in place of 3.6, 6.8 and 5.5).

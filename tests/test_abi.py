@@ -229,6 +229,17 @@ def test_built_kernels_keep_their_state_in_registers_and_lds():
             assert vgpr + agpr <= 256 and occupancy >= 2, name
 
 
+def test_the_wide_int2_key_kernel_is_built_resident_too():
+    """INT2-K groups of more than 8 query heads: 2 row types x 3 rotations, two workgroups per CU."""
+    from r2omni_amd.build import ROOT_DIR
+
+    rows = open(os.path.join(ROOT_DIR, "_build", "r2o_decode.resources.txt")).read().splitlines()[1:]
+    wide = [ln.split(" ", 1)[1].split(" | ") for ln in rows if "decode_partial_wide_kernel" in ln]
+    assert len(wide) == 6
+    for vgpr, agpr, _, _, _, _, occupancy, _ in wide:
+        assert int(vgpr) + int(agpr) <= 256 and int(occupancy) >= 2
+
+
 def test_resource_check_rejects_a_kernel_with_scratch(tmp_path):
     from r2omni_amd.build import _check_resources, kernel_resources
 
